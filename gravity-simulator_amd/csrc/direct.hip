@@ -1,11 +1,12 @@
 // direct.hip -- direct-summation force kernels for gfx950.
 //
-//  k_direct_f64    FP64, one target per lane, sources staged through LDS in
-//                  index order: every target sums its sources l = 0..N-1
+//  k_direct_f64, k_direct_f64_wide
+//                  FP64: every target sums its sources l = 0..N-1
 //                  (l != k) in the order the reference's symmetric i<j loop
 //                  produces (src/acceleration.c:198-231), with the same
-//                  per-term operation order, contraction off and IEEE sqrt
-//                  and divide, so results are bitwise equal to the reference.
+//                  per-term operation order, contraction off and correctly
+//                  rounded sqrt and divide (fp64_inrange.h), so results are
+//                  bitwise equal to the reference.
 //  k_direct_f32    FP32 split precision: sources converted once per target
 //                  block to FP32 offsets from the block centre and staged as
 //                  float4 tiles in LDS; each lane holds IPT targets in
@@ -15,6 +16,7 @@
 //  k_energy        FP64 kinetic + pair potential energy (src/utils.c:27-59).
 //  k_lf_*          Leapfrog updates with the reference's compensated
 //                  summation (src/integrator.c:973-1094).
+#include "fp64_inrange.h"
 #include "gs_internal.h"
 
 #pragma clang fp contract(off)
@@ -26,29 +28,45 @@ constexpr int F64_BLOCK = 256;
 // ------------------------------------------------------------------ FP64
 // Bitwise reference sums: every target adds its terms in source-index order,
 // term = fl(fl(G / fl(fl(r*r)*r) * fl(x_l - x_k)) * m_l), l != k
-// (src/acceleration.c:206-229 as restated per target).  A workgroup takes
-// TB targets; per tile of 256 sources every thread computes its source's
-// terms for all TB targets into LDS (the expensive sqrt and division run on
-// all lanes), then one thread per (target, component) adds the tile's terms
-// in index order.  The additions are the reference's, in the reference's
-// order, so the result is bit for bit the serial one.  A source the
-// reference skips (the target itself; massless sources in the massless form;
-// past n) stores +0.0 instead: the running sum starts at +0.0 and a sum in
-// round-to-nearest is -0.0 only when both operands are, so the sum is never
-// -0.0 and adding +0.0 leaves it unchanged bit for bit.  The adds then form
-// one dependent chain of plain FP64 additions per (target, component), with
-// no selects.  TB = 4 for small N (more workgroups to fill the chip), 8
-// otherwise.
-// With LF the kernel is one whole Leapfrog step of the FP64 direct sum: every
-// position it reads (source or target) is first drifted as k_lf_drift drifts
-// it (compensated, src/integrator.c:1008-1018), and the thread that holds a
-// target component's sum then kicks that velocity component as k_lf_kick
-// does (src/integrator.c:1030-1039) and writes the drifted position, so the
-// three kernels' arithmetic is unchanged and one launch replaces three.
-// Positions, their compensation and velocities are read from one set of
-// buffers and written to another (every workgroup reads all positions while
-// others write theirs); a velocity's compensation is read and written only
-// by its own thread, in place.
+// (src/acceleration.c:206-229 as restated per target).  The terms are
+// computed by W wavefronts into LDS, tile by tile, while one more wavefront
+// adds the previous tile's in index order: the additions are the reference's,
+// in the reference's order, so the result is bit for bit the serial one.  A
+// source the reference skips (the target itself; massless sources in the
+// massless form; past n) stores +0.0 instead: the running sum starts at +0.0
+// and a sum in round-to-nearest is -0.0 only when both operands are, so the
+// sum is never -0.0 and adding +0.0 leaves it unchanged bit for bit.
+//
+// Two shapes, chosen by the number of targets (launch_f64):
+//   k_direct_f64       TB <= 16 targets per workgroup.  A thread holds K
+//                      targets and one source column of the tile; the adding
+//                      wavefront has one lane per (target, component), each
+//                      reading its own LDS row.  What bounds it: the chain of
+//                      n dependent additions, 12 cycles each on gfx950 (5 ns:
+//                      n = 1024 cannot take less than 5.1 us), while the
+//                      workgroups are no more than the CUs; then FP64 issue.
+//   k_direct_f64_wide  64 targets per workgroup, one per lane; sources come
+//                      through scalar loads, the adding wavefront runs three
+//                      chains per lane.  Bound by FP64 issue: 34 instructions
+//                      of 4.75 cycles and v_rsq_f64 (16) per 64 terms.
+// One MI355X, kernel alone, before (one wavefront of 12 to 24 lanes adding
+// after every tile, its rows 2048 bytes apart, so every read a bank conflict)
+// and now: n = 1024 13.0 -> 8.2 us, 4096 91 -> 44, 16384 1150 -> 461,
+// 65536 17.5 -> 6.9 ms, 100000 40.9 -> 16.6 ms (2.4e11 -> 6.0e11 pairs/s).
+//
+// LF_STEP: the kernel is one whole Leapfrog step of the FP64 direct sum:
+// every position it reads (source or target) is first drifted as k_lf_drift
+// drifts it (compensated, src/integrator.c:1008-1018), and the thread that
+// holds a target component's sum then kicks that velocity component as
+// k_lf_kick does (src/integrator.c:1030-1039) and writes the drifted
+// position, so the three kernels' arithmetic is unchanged and one launch
+// replaces three.  Positions, their compensation and velocities are read from
+// one set of buffers and written to another (every workgroup reads all
+// positions while others write theirs); a velocity's compensation is read and
+// written only by its own thread, in place.  LF_KICK: x is already drifted;
+// the kick only.
+enum LfMode { LF_NONE, LF_STEP, LF_KICK };
+
 struct LfStep {
     const double *xe = nullptr, *v = nullptr;  // state at the start of the step (with x)
     double *xo = nullptr, *xeo = nullptr, *vo = nullptr;  // drifted positions, kicked velocities
@@ -65,104 +83,273 @@ __device__ __forceinline__ double lf_drifted(double x0, double xe, double v, dou
     return x1;
 }
 
-template <int TB, bool SKIP_MASSLESS, bool LF>
-__global__ __launch_bounds__(F64_BLOCK) void k_direct_f64(const double *__restrict__ x,
-                                                          const double *__restrict__ m, int n,
-                                                          double G, double eps2,
-                                                          const int *__restrict__ targets,
-                                                          int num_targets,
-                                                          double *__restrict__ a, LfStep lf)
+__device__ __forceinline__ void lf_kicked(const LfStep &lf, int q, double acc)
 {
-    __shared__ double term[TB][3][F64_BLOCK];
+    const double v0 = lf.v[q];
+    double e = lf.ve[q] + acc * lf.dt;
+    const double v1 = v0 + e;
+    e += v0 - v1;
+    lf.vo[q] = v1;
+    lf.ve[q] = e;
+}
+
+// Targets first .. first + num_targets - 1.
+template <int TB, int W, int K, bool SKIP_MASSLESS, int LF>
+__global__ __launch_bounds__(64 * (W + 1)) void k_direct_f64(const double *__restrict__ x,
+                                                             const double *__restrict__ m, int n,
+                                                             double G, double eps2, int first,
+                                                             int num_targets,
+                                                             double *__restrict__ a, LfStep lf)
+{
+    constexpr int TILE = 64 * W * K / TB;
+    // rows of TILE + 2 doubles: the adding lanes read the same columns of
+    // 3 TB rows, 16 bytes each, from different banks
+    constexpr int ROW = TILE + 2;
+    static_assert(3 * TB <= 64 && TB % K == 0 && TILE % 2 == 0, "one adding wavefront");
+    __shared__ __align__(16) double term[2][3 * TB][ROW];
     __shared__ double tx[TB][3];
-    __shared__ int tk[TB];
     const int tid = threadIdx.x;
-    const int t0 = blockIdx.x * TB;
+    const int t0 = first + blockIdx.x * TB;
+    const int tend = first + num_targets;
     auto pos = [&](int q) {
-        if (!LF) return x[q];
+        if (LF != LF_STEP) return x[q];
         double e;
         return lf_drifted(x[q], lf.xe[q], lf.v[q], lf.dt, e);
     };
-    if (tid < TB) {
-        const int t = t0 + tid;
-        const int k = t < num_targets ? (targets ? targets[t] : t) : -1;
-        tk[tid] = k;
-        tx[tid][0] = k >= 0 ? pos(3 * k + 0) : 0.0;
-        tx[tid][1] = k >= 0 ? pos(3 * k + 1) : 0.0;
-        tx[tid][2] = k >= 0 ? pos(3 * k + 2) : 0.0;
+    if (tid < 3 * TB) {
+        const int t = t0 + tid / 3 < tend ? t0 + tid / 3 : t0;
+        tx[tid / 3][tid % 3] = pos(3 * t + tid % 3);
     }
     __syncthreads();
-    // accumulator of (target tid / 3, component tid % 3) for tid < 3 TB
-    double acc = 0.0;
-    const int at = tid / 3, ac = tid % 3;
-    for (int base = 0; base < n; base += F64_BLOCK) {
-        const int j = base + tid;
-        const bool src = j < n;
+    const int ntiles = (n + TILE - 1) / TILE;
+    if (tid < 64 * W) {
+        // column c of the tile, targets tb .. tb + K - 1
+        const int c = tid % TILE;
+        const int tb = (tid / TILE) * K;
+        double k0[K], k1[K], k2[K];
+#pragma unroll
+        for (int u = 0; u < K; u++) {
+            k0[u] = tx[tb + u][0];
+            k1[u] = tx[tb + u][1];
+            k2[u] = tx[tb + u][2];
+        }
+        const bool g_in = numerator_in_range(G);
         double xj0 = 0.0, xj1 = 0.0, xj2 = 0.0, mj = 0.0;
-        if (src) {
-            xj0 = pos(3 * j + 0);
-            xj1 = pos(3 * j + 1);
-            xj2 = pos(3 * j + 2);
-            mj = m[j];
-        }
-#pragma unroll 2
-        for (int tt = 0; tt < TB; tt++) {
-            const int k = tk[tt];
-            const bool sk = !src || k < 0 || j == k || (SKIP_MASSLESS && mj == 0.0);
-            double t0v = 0.0, t1v = 0.0, t2v = 0.0;
-            if (!sk) {
-                const double R0 = xj0 - tx[tt][0];
-                const double R1 = xj1 - tx[tt][1];
-                const double R2 = xj2 - tx[tt][2];
-                const double r = __builtin_sqrt(R0 * R0 + R1 * R1 + R2 * R2 + eps2);
-                const double tv = G / (r * r * r);
-                t0v = (tv * R0) * mj;
-                t1v = (tv * R1) * mj;
-                t2v = (tv * R2) * mj;
+        auto load = [&](int j) {
+            if (j < n) {
+                xj0 = pos(3 * j + 0);
+                xj1 = pos(3 * j + 1);
+                xj2 = pos(3 * j + 2);
+                mj = m[j];
             }
-            term[tt][0][tid] = t0v;
-            term[tt][1][tid] = t1v;
-            term[tt][2][tid] = t2v;
+        };
+        load(c);
+        for (int tile = 0; tile < ntiles; tile++) {
+            const int j0 = tile * TILE;
+            const int j = j0 + c;
+            const double s0 = xj0, s1 = xj1, s2 = xj2, ms = mj;
+            load(j + TILE);  // the next tile's source, while this one's terms are formed
+            double R0[K], R1[K], R2[K], r2[K], tv[K];
+            bool in = g_in;
+#pragma unroll
+            for (int u = 0; u < K; u++) {
+                R0[u] = s0 - k0[u];
+                R1[u] = s1 - k1[u];
+                R2[u] = s2 - k2[u];
+                r2[u] = R0[u] * R0[u] + R1[u] * R1[u] + R2[u] * R2[u] + eps2;
+                in = in && r2_in_range(r2[u]);
+            }
+            if (__all(in)) {
+                over_r3<K>(G, r2, tv);
+            } else {
+#pragma unroll 1
+                for (int u = 0; u < K; u++) tv[u] = over_r3_any(G, r2[u]);
+            }
+            double(*row)[ROW] = &term[tile & 1][3 * tb];
+            // (the same for the whole workgroup: a tile that holds targets, or runs past n)
+            const bool special = SKIP_MASSLESS || (j0 < t0 + TB && j0 + TILE > t0) || j0 + TILE > n;
+            if (special) {
+                const bool src = j < n && !(SKIP_MASSLESS && ms == 0.0);
+#pragma unroll
+                for (int u = 0; u < K; u++) {
+                    const bool use = src && t0 + tb + u != j;
+                    row[3 * u + 0][c] = use ? (tv[u] * R0[u]) * ms : 0.0;
+                    row[3 * u + 1][c] = use ? (tv[u] * R1[u]) * ms : 0.0;
+                    row[3 * u + 2][c] = use ? (tv[u] * R2[u]) * ms : 0.0;
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < K; u++) {
+                    row[3 * u + 0][c] = (tv[u] * R0[u]) * ms;
+                    row[3 * u + 1][c] = (tv[u] * R1[u]) * ms;
+                    row[3 * u + 2][c] = (tv[u] * R2[u]) * ms;
+                }
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        if (tid < 3 * TB) {
-            const double *tp = term[at][ac];
-#pragma unroll 32
-            for (int jj = 0; jj < F64_BLOCK; jj++) acc = acc + tp[jj];
-        }
-        __syncthreads();
+        return;
     }
-    if (tid < 3 * TB && t0 + at < num_targets) {
-        const int q = 3 * (t0 + at) + ac;
+    // the adding wavefront: lane 3 t + d holds target t's component d
+    __builtin_amdgcn_s_setprio(3);
+    const int lane = tid - 64 * W;
+    const int r = lane < 3 * TB ? lane : 0;
+    double acc = 0.0;
+    for (int tile = 0; tile < ntiles; tile++) {
+        __syncthreads();
+        const double2 *tp = reinterpret_cast<const double2 *>(term[tile & 1][r]);
+#pragma unroll 16
+        for (int jj = 0; jj < TILE / 2; jj++) {
+            const double2 t = tp[jj];
+            acc = acc + t.x;
+            acc = acc + t.y;
+        }
+    }
+    if (lane < 3 * TB && t0 + lane / 3 < tend) {
+        const int q = 3 * t0 + lane;
         a[q] = acc;
-        if (LF) {
+        if (LF == LF_STEP) {
             double ex;
             lf.xo[q] = lf_drifted(x[q], lf.xe[q], lf.v[q], lf.dt, ex);
             lf.xeo[q] = ex;
-            const double v0 = lf.v[q];
-            double e = lf.ve[q] + acc * lf.dt;
-            const double v1 = v0 + e;
-            e += v0 - v1;
-            lf.vo[q] = v1;
-            lf.ve[q] = e;
         }
+        if (LF != LF_NONE) lf_kicked(lf, q, acc);
     }
 }
 
-template <bool SKIP_MASSLESS, bool LF = false>
-static void launch_f64_shape(Context *c, int n, const double *x, const double *m, double G,
-                             double eps2, const int *targets, int num_targets, double *out,
-                             const LfStep &lf = LfStep())
+// 64 targets per workgroup, one per lane, tiles of W K sources (the last
+// tile's missing sources are repeats of the last one, never added).
+template <int W, int K, bool SKIP_MASSLESS, int LF>
+__global__ __launch_bounds__(64 * (W + 1)) void k_direct_f64_wide(const double *__restrict__ x,
+                                                                  const double *__restrict__ m,
+                                                                  int n, double G, double eps2,
+                                                                  double *__restrict__ a,
+                                                                  LfStep lf)
 {
-    // 4 targets per workgroup while 8 would leave CUs idle
-    if ((num_targets + 7) / 8 < 2 * c->cu_count)
-        hipLaunchKernelGGL((k_direct_f64<4, SKIP_MASSLESS, LF>), dim3((num_targets + 3) / 4),
-                           dim3(F64_BLOCK), 0, c->stream, x, m, n, G, eps2, targets, num_targets,
-                           out, lf);
-    else
-        hipLaunchKernelGGL((k_direct_f64<8, SKIP_MASSLESS, LF>), dim3((num_targets + 7) / 8),
-                           dim3(F64_BLOCK), 0, c->stream, x, m, n, G, eps2, targets, num_targets,
-                           out, lf);
+    static_assert(LF != LF_STEP, "the wide form takes drifted positions");
+    constexpr int TILE = W * K;
+    __shared__ double term[2][TILE][3][64];
+    const int lane = threadIdx.x & 63;
+    // (uniform; readfirstlane lets the compiler keep the sources in SGPRs)
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t0 = blockIdx.x * 64;
+    const int t = t0 + lane;
+    const int ntiles = (n + TILE - 1) / TILE;
+    if (wv < W) {
+        const int k = t < n ? t : t0;
+        const double k0 = x[3 * k + 0], k1 = x[3 * k + 1], k2 = x[3 * k + 2];
+        const bool g_in = numerator_in_range(G);
+        for (int tile = 0; tile < ntiles; tile++) {
+            const int j0 = tile * TILE + wv * K;
+            double R0[K], R1[K], R2[K], r2[K], tv[K], ms[K];
+            bool in = g_in;
+#pragma unroll
+            for (int u = 0; u < K; u++) {
+                const int j = j0 + u < n ? j0 + u : n - 1;
+                ms[u] = m[j];
+                R0[u] = x[3 * j + 0] - k0;
+                R1[u] = x[3 * j + 1] - k1;
+                R2[u] = x[3 * j + 2] - k2;
+                r2[u] = R0[u] * R0[u] + R1[u] * R1[u] + R2[u] * R2[u] + eps2;
+                in = in && r2_in_range(r2[u]);
+            }
+            if (__all(in)) {
+                over_r3<K>(G, r2, tv);
+            } else {
+#pragma unroll 1
+                for (int u = 0; u < K; u++) tv[u] = over_r3_any(G, r2[u]);
+            }
+            double(*row)[3][64] = &term[tile & 1][wv * K];
+#pragma unroll
+            for (int u = 0; u < K; u++) {
+                row[u][0][lane] = (tv[u] * R0[u]) * ms[u];
+                row[u][1][lane] = (tv[u] * R1[u]) * ms[u];
+                row[u][2][lane] = (tv[u] * R2[u]) * ms[u];
+            }
+            if (SKIP_MASSLESS || (j0 < t0 + 64 && j0 + K > t0)) {
+#pragma unroll
+                for (int u = 0; u < K; u++)
+                    if (j0 + u == t || (SKIP_MASSLESS && ms[u] == 0.0))
+                        row[u][0][lane] = row[u][1][lane] = row[u][2][lane] = 0.0;
+            }
+            __syncthreads();
+        }
+        return;
+    }
+    __builtin_amdgcn_s_setprio(3);
+    double acc[3] = {0.0, 0.0, 0.0};
+    for (int tile = 0; tile < ntiles; tile++) {
+        __syncthreads();
+        const double(*row)[3][64] = term[tile & 1];
+        const int cnt = min(TILE, n - tile * TILE);
+        if (cnt == TILE) {
+#pragma unroll
+            for (int u = 0; u < TILE; u++)
+#pragma unroll
+                for (int d = 0; d < 3; d++) acc[d] = acc[d] + row[u][d][lane];
+        } else {
+            for (int u = 0; u < cnt; u++)
+#pragma unroll
+                for (int d = 0; d < 3; d++) acc[d] = acc[d] + row[u][d][lane];
+        }
+    }
+    if (t >= n) return;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const int q = 3 * t + d;
+        a[q] = acc[d];
+        if (LF == LF_KICK) lf_kicked(lf, q, acc[d]);
+    }
+}
+
+// The wide form runs one workgroup per CU (138 KB of LDS), so its time goes
+// by whole rounds of 64 cu_count targets: it takes as many targets as fill
+// rounds, and the rest too when that fills more than 3/5 of one; below that
+// the narrow form is faster for the rest (n = 8192, half a round: 150 us
+// against 230; n = 12000: 312 against 337; n = 16384: 557 against 461).
+static int f64_wide_targets(int n, int cu_count)
+{
+    const long long round = 64ll * cu_count;
+    const long long rest = n % round;
+    return static_cast<int>(5 * rest > 3 * round ? n : n - rest);
+}
+
+template <bool SKIP_MASSLESS, int LF>
+static void launch_f64(Context *c, int n, const double *x, const double *m, double G, double eps2,
+                       double *out, const LfStep &lf = LfStep())
+{
+    constexpr int AFTER = LF == LF_STEP ? LF_KICK : LF;
+    const int wide = LF == LF_STEP ? 0 : f64_wide_targets(n, c->cu_count);
+    if (wide > 0)
+        hipLaunchKernelGGL((k_direct_f64_wide<15, 3, SKIP_MASSLESS, AFTER>), dim3((wide + 63) / 64),
+                           dim3(1024), 0, c->stream, x, m, n, G, eps2, out, lf);
+    const int rest = n - wide;
+    if (rest <= 0) return;
+    auto narrow = [&](auto kernel, int tb, int w) {
+        hipLaunchKernelGGL(kernel, dim3((rest + tb - 1) / tb), dim3(64 * (w + 1)), 0, c->stream, x,
+                           m, n, G, eps2, wide, rest, out, lf);
+    };
+    // The fewest targets per workgroup that still leave about one workgroup
+    // per CU: the chain of additions is the time, and the CU's wavefronts
+    // have the terms ready before it (measured: 2048 targets, TB = 4 / 8 / 16:
+    // 21 / 19 / 24 us; 4096: 72 / 51 / 44).  Past one workgroup per CU fewer
+    // wavefronts per workgroup, so that several share a CU (6000: 109 -> 101
+    // us with TB = 8, 8192: 173 and 211 with TB = 8 against 148).
+    const int cu = c->cu_count;
+    if (rest <= 4 * cu) narrow(k_direct_f64<4, 4, 4, SKIP_MASSLESS, LF>, 4, 4);
+    else if (rest <= 8 * cu) narrow(k_direct_f64<8, 8, 2, SKIP_MASSLESS, LF>, 8, 8);
+    else if (rest <= 16 * cu) narrow(k_direct_f64<16, 15, 2, SKIP_MASSLESS, LF>, 16, 15);
+    else narrow(k_direct_f64<16, 8, 2, SKIP_MASSLESS, LF>, 16, 8);
+}
+
+__global__ void k_lf_drift_to(const double *__restrict__ x, const double *__restrict__ xe,
+                              const double *__restrict__ v, int n3, double dt,
+                              double *__restrict__ xo, double *__restrict__ xeo)
+{
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= n3) return;
+    double e;
+    xo[q] = lf_drifted(x[q], xe[q], v[q], dt, e);
+    xeo[q] = e;
 }
 
 hipError_t launch_lf_step_f64(Context *c, const double *x, const double *xe, const double *v,
@@ -178,10 +365,19 @@ hipError_t launch_lf_step_f64(Context *c, const double *x, const double *xe, con
     lf.ve = ve;
     lf.dt = dt;
     const int rec = timing_begin(c, "direct_f64");
-    if (skip_massless)
-        launch_f64_shape<true, true>(c, n, x, m, G, eps * eps, nullptr, n, a, lf);
-    else
-        launch_f64_shape<false, true>(c, n, x, m, G, eps * eps, nullptr, n, a, lf);
+    if (f64_wide_targets(n, c->cu_count) > 0) {
+        // the drift as a pass of its own (a few us of a step of at least 0.3 ms)
+        hipLaunchKernelGGL(k_lf_drift_to, dim3((3 * n + 255) / 256), dim3(256), 0, c->stream, x, xe,
+                           v, 3 * n, dt, xo, xeo);
+        if (skip_massless)
+            launch_f64<true, LF_KICK>(c, n, xo, m, G, eps * eps, a, lf);
+        else
+            launch_f64<false, LF_KICK>(c, n, xo, m, G, eps * eps, a, lf);
+    } else if (skip_massless) {
+        launch_f64<true, LF_STEP>(c, n, x, m, G, eps * eps, a, lf);
+    } else {
+        launch_f64<false, LF_STEP>(c, n, x, m, G, eps * eps, a, lf);
+    }
     timing_end(c, rec);
     return hipGetLastError();
 }
@@ -191,23 +387,10 @@ hipError_t launch_direct_f64(Context *c, const double *x, const double *m, int n
 {
     const int rec = timing_begin(c, "direct_f64");
     if (skip_massless)
-        launch_f64_shape<true>(c, n, x, m, G, eps * eps, nullptr, n, a);
+        launch_f64<true, LF_NONE>(c, n, x, m, G, eps * eps, a);
     else
-        launch_f64_shape<false>(c, n, x, m, G, eps * eps, nullptr, n, a);
+        launch_f64<false, LF_NONE>(c, n, x, m, G, eps * eps, a);
     timing_end(c, rec);
-    return hipGetLastError();
-}
-
-// FP64 direct sum for a list of targets (the GPU FP64 oracle for sampled
-// error checks); out[t] is the acceleration of particle targets[t].
-hipError_t launch_direct_f64_targets(Context *c, const double *x, const double *m, int n,
-                                     double G, double eps, bool skip_massless,
-                                     const int *targets, int num_targets, double *out)
-{
-    if (skip_massless)
-        launch_f64_shape<true>(c, n, x, m, G, eps * eps, targets, num_targets, out);
-    else
-        launch_f64_shape<false>(c, n, x, m, G, eps * eps, targets, num_targets, out);
     return hipGetLastError();
 }
 

@@ -1,0 +1,76 @@
+// fp64_inrange.h -- IEEE square root and division of FP64 operands known to
+// lie well inside the exponent range.
+//
+// The compiler's expansions of sqrt and / carry steps for operands near the
+// ends of the range (scale, class and fix-up instructions; the division's go
+// through the one VCC register, which keeps independent divisions of a lane
+// from overlapping).  Inside the range the remaining steps give the same
+// correctly rounded results on their own.  Measured issue cost per wave64 on
+// MI355X: sqrt 86 cycles and division 61, against 59 and 38 here.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+namespace gs {
+
+// r2 in [2^-400, 2^400): the operands inverse_cube_ready accepts.
+constexpr unsigned R2_HI_MIN = (1023u - 400u) << 20;
+constexpr unsigned R2_HI_SPAN = 800u << 20;
+
+// G in [2^-300, 2^300) in magnitude
+__device__ __forceinline__ bool numerator_in_range(double G)
+{
+    const unsigned e = static_cast<unsigned>(__double_as_longlong(G) >> 32) & 0x7fffffffu;
+    return e - ((1023u - 300u) << 20) < (600u << 20);
+}
+
+// False for zeros, subnormals, infinities, NaN and negative values too.
+__device__ __forceinline__ bool r2_in_range(double r2)
+{
+    return static_cast<unsigned>(__double_as_longlong(r2) >> 32) - R2_HI_MIN < R2_HI_SPAN;
+}
+
+// t[u] = fl(G / fl(fl(r * r) * r)) with r = fl(sqrt(r2[u])), for
+// r2_in_range(r2[u]) and numerator_in_range(G).  Square root: Goldschmidt
+// steps from v_rsq_f64, then two residual corrections (fma(-s, s, x) is
+// exact).  Division by d = r^3: the half reciprocal root h gives 1/d to about
+// 2^-49 as (2 h)^3, one Newton step brings it to half an ulp, and the
+// quotient's exact remainder corrects the quotient (Markstein's theorem).
+// K independent values step by step: an FP64 result is ready 12 cycles after
+// its issue and issues every 4 to 5, so one chain alone leaves the unit idle.
+template <int K>
+__device__ __forceinline__ void over_r3(double G, const double (&r2)[K], double (&t)[K])
+{
+    double h[K], s[K], e[K], d[K], y[K], q[K];
+#define GS_EACH _Pragma("unroll") for (int u = 0; u < K; u++)
+    GS_EACH y[u] = __builtin_amdgcn_rsq(r2[u]);
+    GS_EACH h[u] = 0.5 * y[u];
+    GS_EACH s[u] = r2[u] * y[u];
+    GS_EACH e[u] = __builtin_fma(-h[u], s[u], 0.5);
+    GS_EACH h[u] = __builtin_fma(h[u], e[u], h[u]);
+    GS_EACH s[u] = __builtin_fma(s[u], e[u], s[u]);
+    GS_EACH e[u] = __builtin_fma(-s[u], s[u], r2[u]);
+    GS_EACH s[u] = __builtin_fma(e[u], h[u], s[u]);
+    GS_EACH e[u] = __builtin_fma(-s[u], s[u], r2[u]);
+    GS_EACH s[u] = __builtin_fma(e[u], h[u], s[u]);
+    GS_EACH h[u] = h[u] + h[u];
+    GS_EACH d[u] = s[u] * s[u];
+    GS_EACH y[u] = h[u] * h[u];
+    GS_EACH d[u] = d[u] * s[u];
+    GS_EACH y[u] = y[u] * h[u];
+    GS_EACH e[u] = __builtin_fma(-d[u], y[u], 1.0);
+    GS_EACH y[u] = __builtin_fma(y[u], e[u], y[u]);
+    GS_EACH q[u] = G * y[u];
+    GS_EACH e[u] = __builtin_fma(-d[u], q[u], G);
+    GS_EACH t[u] = __builtin_fma(e[u], y[u], q[u]);
+#undef GS_EACH
+}
+
+// The same for any operands.
+__device__ __forceinline__ double over_r3_any(double G, double r2)
+{
+    const double r = __builtin_sqrt(r2);
+    return G / ((r * r) * r);
+}
+
+}  // namespace gs

@@ -138,19 +138,16 @@ hipError_t launch_direct_f64_sampled(Context *c, const double *x, const double *
                                      double eps, bool skip_massless, const int *targets, int nt,
                                      double *out, void *buf, size_t bytes);
 size_t direct_f64_sampled_bytes(int n, int nt);
-// FP64 reference-order sums for the listed targets.
-hipError_t launch_direct_f64_targets(Context *c, const double *x, const double *m, int n,
-                                     double G, double eps, bool skip_massless, const int *targets,
-                                     int num_targets, double *out);
 Fp32Config &fp32_config();
 
 // FP64 energy (src/utils.c:27-59 formula; reduction order differs).
 hipError_t launch_energy(Context *c, const double *x, const double *v, const double *m, int n,
                          double G, double *partials, int *num_partials);
 
-// One Leapfrog step with the FP64 direct sum in one launch: drift (x, xe, v)
-// into (xo, xeo), forces of the drifted positions into a, kick v into vo with
-// ve updated in place -- the arithmetic of launch_lf_drift, launch_direct_f64
+// One Leapfrog step with the FP64 direct sum (one launch; for many particles
+// the drift, then the sums with the kick): drift (x, xe, v) into (xo, xeo),
+// forces of the drifted positions into a, kick v into vo with ve updated in
+// place -- the arithmetic of launch_lf_drift, launch_direct_f64
 // and launch_lf_kick in that order.  The output buffers must not alias the
 // inputs.
 hipError_t launch_lf_step_f64(Context *c, const double *x, const double *xe, const double *v,
