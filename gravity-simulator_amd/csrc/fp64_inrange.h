@@ -73,4 +73,21 @@ __device__ __forceinline__ double over_r3_any(double G, double r2)
     return G / ((r * r) * r);
 }
 
+// z / b for a constant b > 1 with y = RN(1 / b), correctly rounded with one
+// multiply and two FMAs instead of a full division (Markstein's theorem: with
+// q = RN(z y) within an ulp of z / b, the remainder r = z - b q is exact and
+// RN(q + r y) = RN(z / b)).  Quotients near the subnormal range, where the
+// remainder can be inexact, take the division itself, and so do infinities
+// and NaN.
+__device__ __forceinline__ double div_const(double z, double b, double y)
+{
+    const double az = fabs(z);
+    if (!(az >= 0x1p-900 && az < 0x1p1000)) return z / b;
+    const double q = z * y;
+    const double r = __builtin_fma(-q, b, z);
+    return __builtin_fma(r, y, q);
+}
+
+#define GS_DIVC(z, b) ::gs::div_const((z), (b), 1.0 / (b))
+
 }  // namespace gs

@@ -12,6 +12,7 @@
 
 #include "gs_internal.h"
 #include "ias15_coeffs.h"
+#include "small_n.h"
 
 #pragma clang fp contract(off)
 
@@ -27,37 +28,32 @@ struct IasK {
 
 #define AT(arr, slot) (arr)[static_cast<size_t>(slot) * n3 + q]
 
-// predictor at spacing h (src/integrator_ias15.c:808-919)
-__global__ void k_ias_predict(double *__restrict__ x1, double *__restrict__ v1,
-                              const double *__restrict__ x, const double *__restrict__ v,
-                              const double *__restrict__ a, const double *__restrict__ b,
-                              const double *__restrict__ xc, const double *__restrict__ vc,
-                              double h, double dt, size_t n3)
+// predicted position at spacing h (src/integrator_ias15.c:808-875; the
+// predicted velocity, :877-919, enters no force and is not formed)
+__device__ __forceinline__ double ias_predicted(double x, double v, double a, double xc,
+                                                const double (&b)[7], double h, double dt)
+{
+    double px = GS_DIVC(b[5], 28.0) + GS_DIVC(h * b[6], 36.0);
+    px = GS_DIVC(b[4], 21.0) + h * px;
+    px = GS_DIVC(b[3], 15.0) + h * px;
+    px = GS_DIVC(b[2], 10.0) + h * px;
+    px = GS_DIVC(b[1], 6.0) + h * px;
+    px = GS_DIVC(b[0], 3.0) + h * px;
+    px = a + h * px;
+    double xn = x;
+    xn += xc + dt * h * (v + dt * h * px / 2.0);
+    return xn;
+}
+
+__global__ void k_ias_predict(double *__restrict__ x1, const double *__restrict__ x,
+                              const double *__restrict__ v, const double *__restrict__ a,
+                              const double *__restrict__ b, const double *__restrict__ xc, double h,
+                              double dt, size_t n3)
 {
     const size_t q = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
     if (q >= n3) return;
-    const double b0 = AT(b, 0), b1 = AT(b, 1), b2 = AT(b, 2), b3 = AT(b, 3), b4 = AT(b, 4),
-                 b5 = AT(b, 5), b6 = AT(b, 6);
-    double px = b5 / 28.0 + h * b6 / 36.0;
-    px = b4 / 21.0 + h * px;
-    px = b3 / 15.0 + h * px;
-    px = b2 / 10.0 + h * px;
-    px = b1 / 6.0 + h * px;
-    px = b0 / 3.0 + h * px;
-    px = a[q] + h * px;
-    double xn = x[q];
-    xn += xc[q] + dt * h * (v[q] + dt * h * px / 2.0);
-    x1[q] = xn;
-
-    double pv = b5 / 7.0 + h * b6 / 8.0;
-    pv = b4 / 6.0 + h * pv;
-    pv = b3 / 5.0 + h * pv;
-    pv = b2 / 4.0 + h * pv;
-    pv = b1 / 3.0 + h * pv;
-    pv = b0 / 2.0 + h * pv;
-    double vn = v[q];
-    vn += vc[q] + dt * h * (a[q] + h * pv);
-    v1[q] = vn;
+    const double bl[7] = {AT(b, 0), AT(b, 1), AT(b, 2), AT(b, 3), AT(b, 4), AT(b, 5), AT(b, 6)};
+    x1[q] = ias_predicted(x[q], v[q], a[q], xc[q], bl, h, dt);
 }
 
 // g (divided differences of the forces F at spacings 0..i) and b after the
@@ -153,6 +149,25 @@ __global__ __launch_bounds__(IAS_BLOCK) void k_absmax2(const double *__restrict_
 
 // end point of the step with compensated sums (src/integrator_ias15.c:921-983);
 // the compensation terms start from the accepted ones (txc = xc + ...)
+__device__ __forceinline__ void ias_end_point(double x, double v, double a, double xc, double vc,
+                                              const double (&b)[7], double dt, double &x1,
+                                              double &v1, double &cx, double &cv)
+{
+    const double sx = a + b[0] / 3.0 + b[1] / 6.0 + b[2] / 10.0 + b[3] / 15.0 + b[4] / 21.0 +
+                      b[5] / 28.0 + b[6] / 36.0;
+    cx = xc;
+    cx += dt * (v + dt * sx / 2.0);
+    x1 = x + cx;
+    cx += (x - x1);
+
+    const double sv = a + b[0] / 2.0 + b[1] / 3.0 + b[2] / 4.0 + b[3] / 5.0 + b[4] / 6.0 +
+                      b[5] / 7.0 + b[6] / 8.0;
+    cv = vc;
+    cv += dt * sv;
+    v1 = v + cv;
+    cv += (v - v1);
+}
+
 __global__ void k_ias_step(double *__restrict__ x1, double *__restrict__ v1,
                            double *__restrict__ txc, double *__restrict__ tvc,
                            const double *__restrict__ x, const double *__restrict__ v,
@@ -162,52 +177,43 @@ __global__ void k_ias_step(double *__restrict__ x1, double *__restrict__ v1,
 {
     const size_t q = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
     if (q >= n3) return;
-    const double b0 = AT(b, 0), b1 = AT(b, 1), b2 = AT(b, 2), b3 = AT(b, 3), b4 = AT(b, 4),
-                 b5 = AT(b, 5), b6 = AT(b, 6);
-    const double sx = a[q] + b0 / 3.0 + b1 / 6.0 + b2 / 10.0 + b3 / 15.0 + b4 / 21.0 + b5 / 28.0 +
-                      b6 / 36.0;
-    double cx = xc[q];
-    cx += dt * (v[q] + dt * sx / 2.0);
-    const double xn = x[q] + cx;
-    cx += (x[q] - xn);
-    x1[q] = xn;
-    txc[q] = cx;
-
-    const double sv = a[q] + b0 / 2.0 + b1 / 3.0 + b2 / 4.0 + b3 / 5.0 + b4 / 6.0 + b5 / 7.0 +
-                      b6 / 8.0;
-    double cv = vc[q];
-    cv += dt * sv;
-    const double vn = v[q] + cv;
-    cv += (v[q] - vn);
-    v1[q] = vn;
-    tvc[q] = cv;
+    const double bl[7] = {AT(b, 0), AT(b, 1), AT(b, 2), AT(b, 3), AT(b, 4), AT(b, 5), AT(b, 6)};
+    ias_end_point(x[q], v[q], a[q], xc[q], vc[q], bl, dt, x1[q], v1[q], txc[q], tvc[q]);
 }
 
-// b for the next step (src/integrator_ias15.c:1276-1382)
+// b for the next step (src/integrator_ias15.c:1276-1382): b in place, en the new e
+__device__ __forceinline__ void ias_refined(double (&b)[7], const double (&e)[7], double q1,
+                                            int refine, double (&en)[7])
+{
+    const double q2 = q1 * q1, q3 = q2 * q1, q4 = q3 * q1, q5 = q4 * q1, q6 = q5 * q1,
+                 q7 = q6 * q1;
+    double db[7];
+#pragma unroll
+    for (int j = 0; j < 7; j++) db[j] = refine ? b[j] - e[j] : 0.0;
+    en[0] = q1 * (b[6] * 7.0 + b[5] * 6.0 + b[4] * 5.0 + b[3] * 4.0 + b[2] * 3.0 + b[1] * 2.0 + b[0]);
+    en[1] = q2 * (b[6] * 21.0 + b[5] * 15.0 + b[4] * 10.0 + b[3] * 6.0 + b[2] * 3.0 + b[1]);
+    en[2] = q3 * (b[6] * 35.0 + b[5] * 20.0 + b[4] * 10.0 + b[3] * 4.0 + b[2]);
+    en[3] = q4 * (b[6] * 35.0 + b[5] * 15.0 + b[4] * 5.0 + b[3]);
+    en[4] = q5 * (b[6] * 21.0 + b[5] * 6.0 + b[4]);
+    en[5] = q6 * (b[6] * 7.0 + b[5]);
+    en[6] = q7 * b[6];
+#pragma unroll
+    for (int j = 0; j < 7; j++) b[j] = en[j] + db[j];
+}
+
 __global__ void k_ias_refine(double *__restrict__ b, double *__restrict__ e, double q1, int refine,
                              size_t n3)
 {
     const size_t q = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
     if (q >= n3) return;
-    const double q2 = q1 * q1, q3 = q2 * q1, q4 = q3 * q1, q5 = q4 * q1, q6 = q5 * q1,
-                 q7 = q6 * q1;
-    double db[7];
+    double bl[7], el[7], en[7];
 #pragma unroll
-    for (int j = 0; j < 7; j++) db[j] = refine ? AT(b, j) - AT(e, j) : 0.0;
-    const double b0 = AT(b, 0), b1 = AT(b, 1), b2 = AT(b, 2), b3 = AT(b, 3), b4 = AT(b, 4),
-                 b5 = AT(b, 5), b6 = AT(b, 6);
-    double en[7];
-    en[0] = q1 * (b6 * 7.0 + b5 * 6.0 + b4 * 5.0 + b3 * 4.0 + b2 * 3.0 + b1 * 2.0 + b0);
-    en[1] = q2 * (b6 * 21.0 + b5 * 15.0 + b4 * 10.0 + b3 * 6.0 + b2 * 3.0 + b1);
-    en[2] = q3 * (b6 * 35.0 + b5 * 20.0 + b4 * 10.0 + b3 * 4.0 + b2);
-    en[3] = q4 * (b6 * 35.0 + b5 * 15.0 + b4 * 5.0 + b3);
-    en[4] = q5 * (b6 * 21.0 + b5 * 6.0 + b4);
-    en[5] = q6 * (b6 * 7.0 + b5);
-    en[6] = q7 * b6;
+    for (int j = 0; j < 7; j++) bl[j] = AT(b, j), el[j] = AT(e, j);
+    ias_refined(bl, el, q1, refine, en);
 #pragma unroll
     for (int j = 0; j < 7; j++) {
         AT(e, j) = en[j];
-        AT(b, j) = en[j] + db[j];
+        AT(b, j) = bl[j];
     }
 }
 
@@ -223,6 +229,101 @@ __global__ void k_ias_sub(double *__restrict__ a1, const double *__restrict__ a,
 {
     const size_t q = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
     if (q < n3) a1[q] = a1[q] - a[q];
+}
+
+// One step attempt of a small system in one workgroup: (after an accepted
+// attempt) the refinement of b, the corrector iterations to convergence, the
+// end point, the acceleration there and the two maxima of the error estimate,
+// which go to host memory -- the kernels above in their order, thread q
+// holding component q, so every value is the same.  The predictor's
+// velocities are not formed (the forces do not read them), the force at
+// spacing 0 once (x + xc in every iteration), and of the divided differences
+// at spacing i only the one that changed.
+// Bound by latency: a stage is a chain of about 100 dependent FP64 operations
+// of 12 cycles and three barriers.  One MI355X, a run of 26 steps of 9 bodies:
+// 31.0 ms with three launches a stage, 3.0 ms here; 82 steps of 64: 77.8 and
+// 22.2; 111 steps of 128: 118 and 96 (SN_MAX: beyond it one CU's pairs cost
+// more than the launches).
+struct IasSmall {
+    double *x, *v, *m, *a, *x1, *v1, *a1, *g, *b, *b06, *e, *xc, *vc, *txc, *tvc;
+    double *out;  // host memory: max |b6|, max |a1|
+    double G, eps2, dt, q1;
+    int skip_massless, accepted, refine;
+    double h[8];
+    IasK k;
+};
+
+__global__ __launch_bounds__(1024) void k_ias_attempt(IasSmall A, SmallN sn)
+{
+    extern __shared__ double lds[];
+    const SmallNLds w(lds, sn);
+    const size_t n3 = 3 * static_cast<size_t>(sn.n);
+    const size_t q = threadIdx.x;
+    const bool live = q < n3;
+    double b[7], g[7], x = 0.0, v = 0.0, a = 0.0, xc = 0.0, vc = 0.0, b06 = 0.0;
+#pragma unroll
+    for (int j = 0; j < 7; j++) b[j] = g[j] = 0.0;
+    if (live) {
+        x = A.x[q], v = A.v[q], a = A.a[q], xc = A.xc[q], vc = A.vc[q], b06 = A.b06[q];
+#pragma unroll
+        for (int j = 0; j < 7; j++) b[j] = AT(A.b, j), g[j] = AT(A.g, j);
+        if (A.accepted) {
+            double en[7], e[7];
+#pragma unroll
+            for (int j = 0; j < 7; j++) e[j] = AT(A.e, j);
+            ias_refined(b, e, A.q1, A.refine, en);
+#pragma unroll
+            for (int j = 0; j < 7; j++) AT(A.e, j) = en[j];
+        }
+    }
+    for (int i = threadIdx.x; i < sn.n; i += blockDim.x) w.m[i] = A.m[i];
+    const double dt = A.dt;
+    double f0 = 0.0;
+    for (int it = 0; it < 12; it++) {
+        double f = 0.0;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            if (i == 0 && it > 0) continue;
+            if (live) w.x[q] = ias_predicted(x, v, a, xc, b, A.h[i], dt);
+            f = small_n_force(sn, w, A.G, A.eps2, A.skip_massless != 0);
+            if (i == 0) {
+                f0 = f;
+                continue;
+            }
+            double t = (f - f0) * A.k.r[i][0];
+#pragma unroll
+            for (int l = 1; l < i; l++) t = (t - g[l - 1]) * A.k.r[i][l];
+            g[i - 1] = t;
+#pragma unroll
+            for (int j = 0; j < i; j++) {
+                double s = A.k.c[j][j] * g[j];
+#pragma unroll
+                for (int l = j + 1; l < 7; l++) s = s + A.k.c[l][j] * g[l];
+                b[j] = s;
+            }
+        }
+        double md = live ? fmax(0.0, fabs(b[6] - b06)) : 0.0, ma = live ? fmax(0.0, fabs(f)) : 0.0;
+        b06 = b[6];
+        small_n_max2(w, md, ma);
+        if (md / ma < 1e-16) break;
+    }
+    double x1 = 0.0, v1 = 0.0, cx = 0.0, cv = 0.0;
+    if (live) {
+        ias_end_point(x, v, a, xc, vc, b, dt, x1, v1, cx, cv);
+        w.x[q] = x1;
+    }
+    const double a1 = small_n_force(sn, w, A.G, A.eps2, A.skip_massless != 0);
+    double mb = live ? fmax(0.0, fabs(b[6])) : 0.0, ma = live ? fmax(0.0, fabs(a1)) : 0.0;
+    small_n_max2(w, mb, ma);
+    if (live) {
+        A.x1[q] = x1, A.v1[q] = v1, A.txc[q] = cx, A.tvc[q] = cv, A.a1[q] = a1, A.b06[q] = b06;
+#pragma unroll
+        for (int j = 0; j < 7; j++) AT(A.b, j) = b[j], AT(A.g, j) = g[j];
+    }
+    if (threadIdx.x == 0) {
+        A.out[0] = mb;
+        A.out[1] = ma;
+    }
 }
 
 #undef AT
@@ -378,32 +479,65 @@ ErrorStatus ias15_gpu(System *system, IntegratorParam *ip, AccelerationParam *ap
     status->dt = dt;
     status->num_steps = 0;
     bool refine_flag = false;
+    // small systems with the FP64 direct sums: an attempt is one launch, the
+    // refinement after an accepted one at the start of the next
+    const bool small = n <= SN_MAX && (ap->method == ACCELERATION_METHOD_PAIRWISE ||
+                                       ap->method == ACCELERATION_METHOD_MASSLESS);
+    SmallN sn;
+    IasSmall A;
+    const double *hmax = nullptr;
+    if (small) {
+        void *hp;
+        GS_TRY(pinned(c, 64, &hp));
+        hmax = static_cast<const double *>(hp);
+        sn = SmallN::plan(n);
+        A.m = S.m, A.g = S.g, A.b = S.b, A.b06 = S.b0 + 6 * n3, A.e = S.e;
+        A.out = static_cast<double *>(hp);
+        A.G = G, A.eps2 = ap->softening_length * ap->softening_length;
+        A.skip_massless = ap->method == ACCELERATION_METHOD_MASSLESS;
+        A.accepted = 0, A.refine = 0, A.q1 = 1.0;
+        for (int i = 0; i < 8; i++) A.h[i] = K.h[i];
+        A.k = k;
+    }
     while (status->t < tf) {
-        for (int it = 0; it < 12; it++) {
-            for (int i = 0; i < 8; i++) {
-                hipLaunchKernelGGL(k_ias_predict, grid, block, 0, c->stream, S.x1, S.v1, S.x, S.v,
-                                   S.a, S.b, S.xc, S.vc, K.h[i], dt, n3);
-                GS_HIP(hipGetLastError());
-                GS_TRY(device_acceleration(c, S.x1, S.m, n, G, ap, S.F + i * n3));
-                hipLaunchKernelGGL(k_ias_gb, grid, block, 0, c->stream, S.g, S.b, S.F, i, k, n3);
-                GS_HIP(hipGetLastError());
-            }
-            hipLaunchKernelGGL(k_ias_conv, rgrid, block, 0, c->stream, S.b, S.b0, S.F + 7 * n3,
-                               S.part, n3);
-            GS_HIP(hipGetLastError());
-            double md, ma;
-            GS_TRY(S.maxima(&md, &ma));
-            if ((md / ma) < tolerance_pc) break;
-        }
-
-        hipLaunchKernelGGL(k_ias_step, grid, block, 0, c->stream, S.x1, S.v1, S.txc, S.tvc, S.x,
-                           S.v, S.a, S.b, S.xc, S.vc, dt, n3);
-        GS_HIP(hipGetLastError());
-        GS_TRY(device_acceleration(c, S.x1, S.m, n, G, ap, S.a1));
-        hipLaunchKernelGGL(k_ias_errmax, rgrid, block, 0, c->stream, S.b, S.a1, S.part, n3);
-        GS_HIP(hipGetLastError());
         double mb, ma1;
-        GS_TRY(S.maxima(&mb, &ma1));
+        if (small) {
+            A.x = S.x, A.v = S.v, A.a = S.a, A.x1 = S.x1, A.v1 = S.v1, A.a1 = S.a1;
+            A.xc = S.xc, A.vc = S.vc, A.txc = S.txc, A.tvc = S.tvc;
+            A.dt = dt;
+            hipLaunchKernelGGL(k_ias_attempt, dim3(1), dim3(sn.block), sn.lds, c->stream, A, sn);
+            GS_HIP(hipGetLastError());
+            GS_HIP(hipStreamSynchronize(c->stream));
+            mb = hmax[0];
+            ma1 = hmax[1];
+            A.accepted = 0;
+        } else {
+            for (int it = 0; it < 12; it++) {
+                // (the force at spacing 0, at x + xc, is the first iteration's)
+                for (int i = it == 0 ? 0 : 1; i < 8; i++) {
+                    hipLaunchKernelGGL(k_ias_predict, grid, block, 0, c->stream, S.x1, S.x, S.v, S.a,
+                                       S.b, S.xc, K.h[i], dt, n3);
+                    GS_HIP(hipGetLastError());
+                    GS_TRY(device_acceleration(c, S.x1, S.m, n, G, ap, S.F + i * n3));
+                    hipLaunchKernelGGL(k_ias_gb, grid, block, 0, c->stream, S.g, S.b, S.F, i, k, n3);
+                    GS_HIP(hipGetLastError());
+                }
+                hipLaunchKernelGGL(k_ias_conv, rgrid, block, 0, c->stream, S.b, S.b0, S.F + 7 * n3,
+                                   S.part, n3);
+                GS_HIP(hipGetLastError());
+                double md, ma;
+                GS_TRY(S.maxima(&md, &ma));
+                if ((md / ma) < tolerance_pc) break;
+            }
+
+            hipLaunchKernelGGL(k_ias_step, grid, block, 0, c->stream, S.x1, S.v1, S.txc, S.tvc, S.x,
+                               S.v, S.a, S.b, S.xc, S.vc, dt, n3);
+            GS_HIP(hipGetLastError());
+            GS_TRY(device_acceleration(c, S.x1, S.m, n, G, ap, S.a1));
+            hipLaunchKernelGGL(k_ias_errmax, rgrid, block, 0, c->stream, S.b, S.a1, S.part, n3);
+            GS_HIP(hipGetLastError());
+            GS_TRY(S.maxima(&mb, &ma1));
+        }
         const double error_b7 = mb / ma1;
         double error = pow((error_b7 / tolerance), exponent);
         if (error < 1e-10) error = 1e-10;
@@ -412,9 +546,15 @@ ErrorStatus ias15_gpu(System *system, IntegratorParam *ip, AccelerationParam *ap
         if (error <= 1.0 || dt == tf * 1e-12) {
             status->num_steps++;
             status->t += dt;
-            hipLaunchKernelGGL(k_ias_refine, grid, block, 0, c->stream, S.b, S.e, dt_new / dt,
-                               refine_flag ? 1 : 0, n3);
-            GS_HIP(hipGetLastError());
+            if (small) {
+                A.accepted = 1;
+                A.q1 = dt_new / dt;
+                A.refine = refine_flag ? 1 : 0;
+            } else {
+                hipLaunchKernelGGL(k_ias_refine, grid, block, 0, c->stream, S.b, S.e, dt_new / dt,
+                                   refine_flag ? 1 : 0, n3);
+                GS_HIP(hipGetLastError());
+            }
             refine_flag = true;
             // accepted: the trial state and its compensation terms become current
             std::swap(S.xc, S.txc);

@@ -22,6 +22,7 @@
 #include <numeric>
 #include <vector>
 
+#include "fp64_inrange.h"
 #include "gs_internal.h"
 
 #pragma clang fp contract(off)
@@ -58,21 +59,8 @@ __device__ __forceinline__ double norm3(double a, double b, double c)
     return __builtin_sqrt(a * a + b * b + c * c);
 }
 
-// z / b for the constant divisors of the Stumpff series, correctly rounded
-// with one multiply and two FMAs instead of a full division (Markstein's
-// theorem: with y = RN(1/b) and q = RN(z y) within an ulp of z / b, the
-// remainder r = z - b q is exact and RN(q + r y) = RN(z / b)).  Quotients
-// near the subnormal range, where the remainder can be inexact, take the
-// division itself.
-__device__ __forceinline__ double div_const(double z, double b, double y)
-{
-    if (!(fabs(z) >= 0x1p-900)) return z / b;
-    const double q = z * y;
-    const double r = __builtin_fma(-q, b, z);
-    return __builtin_fma(r, y, q);
-}
-
-#define DIVC(z, b) div_const((z), (b), 1.0 / (b))
+// (the Stumpff series' constant divisors)
+#define DIVC(z, b) GS_DIVC(z, b)
 
 // src/integrator_whfast.c:774-815
 __device__ void stumpff(double z, double &c0, double &c1, double &c2, double &c3)

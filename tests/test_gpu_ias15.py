@@ -55,3 +55,19 @@ def test_ias15_n1024_bitwise_and_energy():
     e0, e1 = O.energy(x, v, m, 1.0), O.energy(xg, vg, mg, 1.0)
     print(f"N=1024 IAS15 to t=0.05: {steps} steps, |dE/E| {abs(e1 - e0) / abs(e0):.2e}")
     assert abs(e1 - e0) / abs(e0) < 1e-5
+
+
+@pytest.mark.parametrize("n", [2, 5, 48, 49, 64, 85, 86, 128, 129])
+def test_ias15_one_workgroup_sizes_bitwise(n):
+    """Around the sizes where the one-workgroup step changes: its source tiles
+    (48 / 49), its wavefronts (85 / 86) and the limit beyond which every stage
+    is launched on its own (128 / 129)."""
+    x, v, m = ic.plummer(n, 40 + n)
+    for method in (1, 2):
+        if method == 2:
+            m[(n + 1) // 2:] = 0.0
+        ids, xg, vg, mg, steps = L.launch_simulation(x, v, m, 1.0, IAS15, -1.0, 0.05, method=method, eps=1e-2,
+                                                     tolerance=1e-9, initial_dt=1e-2)
+        xo, vo, so = O.ias15(x, v, m, 1.0, 1e-9, 0.05, eps=1e-2, method=method, initial_dt=1e-2)
+        assert steps == so
+        assert np.array_equal(xg, xo) and np.array_equal(vg, vo)
