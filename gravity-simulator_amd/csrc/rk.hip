@@ -15,6 +15,7 @@
 
 #include "gs_internal.h"
 #include "rk_tableaus.h"
+#include "small_n.h"
 
 #pragma clang fp contract(off)
 
@@ -121,10 +122,55 @@ struct RkWeights {
     double dw[RK_MAX_STAGES];  // weights - weights_test
 };
 
-// Embedded RK update and error terms (src/integrator_rk_embedded.c:786-853):
-// the propagated state with compensated sums into (x1, v1, txe, tve), and
-// per component the two squared scaled errors (velocity, then position) in
-// the order the reference sums them
+// Embedded RK update and error terms (src/integrator_rk_embedded.c:786-853)
+// of one component: the propagated state with compensated sums, and the two
+// squared scaled errors (velocity, then position)
+struct RkeSums {
+    double sv = 0.0, sx = 0.0, ev = 0.0, ex = 0.0;
+    __device__ __forceinline__ void add(double wgt, double dw, double dt, double vks, double xks)
+    {
+        sv += wgt * vks;
+        sx += wgt * xks;
+        ev += dt * dw * vks;
+        ex += dt * dw * xks;
+    }
+};
+
+__device__ __forceinline__ void rke_finish(const RkeSums &S, double xq, double vq, double xe,
+                                           double ve, double dt, double tol, double &x1, double &v1,
+                                           double &txe, double &tve, double &e0, double &e1)
+{
+    double tv = ve, tx = xe;
+    tv += dt * S.sv;
+    tx += dt * S.sx;
+    const double v1q = vq + tv, x1q = xq + tx;
+    tv += vq - v1q;
+    tx += xq - x1q;
+    v1 = v1q;
+    x1 = x1q;
+    tve = tv;
+    txe = tx;
+    const double scv = tol + fmax(fabs(vq), fabs(v1q)) * tol;
+    const double scx = tol + fmax(fabs(xq), fabs(x1q)) * tol;
+    const double q0 = S.ev / scv, q1 = S.ex / scx;
+    e0 = q0 * q0;
+    e1 = q1 * q1;
+}
+
+template <int ST>
+__device__ __forceinline__ void rke_propagated(double x, double v, double xe, double ve,
+                                               const double (&xk)[ST], const double (&vk)[ST],
+                                               const RkWeights &W, double dt, double tol, double &x1,
+                                               double &v1, double &txe, double &tve, double &e0,
+                                               double &e1)
+{
+    RkeSums S;
+#pragma unroll
+    for (int s = 0; s < ST; s++) S.add(W.w[s], W.dw[s], dt, vk[s], xk[s]);
+    rke_finish(S, x, v, xe, ve, dt, tol, x1, v1, txe, tve, e0, e1);
+}
+
+// the same over the stage arrays; terms in the order the reference sums them
 __global__ void k_rke_final(double *__restrict__ x1, double *__restrict__ v1,
                             double *__restrict__ txe, double *__restrict__ tve,
                             double *__restrict__ terms, const double *__restrict__ x,
@@ -135,30 +181,10 @@ __global__ void k_rke_final(double *__restrict__ x1, double *__restrict__ v1,
 {
     const size_t q = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
     if (q >= n3) return;
-    double sv = 0.0, sx = 0.0, ev = 0.0, ex = 0.0;
-    for (int s = 0; s < S; s++) {
-        const double vks = vk[s * n3 + q], xks = xk[s * n3 + q];
-        sv += W.w[s] * vks;
-        sx += W.w[s] * xks;
-        ev += dt * W.dw[s] * vks;
-        ex += dt * W.dw[s] * xks;
-    }
-    const double vq = v[q], xq = x[q];
-    double tv = ve[q], tx = xe[q];
-    tv += dt * sv;
-    tx += dt * sx;
-    const double v1q = vq + tv, x1q = xq + tx;
-    tv += vq - v1q;
-    tx += xq - x1q;
-    v1[q] = v1q;
-    x1[q] = x1q;
-    tve[q] = tv;
-    txe[q] = tx;
-    const double scv = tol + fmax(fabs(vq), fabs(v1q)) * tol;
-    const double scx = tol + fmax(fabs(xq), fabs(x1q)) * tol;
-    const double e0 = ev / scv, e1 = ex / scx;
-    terms[2 * q] = e0 * e0;
-    terms[2 * q + 1] = e1 * e1;
+    RkeSums sum;
+    for (int s = 0; s < S; s++) sum.add(W.w[s], W.dw[s], dt, vk[s * n3 + q], xk[s * n3 + q]);
+    rke_finish(sum, x[q], v[q], xe[q], ve[q], dt, tol, x1[q], v1[q], txe[q], tve[q], terms[2 * q],
+               terms[2 * q + 1]);
 }
 
 // Initial-step terms (src/integrator_rk_embedded.c:408-437): per component
@@ -203,22 +229,102 @@ __global__ void k_rke_init_terms2(double *__restrict__ t2, const double *__restr
     t2[2 * q + 1] = da * da;
 }
 
-// Sum of `count` terms in index order by one lane (the reference's
-// sequential sums, rounding included); the loads run ahead of the adds.
-__global__ void k_seq_sum(const double *__restrict__ terms, size_t count, double *__restrict__ out)
+// Sum of `count` terms in index order (the reference's sequential sums,
+// rounding included) into *out: the workgroup stages the terms in LDS, one
+// lane adds them.  Bound by the chain of additions, 12 cycles each on gfx950:
+// 6144 terms (1024 particles) take 35 us, of which the chain alone is 31; one
+// lane loading from device memory between its additions took 185.
+constexpr int SEQ_TILE = 4096;
+
+__global__ __launch_bounds__(RK_BLOCK) void k_seq_sum(const double *__restrict__ terms, size_t count,
+                                                      double *__restrict__ out)
 {
-    if (threadIdx.x != 0) return;
+    __shared__ __align__(16) double buf[SEQ_TILE];
     double s = 0.0;
-    size_t k = 0;
-    for (; k + 8 <= count; k += 8) {
-        double t[8];
+    for (size_t base = 0; base < count; base += SEQ_TILE) {
+        const int cnt = static_cast<int>(count - base < SEQ_TILE ? count - base : SEQ_TILE);
+        __syncthreads();
+        for (int k = threadIdx.x; k < cnt; k += RK_BLOCK) buf[k] = terms[base + k];
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int k = 0;
+            for (; k + 32 <= cnt; k += 32)
 #pragma unroll
-        for (int j = 0; j < 8; j++) t[j] = terms[k + j];
-#pragma unroll
-        for (int j = 0; j < 8; j++) s += t[j];
+                for (int j = 0; j < 32; j += 2) {
+                    const double2 t = *reinterpret_cast<const double2 *>(&buf[k + j]);
+                    s += t.x;
+                    s += t.y;
+                }
+            for (; k < cnt; k++) s += buf[k];
+        }
     }
-    for (; k < count; k++) s += terms[k];
-    *out = s;
+    if (threadIdx.x == 0) *out = s;
+}
+
+// One step attempt of an embedded method for a small system in one
+// workgroup: the stages, the propagated state and the error sum, thread q
+// holding component q, with the operations of k_rke_stage, k_rke_final and
+// k_seq_sum in their order.  The sum goes to host memory.  DOPRI runs on one
+// MI355X, as 17 launches a step and here: 9 bodies (16 steps) 1.60 -> 0.43 ms,
+// 64 (25 steps) 2.48 -> 1.30, 96 (18) 1.98 -> 1.61, 128 (39) 4.0 -> 4.9 ms:
+// hence the limit.
+constexpr int RKE_SMALL_MAX = 96;
+static_assert(RKE_SMALL_MAX <= SN_MAX, "the one-workgroup force's limit");
+
+struct RkeSmall {
+    const double *x, *v, *m, *xe, *ve;
+    double *x1, *v1, *txe, *tve;
+    double *out;  // host memory: the error sum
+    double G, eps2, dt, tol;
+    int skip_massless;
+    double coeff[(RK_MAX_STAGES - 1) * (RK_MAX_STAGES - 1)];
+    RkWeights W;
+};
+
+template <int ST>
+__global__ __launch_bounds__(1024) void k_rke_attempt(RkeSmall A, SmallN sn)
+{
+    extern __shared__ double lds[];
+    const SmallNLds w(lds, sn);
+    const int q = threadIdx.x;
+    const bool live = q < 3 * sn.n;
+    double x = 0.0, v = 0.0, xe = 0.0, ve = 0.0;
+    if (live) x = A.x[q], v = A.v[q], xe = A.xe[q], ve = A.ve[q];
+    for (int i = q; i < sn.n; i += blockDim.x) w.m[i] = A.m[i];
+    const double dt = A.dt;
+    double xk[ST], vk[ST];
+#pragma unroll
+    for (int s = 0; s < ST; s++) {
+        if (s == 0) {
+            xk[0] = v;
+            if (live) w.x[q] = x;
+        } else {
+            double sv = 0.0, sx = 0.0;
+#pragma unroll
+            for (int i = 0; i < s; i++) {
+                const double c = A.coeff[(s - 1) * (ST - 1) + i];
+                sv += c * vk[i];
+                sx += c * xk[i];
+            }
+            xk[s] = v + dt * sv + ve;
+            if (live) w.x[q] = x + dt * sx + xe;
+        }
+        vk[s] = small_n_force(sn, w, A.G, A.eps2, A.skip_massless != 0);
+    }
+    if (live) {
+        double e0, e1;
+        rke_propagated<ST>(x, v, xe, ve, xk, vk, A.W, dt, A.tol, A.x1[q], A.v1[q], A.txe[q], A.tve[q],
+                           e0, e1);
+        w.term[2 * q] = e0;
+        w.term[2 * q + 1] = e1;
+    }
+    __syncthreads();
+    if (q == 0) {
+        double s = 0.0;
+#pragma unroll 8
+        for (int k = 0; k < 6 * sn.n; k++) s += w.term[k];
+        *A.out = s;
+    }
 }
 
 namespace {
@@ -275,13 +381,11 @@ ErrorStatus check_args(System *system, AccelerationParam *ap)
     return make_success_error_status();
 }
 
-// sequential sum of `count` device terms, read back
-ErrorStatus seq_sum(Context *c, const double *terms, size_t count, double *dev_out,
-                    double *host_out)
+// sequential sum of `count` device terms into pinned host memory
+ErrorStatus seq_sum(Context *c, const double *terms, size_t count, double *host_out)
 {
-    hipLaunchKernelGGL(k_seq_sum, dim3(1), dim3(64), 0, c->stream, terms, count, dev_out);
+    hipLaunchKernelGGL(k_seq_sum, dim3(1), dim3(RK_BLOCK), 0, c->stream, terms, count, host_out);
     GS_HIP(hipGetLastError());
-    GS_HIP(hipMemcpyAsync(host_out, dev_out, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     GS_HIP(hipStreamSynchronize(c->stream));
     return make_success_error_status();
 }
@@ -418,11 +522,11 @@ ErrorStatus rk_embedded_gpu(System *system, IntegratorParam *ip, AccelerationPar
     RkState S;
     double *rest;
     const size_t n3 = static_cast<size_t>(n) * 3;
-    // x1, v1, xe, ve, txe, tve, tx (7 n3), xk, vk (2 St n3), terms (2 n3), sums
-    GS_TRY(S.alloc(c, n, (9 + 2 * static_cast<size_t>(St)) * n3 + 8, &rest));
+    // x1, v1, xe, ve, txe, tve, tx (7 n3), xk, vk (2 St n3), terms (2 n3)
+    GS_TRY(S.alloc(c, n, (9 + 2 * static_cast<size_t>(St)) * n3, &rest));
     double *x1 = rest, *v1 = x1 + n3, *xe = v1 + n3, *ve = xe + n3, *txe = ve + n3,
            *tve = txe + n3, *tx = tve + n3, *xk = tx + n3, *vk = xk + St * n3,
-           *terms = vk + St * n3, *dsum = terms + 2 * n3;
+           *terms = vk + St * n3;
     void *hp;
     GS_TRY(pinned(c, 64, &hp));
     double *hsum = static_cast<double *>(hp);
@@ -445,9 +549,9 @@ ErrorStatus rk_embedded_gpu(System *system, IntegratorParam *ip, AccelerationPar
                            tol, n3);
         GS_HIP(hipGetLastError());
         double s0, s1, s2;
-        GS_TRY(seq_sum(c, t0, 2 * n3, dsum, hsum));
+        GS_TRY(seq_sum(c, t0, 2 * n3, hsum));
         s0 = *hsum;
-        GS_TRY(seq_sum(c, t1, 2 * n3, dsum, hsum));
+        GS_TRY(seq_sum(c, t1, 2 * n3, hsum));
         s1 = *hsum;
         const double d0 = sqrt(s0 / (n * 6)), d1 = sqrt(s1 / (n * 6));
         const double dt0 = (d0 < 1e-5 || d1 < 1e-5) ? 1e-4 : d0 / d1;
@@ -457,7 +561,7 @@ ErrorStatus rk_embedded_gpu(System *system, IntegratorParam *ip, AccelerationPar
         hipLaunchKernelGGL(k_rke_init_terms2, grid, block, 0, c->stream, t0, tsx, tsv, v, pv, a,
                            a1, n3);
         GS_HIP(hipGetLastError());
-        GS_TRY(seq_sum(c, t0, 2 * n3, dsum, hsum));
+        GS_TRY(seq_sum(c, t0, 2 * n3, hsum));
         s2 = *hsum;
         const double d2 = sqrt(s2 / (n * 6)) / dt0;
         // (long-double intermediates rounded to double, as the reference's
@@ -475,21 +579,51 @@ ErrorStatus rk_embedded_gpu(System *system, IntegratorParam *ip, AccelerationPar
     double t = 0.0;
     long long steps = 0;
     RkRow row;
+    // small systems with the FP64 direct sums: an attempt is one launch
+    const bool small = n <= RKE_SMALL_MAX && (ap->method == ACCELERATION_METHOD_PAIRWISE ||
+                                       ap->method == ACCELERATION_METHOD_MASSLESS);
+    RkeSmall A;
+    SmallN sn;
+    if (small) {
+        sn = SmallN::plan(n);
+        A.m = S.m, A.out = hsum, A.G = G, A.tol = tol, A.W = W;
+        A.eps2 = ap->softening_length * ap->softening_length;
+        A.skip_massless = ap->method == ACCELERATION_METHOD_MASSLESS;
+        for (int i = 0; i < (St - 1) * (St - 1); i++) A.coeff[i] = T.coeff[i];
+    }
     while (t < tf) {
-        GS_TRY(device_acceleration(c, x, S.m, n, G, ap, vk));
-        GS_HIP(hipMemcpyAsync(xk, v, sizeof(double) * n3, hipMemcpyDeviceToDevice, c->stream));
-        for (int s = 1; s < St; s++) {
-            for (int i = 0; i < RK_MAX_STAGES; i++)
-                row.c[i] = i < s ? T.coeff[(s - 1) * (St - 1) + i] : 0.0;
-            hipLaunchKernelGGL(k_rke_stage, grid, block, 0, c->stream, tx, xk, vk, x, v, xe, ve,
-                               row, s, dt, n3);
+        if (small) {
+            A.x = x, A.v = v, A.xe = xe, A.ve = ve;
+            A.x1 = x1, A.v1 = v1, A.txe = txe, A.tve = tve;
+            A.dt = dt;
+            auto attempt = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(1), dim3(sn.block), sn.lds, c->stream, A, sn);
+            };
+            switch (St) {
+                case 6: attempt(k_rke_attempt<6>); break;
+                case 7: attempt(k_rke_attempt<7>); break;
+                case 8: attempt(k_rke_attempt<8>); break;
+                case 13: attempt(k_rke_attempt<13>); break;
+                default: return WRAP_RAISE_ERROR(GRAV_VALUE_ERROR, "Invalid integrator method");
+            }
             GS_HIP(hipGetLastError());
-            GS_TRY(device_acceleration(c, tx, S.m, n, G, ap, vk + s * n3));
+            GS_HIP(hipStreamSynchronize(c->stream));
+        } else {
+            GS_TRY(device_acceleration(c, x, S.m, n, G, ap, vk));
+            GS_HIP(hipMemcpyAsync(xk, v, sizeof(double) * n3, hipMemcpyDeviceToDevice, c->stream));
+            for (int s = 1; s < St; s++) {
+                for (int i = 0; i < RK_MAX_STAGES; i++)
+                    row.c[i] = i < s ? T.coeff[(s - 1) * (St - 1) + i] : 0.0;
+                hipLaunchKernelGGL(k_rke_stage, grid, block, 0, c->stream, tx, xk, vk, x, v, xe, ve,
+                                   row, s, dt, n3);
+                GS_HIP(hipGetLastError());
+                GS_TRY(device_acceleration(c, tx, S.m, n, G, ap, vk + s * n3));
+            }
+            hipLaunchKernelGGL(k_rke_final, grid, block, 0, c->stream, x1, v1, txe, tve, terms, x, v,
+                               xe, ve, xk, vk, W, St, dt, tol, n3);
+            GS_HIP(hipGetLastError());
+            GS_TRY(seq_sum(c, terms, 2 * n3, hsum));
         }
-        hipLaunchKernelGGL(k_rke_final, grid, block, 0, c->stream, x1, v1, txe, tve, terms, x, v,
-                           xe, ve, xk, vk, W, St, dt, tol, n3);
-        GS_HIP(hipGetLastError());
-        GS_TRY(seq_sum(c, terms, 2 * n3, dsum, hsum));
         double error = sqrt(*hsum / (n * 3 * 2));
         if (error <= 1 || dt <= tf * 1e-12) {
             steps++;

@@ -87,3 +87,19 @@ def test_rk4_fp32_forces_track_fp64():
     e32, e64 = O.energy(x32, v32, m, 1.0), O.energy(x64, v64, m, 1.0)
     print(f"RK4 N=4096 FP32 vs FP64 forces: max |dx| {dx:.2e}, energy rel. diff {abs(e32 - e64) / abs(e64):.2e}")
     assert dx < 1e-7 and abs(e32 - e64) / abs(e64) < 1e-8
+
+
+@pytest.mark.parametrize("integ", [5, 6, 7, 8])
+@pytest.mark.parametrize("n", [2, 49, 86, 96, 97, 700])
+def test_embedded_one_workgroup_sizes_and_sequential_sum_bitwise(integ, n):
+    """Around the sizes where the one-workgroup step changes (source tiles 48 / 49, wavefronts 85 / 86, the limit
+    96 / 97), and an error sum of more terms than one LDS tile holds (700 particles: 4200 terms)."""
+    x, v, m = ic.plummer(n, 60 + n)
+    tf = 0.02 if n < 200 else 0.001
+    for method in (1, 2):
+        if method == 2:
+            m[(n + 1) // 2:] = 0.0
+        r = L.launch_simulation(x, v, m, 1.0, integ, -1.0, tf, method=method, eps=1e-2, tolerance=1e-9)
+        xo, vo, so = O.rk_embedded(x, v, m, 1.0, integ, 1e-9, tf, eps=1e-2, method=method)
+        assert r[4] == so
+        assert np.array_equal(r[1], xo) and np.array_equal(r[2], vo)
