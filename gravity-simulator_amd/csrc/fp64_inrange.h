@@ -76,18 +76,91 @@ __device__ __forceinline__ double over_r3_any(double G, double r2)
 // z / b for a constant b > 1 with y = RN(1 / b), correctly rounded with one
 // multiply and two FMAs instead of a full division (Markstein's theorem: with
 // q = RN(z y) within an ulp of z / b, the remainder r = z - b q is exact and
-// RN(q + r y) = RN(z / b)).  Quotients near the subnormal range, where the
-// remainder can be inexact, take the division itself, and so do infinities
-// and NaN.
+// RN(q + r y) = RN(z / b)); div_const_ready(z) must hold, which excludes
+// quotients near the subnormal range, where the remainder can be inexact,
+// infinities and NaN.
 __device__ __forceinline__ double div_const(double z, double b, double y)
 {
-    const double az = fabs(z);
-    if (!(az >= 0x1p-900 && az < 0x1p1000)) return z / b;
     const double q = z * y;
     const double r = __builtin_fma(-q, b, z);
     return __builtin_fma(r, y, q);
 }
 
-#define GS_DIVC(z, b) ::gs::div_const((z), (b), 1.0 / (b))
+__device__ __forceinline__ bool div_const_ready(double z)
+{
+    const double az = fabs(z);
+    return az >= 0x1p-900 && az < 0x1p1000;
+}
+
+// any z
+#define GS_DIVC(z, b) \
+    (::gs::div_const_ready(z) ? ::gs::div_const((z), (b), 1.0 / (b)) : (z) / (b))
+
+// Zero or in [2^-400, 2^300): differences of two such values are zero or at
+// least 2^-453.
+__device__ __forceinline__ bool coordinate_in_range(double a)
+{
+    const unsigned u = static_cast<unsigned>(__double_as_longlong(a) >> 32) & 0x7fffffffu;
+    return a == 0.0 || u - ((1023u - 400u) << 20) < (700u << 20);
+}
+
+// q[u][d] = fl(fl(gm[u] t[u][d]) / fl(fl(fl(r r) r) + eps3)), r = fl(sqrt(
+// t[u].t[u])) summed left to right: one square root and three divisions by
+// the same value, whose reciprocal is formed once (v_rcp_f64 and two Newton
+// steps) and corrected per quotient by its exact remainder; K of them step by
+// step, so that their chains overlap.  `fast` promises t[u][d] zero or in
+// [2^-453, 2^301), gm[u] in [2^-300, 2^300) and 0 <= eps3 < 2^300; |t|^2 is
+// checked here.  Zero numerators keep their sign (the corrections would turn
+// -0 into +0).
+template <int K>
+__device__ __forceinline__ void pull3(const double (&t)[K][3], const double (&gm)[K], double eps3,
+                                      bool fast, double (&q)[K][3])
+{
+#define GS_EACH _Pragma("unroll") for (int u = 0; u < K; u++)
+    double r2[K];
+    GS_EACH
+    {
+        r2[u] = t[u][0] * t[u][0] + t[u][1] * t[u][1] + t[u][2] * t[u][2];
+        const unsigned hi = static_cast<unsigned>(__double_as_longlong(r2[u]) >> 32);
+        fast = fast && hi - ((1023u - 100u) << 20) < (200u << 20);
+    }
+    if (__all(fast)) {
+        double h[K], s[K], e[K], c[K], y[K];
+        GS_EACH y[u] = __builtin_amdgcn_rsq(r2[u]);
+        GS_EACH h[u] = 0.5 * y[u];
+        GS_EACH s[u] = r2[u] * y[u];
+        GS_EACH e[u] = __builtin_fma(-h[u], s[u], 0.5);
+        GS_EACH h[u] = __builtin_fma(h[u], e[u], h[u]);
+        GS_EACH s[u] = __builtin_fma(s[u], e[u], s[u]);
+        GS_EACH e[u] = __builtin_fma(-s[u], s[u], r2[u]);
+        GS_EACH s[u] = __builtin_fma(e[u], h[u], s[u]);
+        GS_EACH e[u] = __builtin_fma(-s[u], s[u], r2[u]);
+        GS_EACH s[u] = __builtin_fma(e[u], h[u], s[u]);
+        GS_EACH c[u] = (s[u] * s[u] * s[u]) + eps3;
+        GS_EACH y[u] = __builtin_amdgcn_rcp(c[u]);
+        GS_EACH e[u] = __builtin_fma(-c[u], y[u], 1.0);
+        GS_EACH y[u] = __builtin_fma(e[u], y[u], y[u]);
+        GS_EACH e[u] = __builtin_fma(-c[u], y[u], 1.0);
+        GS_EACH y[u] = __builtin_fma(e[u], y[u], y[u]);
+        GS_EACH
+        {
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const double a = gm[u] * t[u][d];
+                const double q0 = a * y[u];
+                q[u][d] = __builtin_copysign(__builtin_fma(__builtin_fma(-c[u], q0, a), y[u], q0), a);
+            }
+        }
+    } else {
+        GS_EACH
+        {
+            const double n = __builtin_sqrt(r2[u]);
+            const double c = (n * n * n) + eps3;
+#pragma unroll
+            for (int d = 0; d < 3; d++) q[u][d] = gm[u] * t[u][d] / c;
+        }
+    }
+#undef GS_EACH
+}
 
 }  // namespace gs

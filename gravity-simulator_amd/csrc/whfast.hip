@@ -59,10 +59,28 @@ __device__ __forceinline__ double norm3(double a, double b, double c)
     return __builtin_sqrt(a * a + b * b + c * c);
 }
 
-// (the Stumpff series' constant divisors)
-#define DIVC(z, b) GS_DIVC(z, b)
+// The Stumpff series (src/integrator_whfast.c:774-815), the reference's
+// nested form, innermost factor first; div(z, b) = z / b for the series'
+// constant divisors.
+template <class Div>
+__device__ __forceinline__ void stumpff_series(double z, Div div, double &t2, double &t3)
+{
+    t3 = 1.0 - div(z, 210.0);
+    t3 = 1.0 - div(z, 156.0) * t3;
+    t3 = 1.0 - div(z, 110.0) * t3;
+    t3 = 1.0 - div(z, 72.0) * t3;
+    t3 = 1.0 - div(z, 42.0) * t3;
+    t3 = 1.0 - div(z, 20.0) * t3;
+    t3 = div(t3, 6.0);
+    t2 = 1.0 - div(z, 182.0);
+    t2 = 1.0 - div(z, 132.0) * t2;
+    t2 = 1.0 - div(z, 90.0) * t2;
+    t2 = 1.0 - div(z, 56.0) * t2;
+    t2 = 1.0 - div(z, 30.0) * t2;
+    t2 = 1.0 - div(z, 12.0) * t2;
+    t2 = t2 / 2.0;
+}
 
-// src/integrator_whfast.c:774-815
 __device__ void stumpff(double z, double &c0, double &c1, double &c2, double &c3)
 {
     int k = 0;
@@ -70,21 +88,13 @@ __device__ void stumpff(double z, double &c0, double &c1, double &c2, double &c3
         z /= 4.0;
         k++;
     }
-    // the reference's nested series, innermost factor first
-    double t3 = 1.0 - DIVC(z, 210.0);
-    t3 = 1.0 - DIVC(z, 156.0) * t3;
-    t3 = 1.0 - DIVC(z, 110.0) * t3;
-    t3 = 1.0 - DIVC(z, 72.0) * t3;
-    t3 = 1.0 - DIVC(z, 42.0) * t3;
-    t3 = 1.0 - DIVC(z, 20.0) * t3;
-    t3 = DIVC(t3, 6.0);
-    double t2 = 1.0 - DIVC(z, 182.0);
-    t2 = 1.0 - DIVC(z, 132.0) * t2;
-    t2 = 1.0 - DIVC(z, 90.0) * t2;
-    t2 = 1.0 - DIVC(z, 56.0) * t2;
-    t2 = 1.0 - DIVC(z, 30.0) * t2;
-    t2 = 1.0 - DIVC(z, 12.0) * t2;
-    t2 = t2 / 2.0;
+    double t2, t3;
+    // (|z| <= 0.1 here and the series' factors lie in [0.9, 1.1]: one check of
+    // the wavefront's z covers all thirteen divisions)
+    if (__all(fabs(z) >= 0x1p-900))
+        stumpff_series(z, [](double a, double b) { return div_const(a, b, 1.0 / b); }, t2, t3);
+    else
+        stumpff_series(z, [](double a, double b) { return a / b; }, t2, t3);
     double t1 = 1.0 - z * t3;
     double t0 = 1.0 - z * t2;
     while (k > 0) {
@@ -192,6 +202,7 @@ struct WfShared {
     int nm;
     int n;
     int any_remove;
+    int kick_slow;  // a massive particle's position or mass outside the range pull3 takes
     int bad;  // bit d: some jq component d is not finite
     int primary;
 };
@@ -476,13 +487,13 @@ __device__ __forceinline__ double run_quotient(const WfShared &S, const WfScratc
 
 // Jacobi -> Cartesian for the whole workgroup, first half.  The recurrence
 // above only needs jq at the massive particles: inside a run of massless
-// particles (finite jq, c != 0) the quotient is c / eta and c becomes
+// particles (finite jq, c not -0) the quotient is c / eta and c becomes
 // eta (c / eta), which reaches a fixed point within a few particles.  Lane d
 // therefore walks the massive particles and the head of each run (at most
 // J2C_K quotients per run) and stores the quotients, with the coordinate of
 // particle 0; then q = jq + quotient for every other particle, in parallel
 // (j2c_fill, or fused into the kick).  Components with bit d of `bad` set (a
-// non-finite jq), or whose walk meets c == 0 or no fixed point within J2C_K,
+// non-finite jq), or whose walk meets c == -0 or no fixed point within J2C_K,
 // are marked in X.j.fallback for the serial recurrence; both give the same
 // bits.  Called by all threads.
 __device__ void j2c_quotients(int n, const double *jq, const WfShared &S, WfScratch &X, int bad)
@@ -506,11 +517,14 @@ __device__ void j2c_quotients(int n, const double *jq, const WfShared &S, WfScra
             const int hi = (g + 1 < nm ? S.mlist[g + 1] : n) - 1;
             int k = 0;
             for (int i = hi; i > lo; i--) {
-                if (k == J2C_K || c == 0.0) {
+                if (k == J2C_K || (c == 0.0 && __builtin_signbit(c))) {
                     fail = true;
                     break;
                 }
-                // (c - 0 * jq) / eta with jq finite and c != 0 is c / eta
+                // (c - 0 * jq) / eta with jq finite is c / eta unless c is -0
+                // (c = +0, a centre of mass exactly at the origin, stays +0:
+                // taking it for the serial recurrence cost such a system 0.48
+                // ms a step instead of 0.07)
                 const double cn = c / eta[i];
                 X.j.exp[g][k][d] = cn;
                 k++;
@@ -597,60 +611,64 @@ __device__ void c2j_component(int n, int d, const double *q, double *jq, const d
 // every particle in the massive list).
 // xi, x0: Cartesian positions of particle i and of particle 0; jxi: its
 // Jacobi position; ginside: for a massless particle, the number of massive
-// particles inside it.
+// particles inside it; fast: the massive particles' positions and G m lie in
+// the range pull3 takes.
 __device__ __forceinline__ void accel_kick_v(const WfShared &S, int i, bool massive, int p,
                                              const double *xi, const double *x0,
                                              const double *jxi, int ginside, double m0, double G,
-                                             double eps3, double *jv, double dt,
+                                             double eps3, double *jv, double dt, bool fast,
                                              double *jv_sync = nullptr)
 {
+    for (int d = 0; d < 3; d++)
+        fast = fast && coordinate_in_range(xi[d]) && coordinate_in_range(jxi[d]);
     double a[3];
-    const double tv0 = xi[0] - x0[0], tv1 = xi[1] - x0[1], tv2 = xi[2] - x0[2];
-    const double c0 = cube_plus(tv0, tv1, tv2, eps3);
-    const double cj = cube_plus(jxi[0], jxi[1], jxi[2], eps3);
     const double ei = S.key[i], ei1 = S.key[i - 1];
-    const double tv[3] = {tv0, tv1, tv2};
-    if (massive) {
-        for (int d = 0; d < 3; d++) a[d] = G * m0 * ei / ei1 * (jxi[d] / cj - tv[d] / c0);
-    } else {
-        for (int d = 0; d < 3; d++) a[d] = G * m0 * (jxi[d] / cj - tv[d] / c0);
+    {
+        const double t[2][3] = {{xi[0] - x0[0], xi[1] - x0[1], xi[2] - x0[2]},
+                                {jxi[0], jxi[1], jxi[2]}};
+        const double one[2] = {1.0, 1.0};
+        double f[2][3];
+        pull3<2>(t, one, eps3, fast, f);
+        if (massive) {
+            for (int d = 0; d < 3; d++) a[d] = G * m0 * ei / ei1 * (f[1][d] - f[0][d]);
+        } else {
+            for (int d = 0; d < 3; d++) a[d] = G * m0 * (f[1][d] - f[0][d]);
+        }
     }
     const int nm = S.nm;
-    double aux0 = 0.0, aux1 = 0.0, aux2 = 0.0;
-    // interior massive particles (ordinal 1.., position < i)
-    for (int q = 1; q < nm; q++) {
-        const int j = S.mlist[q];
-        if (massive ? q >= p : j >= i) break;
-        const double t0 = xi[0] - S.mx[q][0], t1 = xi[1] - S.mx[q][1], t2 = xi[2] - S.mx[q][2];
-        const double cc = cube_plus(t0, t1, t2, eps3);
-        aux0 += G * S.mm[q] * t0 / cc;
-        aux1 += G * S.mm[q] * t1 / cc;
-        aux2 += G * S.mm[q] * t2 / cc;
+    // massive particles inside i (ordinal 1.., position < i) and outside it,
+    // each sum in ordinal order; the pulls of the inner ones are the outer
+    // form's with every sign changed, which is exact
+    double in[3] = {0.0, 0.0, 0.0}, out[3] = {0.0, 0.0, 0.0};
+    constexpr int K = 2;
+    for (int q0 = 1; q0 < nm; q0 += K) {
+        double t[K][3], gm[K], f[K][3];
+#pragma unroll
+        for (int u = 0; u < K; u++) {
+            const int q = q0 + u < nm ? q0 + u : q0;
+            // (a massive particle's pull on itself is formed at a unit offset and not added)
+            const bool self = massive && q == p;
+            gm[u] = G * S.mm[q];
+            for (int d = 0; d < 3; d++) t[u][d] = self ? 1.0 : S.mx[q][d] - xi[d];
+        }
+        pull3<K>(t, gm, eps3, fast, f);
+#pragma unroll
+        for (int u = 0; u < K; u++) {
+            const int q = q0 + u;
+            if (q >= nm || (massive && q == p)) continue;
+            const bool inside = massive ? q < p : S.mlist[q] < i;
+            for (int d = 0; d < 3; d++) {
+                if (inside) in[d] -= f[u][d];
+                else out[d] += f[u][d];
+            }
+        }
     }
-    if (massive) {
-        a[0] -= aux0 * ei / ei1;
-        a[1] -= aux1 * ei / ei1;
-        a[2] -= aux2 * ei / ei1;
-    } else {
-        a[0] -= aux0;
-        a[1] -= aux1;
-        a[2] -= aux2;
+    for (int d = 0; d < 3; d++) {
+        if (massive) a[d] -= in[d] * ei / ei1;
+        else a[d] -= in[d];
+        a[d] += out[d];
     }
-    aux0 = aux1 = aux2 = 0.0;
-    // exterior massive particles
-    for (int q = 1; q < nm; q++) {
-        const int j = S.mlist[q];
-        if (massive ? q <= p : j <= i) continue;
-        const double t0 = S.mx[q][0] - xi[0], t1 = S.mx[q][1] - xi[1], t2 = S.mx[q][2] - xi[2];
-        const double cc = cube_plus(t0, t1, t2, eps3);
-        aux0 += G * S.mm[q] * t0 / cc;
-        aux1 += G * S.mm[q] * t1 / cc;
-        aux2 += G * S.mm[q] * t2 / cc;
-    }
-    a[0] += aux0;
-    a[1] += aux1;
-    a[2] += aux2;
-    aux0 = aux1 = aux2 = 0.0;
+    double aux0, aux1, aux2;
     // pairs straddling i: interior j (ordinal from 0), exterior k; the sum
     // depends only on where i sits among the massive particles
     if (massive) {
@@ -686,7 +704,7 @@ __device__ void accel_kick(const WfShared &S, int i, bool massive, int p, const 
     int g = 0;  // massive particles inside i
     if (!massive)
         while (g < S.nm && S.mlist[g] < i) g++;
-    accel_kick_v(S, i, massive, p, &x[3 * i], x, &jx[3 * i], g, m[0], G, eps3, jv, dt, jv_sync);
+    accel_kick_v(S, i, massive, p, &x[3 * i], x, &jx[3 * i], g, m[0], G, eps3, jv, dt, false, jv_sync);
 }
 
 __device__ void load_massive_positions(WfShared &S, const double *x)
@@ -802,15 +820,19 @@ __device__ void kick_from_quotients(WfShared &S, const WfScratch &X, int n, doub
             const double v = q == 0 ? X.j.q0[d] : X.j.mjq[q][d] + X.j.mq[q][d];
             S.mx[q][d] = v;
             if (write_x) x[3 * j + d] = v;
+            if (!coordinate_in_range(v)) S.kick_slow = 1;
         }
+        const double gm = G * S.mm[q];
+        if (!(gm >= 0x1p-300 && gm < 0x1p300 && eps3 >= 0.0 && eps3 < 0x1p300)) S.kick_slow = 1;
     }
     __syncthreads();
+    const bool fast = S.kick_slow == 0;
     straddle_sums(S, G, eps3);
     const double m0 = S.mm[0];
     for (int p = 1 + static_cast<int>(threadIdx.x); p < nm; p += WF_BLOCK) {
         const int i = S.mlist[p];
         accel_kick_v(S, i, true, p, S.mx[p], S.mx[0], &jx[3 * i], 0, m0, G, eps3, jv, dt,
-                     jv_sync);
+                     fast, jv_sync);
     }
     if (method == 2) {
         MassiveCursor mc;
@@ -827,7 +849,7 @@ __device__ void kick_from_quotients(WfShared &S, const WfScratch &X, int n, doub
                 x[3 * i + 2] = xi[2];
             }
             accel_kick_v(S, i, false, -1, xi, S.mx[0], jxi, g + 1, m0, G, eps3, jv, dt,
-                         jv_sync);
+                         fast, jv_sync);
         }
     }
     __syncthreads();
@@ -894,7 +916,12 @@ __global__ __launch_bounds__(WF_BLOCK) void k_whfast_init(WfArgs A)
 }
 
 // `nsteps` steps of the main loop (src/integrator_whfast.c:290-378).
-__global__ __launch_bounds__(WF_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_whfast_steps(WfArgs A)
+// Bound by the latency of each particle's FP64 chains.  210 VGPRs, two
+// wavefronts per SIMD, and two pulls at a time in the kick: held to 128
+// registers for four wavefronts, with one pull at a time through the
+// compiler's square root and divisions, 4096 systems took 125 ms per 200
+// steps and 512 systems 16.7; now 76 and 13.5 (one pull at a time: 77, 14.1).
+__global__ __launch_bounds__(WF_BLOCK) void k_whfast_steps(WfArgs A)
 {
     __shared__ WfShared S;
     __shared__ WfScratch X;
@@ -929,6 +956,7 @@ __global__ __launch_bounds__(WF_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) v
         if (threadIdx.x == 0) {
             S.any_remove = 0;
             S.bad = 0;
+            S.kick_slow = 0;
         }
         for (int i = threadIdx.x; i < n; i += WF_BLOCK) flags[i] = 0;
         __syncthreads();

@@ -109,3 +109,22 @@ def test_whfast_via_launch_simulation_two_body():
     io, xo, vo, mo = O.whfast(x, v, m, 1.0, 0.01, 3.0, method=2)
     assert steps == 300
     assert np.array_equal(xg, xo) and np.array_equal(vg, vo)
+
+
+@pytest.mark.parametrize("flip", [1.0, -1.0])
+def test_centre_of_mass_coordinate_exactly_zero(flip):
+    """A planar system (every z and vz zero, of either sign) and one whose centre of mass is exactly at the origin: the
+    Jacobi coordinate of the centre of mass is an exact zero, as are the pulls' z components."""
+    off, X, V, M = ic.ensemble(1, 21, max_test=300)
+    x, v, m = X.copy(), V.copy(), M.copy()
+    x[:, 2] = 0.0 * flip
+    v[:, 2] = 0.0 * flip
+    m[:9] = 2.0 ** -20
+    m[0] = 1.0
+    x[0, 0] = -(m[1:9] * x[1:9, 0]).sum()
+    for method in (1, 2):
+        k = 9 if method == 1 else len(m)
+        ((ids, xg, vg, mg),) = L.whfast_ensemble(np.array([0, k]), x[:k], v[:k], m[:k], 1.0, 0.01, 0.4, method=method)
+        io, xo, vo, mo = O.whfast(x[:k], v[:k], m[:k], 1.0, 0.01, 0.4, method=method)
+        assert np.array_equal(ids, io) and np.array_equal(mg, mo)
+        assert np.array_equal(xg, xo) and np.array_equal(vg, vo)
