@@ -404,20 +404,19 @@ double compute_energy(const System *system)
     std::lock_guard<std::recursive_mutex> lk(c->mu);
     const int n = system->num_particles;
     void *dx, *dv, *dm, *dp;
-    const int nparts = (n + 255) / 256;
+    const int nparts = energy_partials(c, n);
     if (slot(c, SLOT_X, sizeof(double) * 3 * n, &dx).return_code ||
         slot(c, SLOT_V, sizeof(double) * 3 * n, &dv).return_code ||
         slot(c, SLOT_M, sizeof(double) * n, &dm).return_code ||
         slot(c, SLOT_PARTIAL, sizeof(double) * nparts, &dp).return_code)
         return NAN;
     std::vector<double> part(nparts);
-    int np = 0;
     if (hipMemcpyAsync(dx, system->x, sizeof(double) * 3 * n, hipMemcpyHostToDevice, c->stream) ||
         hipMemcpyAsync(dv, system->v, sizeof(double) * 3 * n, hipMemcpyHostToDevice, c->stream) ||
         hipMemcpyAsync(dm, system->m, sizeof(double) * n, hipMemcpyHostToDevice, c->stream) ||
         launch_energy(c, static_cast<double *>(dx), static_cast<double *>(dv),
-                      static_cast<double *>(dm), n, system->G, static_cast<double *>(dp), &np) ||
-        hipMemcpyAsync(part.data(), dp, sizeof(double) * np, hipMemcpyDeviceToHost, c->stream) ||
+                      static_cast<double *>(dm), n, system->G, static_cast<double *>(dp)) ||
+        hipMemcpyAsync(part.data(), dp, sizeof(double) * nparts, hipMemcpyDeviceToHost, c->stream) ||
         hipStreamSynchronize(c->stream) != hipSuccess)
         return NAN;
     double e = 0.0;
@@ -630,13 +629,12 @@ ErrorStatus gs_sim_energy(GsSim *s, double *energy)
     Context *c;
     GS_TRY(context(&c));
     std::lock_guard<std::recursive_mutex> lk(c->mu);
-    const int nparts = (s->n + 255) / 256;
+    const int nparts = energy_partials(c, s->n);
     void *dp;
     GS_TRY(slot(c, SLOT_PARTIAL, sizeof(double) * nparts, &dp));
-    int np = 0;
-    GS_HIP(launch_energy(c, s->x, s->v, s->m, s->n, s->G, static_cast<double *>(dp), &np));
-    std::vector<double> part(np);
-    GS_HIP(hipMemcpyAsync(part.data(), dp, sizeof(double) * np, hipMemcpyDeviceToHost, c->stream));
+    GS_HIP(launch_energy(c, s->x, s->v, s->m, s->n, s->G, static_cast<double *>(dp)));
+    std::vector<double> part(nparts);
+    GS_HIP(hipMemcpyAsync(part.data(), dp, sizeof(double) * nparts, hipMemcpyDeviceToHost, c->stream));
     GS_HIP(hipStreamSynchronize(c->stream));
     double e = 0.0;
     for (double v : part) e += v;

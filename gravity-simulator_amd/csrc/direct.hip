@@ -16,6 +16,8 @@
 //  k_energy        FP64 kinetic + pair potential energy (src/utils.c:27-59).
 //  k_lf_*          Leapfrog updates with the reference's compensated
 //                  summation (src/integrator.c:973-1094).
+#include <algorithm>
+
 #include "fp64_inrange.h"
 #include "gs_internal.h"
 
@@ -704,16 +706,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(IPT <= 2 ? 
 
 // The scalar-source kernel with a shared target group and a software-
 // pipelined source stream.  The W wavefronts of a workgroup hold the same 64
-// targets and split the chunk's source tiles into W contiguous runs; at the
+// targets and split the chunk's source units into W contiguous runs; at the
 // end wavefronts 1..W-1 leave their compensated sums in LDS and wavefront 0
 // adds the W sums in wavefront order (FP64, a fixed order), so the FP64
 // partial sums written per chunk are 1/W of k_direct_f32s's at the same
-// number of wavefronts.  Each wavefront reads its run of float4
+// number of wavefronts.  A unit is a tile or, for few targets, a 2^-sh part
+// of one (in the tile's frame), each with its own FP32 partial sum and Kahan
+// fold.  Each wavefront reads its run of float4
 // sources in batches of PF_BATCH through wave-uniform loads and issues the
 // loads of batch b + 1 before the arithmetic of batch b; the last batch
 // re-reads its own sources instead of reading past the run.  Arithmetic, tile
 // frames and Kahan folds are k_direct_f32s's.
 constexpr int PF_BATCH = 4;
+constexpr int F32P_MAX_SH = 4;
 
 template <bool SOFT>
 __device__ __forceinline__ void f32_batch(const float4 (&s)[PF_BATCH], float xi, float yi, float zi,
@@ -740,10 +745,10 @@ __device__ __forceinline__ void f32_batch(const float4 (&s)[PF_BATCH], float xi,
 template <int W, bool SOFT>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(8))) void k_direct_f32p(
     const double *__restrict__ x, int n, const float4 *__restrict__ S,
-    const double4 *__restrict__ C, float eps2, int tiles_per_chunk, int ntiles,
+    const double4 *__restrict__ C, float eps2, int units_per_chunk, int units, int sh, double scale,
     double *__restrict__ partial)
 {
-    static_assert(ST_TILE % (2 * PF_BATCH) == 0, "a tile must hold whole batch pairs");
+    static_assert((ST_TILE >> F32P_MAX_SH) % (2 * PF_BATCH) == 0, "a unit must hold whole batch pairs");
     __shared__ double other[W - 1][3][64];
     const int lane = threadIdx.x & 63;
     // wave-uniform by construction; readfirstlane lets the compiler see it,
@@ -755,25 +760,26 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(8))) voi
     const int ii = i < n ? i : i0;
     const double xd = x[3 * ii + 0], yd = x[3 * ii + 1], zd = x[3 * ii + 2];
     float sx = 0.0f, sy = 0.0f, sz = 0.0f, cx = 0.0f, cy = 0.0f, cz = 0.0f;
-    const int J0 = blockIdx.y * tiles_per_chunk;
-    const int Jc = min(ntiles, J0 + tiles_per_chunk);
-    const int tpw = (Jc - J0 + W - 1) / W;
-    const int Ja = min(Jc, J0 + wv * tpw);
-    const int Jb = min(Jc, Ja + tpw);
+    const int unit = ST_TILE >> sh;  // sources per unit
+    const int J0 = blockIdx.y * units_per_chunk;
+    const int Jc = min(units, J0 + units_per_chunk);
+    const int upw = (Jc - J0 + W - 1) / W;
+    const int Ja = min(Jc, J0 + wv * upw);
+    const int Jb = min(Jc, Ja + upw);
     if (Ja < Jb) {
-        const float4 *__restrict__ base = S + static_cast<size_t>(Ja) * ST_TILE;
-        const int last = (Jb - Ja) * ST_TILE - PF_BATCH;  // start of the run's last batch
+        const float4 *__restrict__ base = S + static_cast<size_t>(Ja) * unit;
+        const int last = (Jb - Ja) * unit - PF_BATCH;  // start of the run's last batch
         float4 a[PF_BATCH], b[PF_BATCH];
 #pragma unroll
         for (int q = 0; q < PF_BATCH; q++) a[q] = base[q];
         int pos = 0;
         for (int J = Ja; J < Jb; J++) {
-            const double4 c = C[J];
+            const double4 c = C[J >> sh];
             const float xi = static_cast<float>(xd - c.x);
             const float yi = static_cast<float>(yd - c.y);
             const float zi = static_cast<float>(zd - c.z);
             float px = 0.0f, py = 0.0f, pz = 0.0f;
-            for (int jj = 0; jj < ST_TILE; jj += 2 * PF_BATCH, pos += 2 * PF_BATCH) {
+            for (int jj = 0; jj < unit; jj += 2 * PF_BATCH, pos += 2 * PF_BATCH) {
                 const float4 *nb = base + min(pos + PF_BATCH, last);
 #pragma unroll
                 for (int q = 0; q < PF_BATCH; q++) b[q] = nb[q];
@@ -804,10 +810,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(8))) voi
             ry += other[w][1][lane];
             rz += other[w][2][lane];
         }
+        // (scale: 1 for partial sums, G where one chunk is the whole sum)
         double *out = partial + static_cast<size_t>(blockIdx.y) * 3 * n;
-        out[3 * i + 0] = rx;
-        out[3 * i + 1] = ry;
-        out[3 * i + 2] = rz;
+        out[3 * i + 0] = scale * rx;
+        out[3 * i + 1] = scale * ry;
+        out[3 * i + 2] = scale * rz;
     }
 }
 
@@ -827,25 +834,57 @@ Fp32Config &fp32_config()
     return cfg;
 }
 
-// Source chunks per evaluation when the configuration leaves it to us:
+static int f32s_tiles(int n) { return (n + ST_TILE - 1) / ST_TILE; }
+
+// How the shared-target kernel (W wavefronts per 64 targets) divides the
+// sources: units of ST_TILE >> sh, units_per_chunk of them per workgroup.
+struct F32pPlan {
+    int sh, units, units_per_chunk, chunks;
+};
+
+// With a given split, tiles in that many chunks.  Otherwise a wavefront takes
+// 4 tiles (1024 sources; more only where 64-target groups alone give over
+// 2^14 workgroups), fewer while that leaves under 8 wavefronts per SIMD, then
+// parts of a tile down to 16 sources: a wavefront waits for its scalar loads
+// about 6 times as long as it computes on them, so the chip needs all its
+// wavefronts, and the sums' folds cost little next to that (n = 6007, kernel:
+// 46 us with whole tiles in one chunk, 14 us here; n = 131072 4.33 ms either way).
+static F32pPlan f32p_plan(int n, int targets, int W, int split, int cu_count)
+{
+    F32pPlan p;
+    const int ntiles = f32s_tiles(n);
+    p.sh = 0;
+    p.units = ntiles;
+    if (split > 0) {
+        p.units_per_chunk = (ntiles + split - 1) / split;
+    } else {
+        const long long groups = (targets + 63) / 64, full = 32ll * cu_count;
+        const long long total = groups * ntiles;  // wavefronts at one tile each
+        long long upw = 1;
+        if (total >= 4 * full) upw = std::max(4ll, (total + 32 * full - 1) / (32 * full));
+        else if (total >= full) upw = total / full;
+        else
+            while (p.sh < F32P_MAX_SH && (total << p.sh) < full) p.sh++;
+        const int unit = ST_TILE >> p.sh;
+        p.units = (n + unit - 1) / unit;
+        p.units_per_chunk = static_cast<int>(std::min<long long>(upw * W, p.units));
+    }
+    p.chunks = (p.units + p.units_per_chunk - 1) / p.units_per_chunk;
+    return p;
+}
+
+// Source chunks of the other kernels when the configuration leaves it to us:
 // about 1024 sources per chunk (128 chunks at N = 2^17).  Measured on
 // MI355X at N = 2^17 with 256-source tiles (kernel only): 2048 per chunk
 // 4.36 ms, 1024 4.35 ms, 512 4.34 ms; each halving doubles the FP64 partial
 // sums (402 MB at 1024) that the reduction reads back (~0.09 ms).
-//
-// The shared-target kernel (kind 2) spreads a chunk over its W wavefronts:
-// 1024 W sources per chunk keep 1024 sources per wavefront (W = 8: 16 chunks
-// at N = 2^17, 50 MB of partial sums).
 static int resolve_split(int n, const Fp32Config &cfg, int cu_count)
 {
-    (void)cu_count;
+    if (cfg.kind == 2) return f32p_plan(n, n, cfg.block, cfg.jsplit, cu_count).chunks;
     if (cfg.jsplit > 0) return cfg.jsplit;
-    const int per_chunk = cfg.kind == 2 ? 1024 * cfg.block : 1024;
-    const int split = (n + per_chunk - 1) / per_chunk;
+    const int split = (n + 1023) / 1024;
     return split < 1 ? 1 : split;
 }
-
-static int f32s_tiles(int n) { return (n + ST_TILE - 1) / ST_TILE; }
 
 size_t direct_f32_partial_bytes(int n, const Fp32Config &cfg, int cu_count)
 {
@@ -883,16 +922,16 @@ static void launch_f32s_shape(Context *c, dim3 grid, const double *x, int n, con
 }
 
 template <int W>
-static void launch_f32p_shape(Context *c, dim3 grid, const double *x, int n, const float4 *S,
-                              const double4 *C, float eps2, bool soft, int tpc, int ntiles,
+static void launch_f32p_shape(Context *c, const F32pPlan &p, const double *x, int targets,
+                              const float4 *S, const double4 *C, float eps2, double scale,
                               double *partial)
 {
-    if (soft)
-        hipLaunchKernelGGL((k_direct_f32p<W, true>), grid, dim3(64 * W), 0, c->stream, x, n, S, C,
-                           eps2, tpc, ntiles, partial);
-    else
-        hipLaunchKernelGGL((k_direct_f32p<W, false>), grid, dim3(64 * W), 0, c->stream, x, n, S,
-                           C, eps2, tpc, ntiles, partial);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((targets + 63) / 64, p.chunks), dim3(64 * W), 0, c->stream, x,
+                           targets, S, C, eps2, p.units_per_chunk, p.units, p.sh, scale, partial);
+    };
+    if (eps2 > 0.0f) launch(k_direct_f32p<W, true>);
+    else launch(k_direct_f32p<W, false>);
 }
 
 hipError_t launch_direct_f32(Context *c, const double *x, const double *m, int n, double G,
@@ -919,12 +958,20 @@ hipError_t launch_direct_f32(Context *c, const double *x, const double *m, int n
         nsplit = (ntiles + tpc - 1) / tpc;
         const int rec = timing_begin(c, "direct_f32");
         if (cfg.kind == 2) {
-            dim3 grid((n + 63) / 64, nsplit);
+            const F32pPlan p = f32p_plan(n, n, cfg.block, cfg.jsplit, c->cu_count);
+            nsplit = p.chunks;
+            // one chunk is the whole sum: no partial sums to add
+            double *out = p.chunks == 1 ? a : partial;
+            const double scale = p.chunks == 1 ? G : 1.0;
             switch (cfg.block) {
-                case 4: launch_f32p_shape<4>(c, grid, x, n, S, C, eps2, soft, tpc, ntiles, partial); break;
-                case 8: launch_f32p_shape<8>(c, grid, x, n, S, C, eps2, soft, tpc, ntiles, partial); break;
-                case 16: launch_f32p_shape<16>(c, grid, x, n, S, C, eps2, soft, tpc, ntiles, partial); break;
+                case 4: launch_f32p_shape<4>(c, p, x, n, S, C, eps2, scale, out); break;
+                case 8: launch_f32p_shape<8>(c, p, x, n, S, C, eps2, scale, out); break;
+                case 16: launch_f32p_shape<16>(c, p, x, n, S, C, eps2, scale, out); break;
                 default: timing_end(c, rec); return hipErrorInvalidValue;
+            }
+            if (p.chunks == 1) {
+                timing_end(c, rec);
+                return hipGetLastError();
             }
         } else {
             const int waves = (n + 64 * cfg.ipt - 1) / (64 * cfg.ipt);
@@ -968,8 +1015,8 @@ hipError_t launch_direct_f32(Context *c, const double *x, const double *m, int n
 // FP32 direct sum for a list of targets against all n sources (the learned
 // correction's labels and spot check).  The shared-target kernel of
 // launch_direct_f32 (kind 2, 16 wavefronts per 64 targets): the targets'
-// positions are gathered into a compact array and the source range is split
-// so that even a few hundred targets fill the chip.
+// positions are gathered into a compact array and the sources divided by the
+// same rule, so that even a few hundred targets fill the chip.
 __global__ void k_gather_targets(const double *__restrict__ x, const int *__restrict__ idx,
                                  int nt, double *__restrict__ xt)
 {
@@ -988,22 +1035,12 @@ hipError_t launch_gather_rows3(Context *c, const double *src, const int *idx, in
 
 constexpr int TARGET_WAVES = 16;  // wavefronts per 64 targets in launch_direct_f32_targets
 
-// Source chunks: about 1024 workgroups in all, each wavefront of a chunk's
-// workgroup with at least one tile.
-static int targets_split(int n, int nt)
-{
-    const int ntiles = f32s_tiles(n);
-    const int wgs = (nt + 63) / 64;
-    int split = (1024 + wgs - 1) / wgs;
-    if (split > ntiles / TARGET_WAVES) split = ntiles / TARGET_WAVES;
-    return split < 1 ? 1 : split;
-}
-
-size_t direct_f32_targets_bytes(int n, int nt)
+size_t direct_f32_targets_bytes(Context *c, int n, int nt)
 {
     const size_t nt3 = 3 * static_cast<size_t>(nt);
     const size_t nt_tiles = f32s_tiles(n);
-    return 512 + nt3 * sizeof(double) * (1 + targets_split(n, nt)) + nt_tiles * ST_TILE * sizeof(float4) +
+    const F32pPlan p = f32p_plan(n, nt, TARGET_WAVES, 0, c->cu_count);
+    return 512 + nt3 * sizeof(double) * (1 + p.chunks) + nt_tiles * ST_TILE * sizeof(float4) +
            nt_tiles * sizeof(double4);
 }
 
@@ -1012,12 +1049,11 @@ hipError_t launch_direct_f32_targets(Context *c, const double *x, const double *
                                      void *buf, size_t bytes)
 {
     if (nt <= 0) return hipSuccess;
-    if (bytes < direct_f32_targets_bytes(n, nt)) return hipErrorInvalidValue;
+    if (bytes < direct_f32_targets_bytes(c, n, nt)) return hipErrorInvalidValue;
     const int ntiles = f32s_tiles(n);
     const int n_pad = ntiles * ST_TILE;
-    const int split = targets_split(n, nt);
-    const int tpc = (ntiles + split - 1) / split;
-    const int nsplit = (ntiles + tpc - 1) / tpc;
+    const F32pPlan plan = f32p_plan(n, nt, TARGET_WAVES, 0, c->cu_count);
+    const int nsplit = plan.chunks;
     const size_t nt3 = 3 * static_cast<size_t>(nt);
     auto align = [](char *p) {
         return reinterpret_cast<char *>((reinterpret_cast<uintptr_t>(p) + 255) & ~uintptr_t(255));
@@ -1033,8 +1069,7 @@ hipError_t launch_direct_f32_targets(Context *c, const double *x, const double *
     hipLaunchKernelGGL(k_f32_sources, dim3((n_pad + 255) / 256), dim3(256), 0, c->stream, x, m, n,
                        n_pad, S, C);
     const float eps2 = static_cast<float>(eps * eps);
-    dim3 grid((nt + 63) / 64, nsplit);
-    launch_f32p_shape<TARGET_WAVES>(c, grid, xt, nt, S, C, eps2, eps2 > 0.0f, tpc, ntiles, partial);
+    launch_f32p_shape<TARGET_WAVES>(c, plan, xt, nt, S, C, eps2, 1.0, partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_reduce_partials, dim3((3 * nt + 255) / 256), dim3(256), 0, c->stream,
@@ -1109,43 +1144,101 @@ hipError_t launch_copy(Context *c, const void *src, void *dst, size_t bytes)
 }
 
 // ------------------------------------------------------------------ energy
-constexpr int EN_BLOCK = 256;
+// One wavefront takes 64 particles, one per lane, and a range of the blocks
+// of 64 that follow it cyclically: block bi meets blocks bi .. bi + nb / 2
+// (mod nb), so every pair of blocks is met once and all wavefronts have the
+// same work (for even nb the last offset belongs to the first half only).
+// The other block's particles come through scalar loads, K at a time.  1 / r
+// from v_rsq_f64 and two Newton steps (within an ulp; the compiler's sqrt and
+// division where r^2 is out of range, coincident particles among them).
+// Bound by FP64 issue.  One MI355X, before (one thread per particle over all
+// later ones) and now: 1024 particles 0.19 ms -> 0.02, 20000 3.2 -> 0.2 ms.
+constexpr int EN_K = 4;
 
-__global__ __launch_bounds__(EN_BLOCK) void k_energy(const double *__restrict__ x,
-                                                     const double *__restrict__ v,
-                                                     const double *__restrict__ m, int n,
-                                                     double G, double *__restrict__ partials)
+__global__ __launch_bounds__(64) void k_energy(const double *__restrict__ x,
+                                               const double *__restrict__ v,
+                                               const double *__restrict__ m, int n, double G,
+                                               int offsets, double *__restrict__ partials)
 {
-    __shared__ double red[EN_BLOCK];
-    const int i = blockIdx.x * EN_BLOCK + threadIdx.x;
+    const int lane = threadIdx.x;
+    const int nb = gridDim.x, bi = blockIdx.x;
+    const int i = bi * 64 + lane;
+    const bool live = i < n;
+    const int ii = live ? i : n - 1;
+    const double x0 = x[3 * ii], x1 = x[3 * ii + 1], x2 = x[3 * ii + 2];
+    const double gm = live ? G * m[ii] : 0.0;
     double e = 0.0;
-    if (i < n) {
+    if (blockIdx.y == 0 && live) {
         const double v0 = v[3 * i], v1 = v[3 * i + 1], v2 = v[3 * i + 2];
         const double vn = __builtin_sqrt(v0 * v0 + v1 * v1 + v2 * v2);
         e = 0.5 * m[i] * vn * vn;
-        const double x0 = x[3 * i], x1 = x[3 * i + 1], x2 = x[3 * i + 2];
-        const double gm = G * m[i];
-        for (int j = i + 1; j < n; j++) {
-            const double r0 = x0 - x[3 * j], r1 = x1 - x[3 * j + 1], r2 = x2 - x[3 * j + 2];
-            e -= gm * m[j] / __builtin_sqrt(r0 * r0 + r1 * r1 + r2 * r2);
+    }
+    const int last = nb / 2;
+    const int d0 = blockIdx.y * offsets, d1 = min(d0 + offsets, last + 1);
+    for (int d = d0; d < d1; d++) {
+        if (d > 0 && 2 * d == nb && bi >= d) break;
+        const int bj = bi + d < nb ? bi + d : bi + d - nb;
+        const int jb = bj * 64, je = min(jb + 64, n);
+        for (int j0 = jb; j0 < je; j0 += EN_K) {
+            double r2[EN_K], w[EN_K], inv[EN_K];
+            bool in = true;
+#pragma unroll
+            for (int u = 0; u < EN_K; u++) {
+                const int j = j0 + u < je ? j0 + u : je - 1;
+                const double r0 = x0 - x[3 * j], r1 = x1 - x[3 * j + 1], rz = x2 - x[3 * j + 2];
+                // pairs not counted here (within a block only j > i): a unit distance, no weight
+                const bool use = live && j0 + u < je && (d > 0 || j > i);
+                r2[u] = use ? r0 * r0 + r1 * r1 + rz * rz : 1.0;
+                w[u] = use ? gm * m[j] : 0.0;
+                in = in && r2_in_range(r2[u]);
+            }
+            if (__all(in)) {
+#pragma unroll
+                for (int u = 0; u < EN_K; u++) {
+                    const double y = __builtin_amdgcn_rsq(r2[u]);
+                    double h = 0.5 * y, s = r2[u] * y;
+                    double c = __builtin_fma(-h, s, 0.5);
+                    h = __builtin_fma(h, c, h);
+                    s = __builtin_fma(s, c, s);
+                    c = __builtin_fma(-h, s, 0.5);
+                    h = __builtin_fma(h, c, h);
+                    inv[u] = h + h;
+                }
+#pragma unroll
+                for (int u = 0; u < EN_K; u++) e -= w[u] * inv[u];
+            } else {
+#pragma unroll
+                for (int u = 0; u < EN_K; u++) e -= w[u] / __builtin_sqrt(r2[u]);
+            }
         }
     }
-    red[threadIdx.x] = e;
-    __syncthreads();
-    for (int s = EN_BLOCK / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partials[blockIdx.x] = red[0];
+    for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o);
+    if (lane == 0) partials[blockIdx.y * nb + bi] = e;
+}
+
+// Wavefronts: enough chunks of offsets for 8 per CU where there are that many offsets.
+static dim3 energy_grid(int n, int cu_count, int *offsets)
+{
+    const int nb = (n + 63) / 64, all = nb / 2 + 1;
+    int chunks = (8 * cu_count + nb - 1) / nb;
+    if (chunks > all) chunks = all;
+    *offsets = (all + chunks - 1) / chunks;
+    return dim3(nb, (all + *offsets - 1) / *offsets);
+}
+
+int energy_partials(Context *c, int n)
+{
+    int offsets;
+    const dim3 g = energy_grid(n, c->cu_count, &offsets);
+    return static_cast<int>(g.x * g.y);
 }
 
 hipError_t launch_energy(Context *c, const double *x, const double *v, const double *m, int n,
-                         double G, double *partials, int *num_partials)
+                         double G, double *partials)
 {
-    const int grid = (n + EN_BLOCK - 1) / EN_BLOCK;
-    *num_partials = grid;
-    hipLaunchKernelGGL(k_energy, dim3(grid), dim3(EN_BLOCK), 0, c->stream, x, v, m, n, G,
-                       partials);
+    int offsets;
+    const dim3 grid = energy_grid(n, c->cu_count, &offsets);
+    hipLaunchKernelGGL(k_energy, grid, dim3(64), 0, c->stream, x, v, m, n, G, offsets, partials);
     return hipGetLastError();
 }
 

@@ -124,7 +124,7 @@ size_t direct_f32_partial_bytes(int n, const Fp32Config &cfg, int cu_count);
 hipError_t launch_direct_f32_targets(Context *c, const double *x, const double *m, int n, double G,
                                      double eps, const int *targets, int nt, double *out,
                                      void *buf, size_t bytes);
-size_t direct_f32_targets_bytes(int n, int nt);
+size_t direct_f32_targets_bytes(Context *c, int n, int nt);
 // out[t] = src[idx[t]] for rows of 3 doubles.
 hipError_t launch_gather_rows3(Context *c, const double *src, const int *idx, int nt, double *out);
 // FP32 issue-rate probe: kind 0 v_fmac_f32, 1 v_mul_f32, 2 v_rsq_f32 chains,
@@ -140,9 +140,11 @@ hipError_t launch_direct_f64_sampled(Context *c, const double *x, const double *
 size_t direct_f64_sampled_bytes(int n, int nt);
 Fp32Config &fp32_config();
 
-// FP64 energy (src/utils.c:27-59 formula; reduction order differs).
+// FP64 energy (src/utils.c:27-59 formula; reduction order differs):
+// energy_partials(c, n) partial sums, whose total is the energy.
+int energy_partials(Context *c, int n);
 hipError_t launch_energy(Context *c, const double *x, const double *v, const double *m, int n,
-                         double G, double *partials, int *num_partials);
+                         double G, double *partials);
 
 // One Leapfrog step with the FP64 direct sum (one launch; for many particles
 // the drift, then the sums with the kick): drift (x, xe, v) into (xo, xeo),

@@ -38,7 +38,7 @@ static ErrorStatus spot_check(Context *c, const double *x, const double *m, int 
                               double eps, const double *a, int ns, double *p99)
 {
     const std::vector<int> tg = strided_targets(n, ns);
-    const size_t need_bytes = direct_f32_targets_bytes(n, ns);
+    const size_t need_bytes = direct_f32_targets_bytes(c, n, ns);
     void *buf, *sp;
     GS_TRY(slot(c, SLOT_PARTIAL, need_bytes, &buf));
     const size_t off = ((sizeof(int) * ns + 255) / 256) * 256;
@@ -270,7 +270,7 @@ static ErrorStatus build_samples(Context *c, const System *system, double eps, d
     S.idx.assign(perm.begin(), perm.begin() + ns);
     // labels from the FP32 split-precision direct sum
     void *sp, *buf;
-    const size_t lb = direct_f32_targets_bytes(n, ns);
+    const size_t lb = direct_f32_targets_bytes(c, n, ns);
     GS_TRY(slot(c, SLOT_PARTIAL, lb, &buf));
     auto up = [](size_t b) { return ((b + 255) / 256) * 256; };
     const size_t off_ref = up(sizeof(int) * ns);

@@ -136,3 +136,29 @@ def test_issue_rate_probe_is_plausible():
     r = L.issue_rates()
     print("issue rates (cycles per wave64 instruction):", r)
     assert 1.0 <= r["mul"] <= 1.1 * r["fma"] and r["rsq"] > r["mul"]
+
+
+@pytest.mark.parametrize("n", [15, 16, 17, 64, 65, 1000, 2047, 5000, 11585, 16384, 23200])
+def test_fp32_source_units_vs_fp64(n):
+    """The automatic division of the sources (16-source units for the fewest targets, whole tiles from about 11 600
+    particles, 1, 2 or 4 tiles per wavefront) against the FP64 sum, with the file's error bounds."""
+    x, v, m = ic.plummer(n, 19)
+    ref = L.acceleration(x, m, 1, G=1.3, eps=1e-2)  # (bitwise the oracle's)
+    a32 = L.acceleration(x, m, 16, G=1.3, eps=1e-2)
+    e = rel_err(a32, ref)
+    assert np.median(e) <= 1e-6 and e.max() <= 1e-4, (np.median(e), e.max())
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 128, 129, 191, 192, 193, 1000, 3001])
+def test_energy_blocks_vs_oracle(n):
+    """Odd and even numbers of 64-particle blocks, ragged last blocks, a massless particle and particles at a distance
+    whose square is outside the fast reciprocal root's range."""
+    rng = np.random.default_rng(n)
+    x, v, m = rng.normal(size=(n, 3)), rng.normal(size=(n, 3)), rng.uniform(0.1, 1.0, n)
+    m[n // 2] = 0.0 if n > 2 else m[n // 2]
+    for scale in (1.0, 1e-70):
+        sim = L.Sim(x * scale, v, m, 0.7)
+        e, ref = sim.energy(), O.energy(x * scale, v, m, 0.7)
+        sim.close()
+        # each term rounds to a few 2^-53; |sum of terms| / |energy| is bounded here by 1e2
+        assert abs(e - ref) <= 1e-13 * abs(ref)
