@@ -844,11 +844,14 @@ struct F32pPlan {
 
 // With a given split, tiles in that many chunks.  Otherwise a wavefront takes
 // 4 tiles (1024 sources; more only where 64-target groups alone give over
-// 2^14 workgroups), fewer while that leaves under 8 wavefronts per SIMD, then
-// parts of a tile down to 16 sources: a wavefront waits for its scalar loads
-// about 6 times as long as it computes on them, so the chip needs all its
-// wavefronts, and the sums' folds cost little next to that (n = 6007, kernel:
-// 46 us with whole tiles in one chunk, 14 us here; n = 131072 4.33 ms either way).
+// 2^14 workgroups), then 2 and 1 while the chip gets fewer rounds of
+// wavefronts (8 per SIMD) than the tail of the last one can hide in, then
+// parts of a tile down to 16 sources until there are two rounds: a wavefront
+// waits for its scalar loads about 6 times as long as it computes on them, so
+// every SIMD needs its 8, and the sums' folds cost little next to that.
+// Evaluations at n = 6007: 49 us with whole tiles in one chunk, 23 here (16
+// and 128 sources a unit: 24 and 27); 12000: 73, 54 (64 and 256: 52 and 61);
+// 24000: 197, 175 (2 tiles: 193); 131072: 4.4 ms either way.
 static F32pPlan f32p_plan(int n, int targets, int W, int split, int cu_count)
 {
     F32pPlan p;
@@ -861,10 +864,10 @@ static F32pPlan f32p_plan(int n, int targets, int W, int split, int cu_count)
         const long long groups = (targets + 63) / 64, full = 32ll * cu_count;
         const long long total = groups * ntiles;  // wavefronts at one tile each
         long long upw = 1;
-        if (total >= 4 * full) upw = std::max(4ll, (total + 32 * full - 1) / (32 * full));
-        else if (total >= full) upw = total / full;
+        if (total > 32 * full) upw = std::max(4ll, (total + 32 * full - 1) / (32 * full));
+        else if (total > 8 * full) upw = 2;
         else
-            while (p.sh < F32P_MAX_SH && (total << p.sh) < full) p.sh++;
+            while (p.sh < F32P_MAX_SH && (total << p.sh) < 2 * full) p.sh++;
         const int unit = ST_TILE >> p.sh;
         p.units = (n + unit - 1) / unit;
         p.units_per_chunk = static_cast<int>(std::min<long long>(upw * W, p.units));
