@@ -15,11 +15,11 @@
 //                  search on the sorted keys, counted, scanned, emitted)
 //   multipoles     bottom-up per level; leaves sum their particles in sorted
 //                  order, internal nodes sum their children (FP64)
-//   k_walk         one wavefront walks for 64 Morton-consecutive targets with
-//                  a shared explicit stack of (node, lane mask): each lane
-//                  applies the reference opening test to its own particle;
-//                  lanes that accept a node add its monopole, the others
-//                  descend.  Geometry and sums in FP64, 1/r^3 through FP32
+//   k_walk         one wavefront walks for 4 to 16 Morton-consecutive targets
+//                  with a shared explicit stack of (node, target mask), up to
+//                  64 entries a pass: each target applies the reference
+//                  opening test itself; those that accept a node add its
+//                  monopole, the others descend.  Geometry and sums in FP64, 1/r^3 through FP32
 //                  rsqrt.
 #include <cmath>
 #include <cstring>
@@ -990,9 +990,11 @@ __global__ void k_fb_fix(NodeRec *__restrict__ nodes, int nn, const long long *_
 }
 
 // ------------------------------------------------------------------ walk
-constexpr int WK_BLOCK = 256;
-constexpr int WK_WAVES = WK_BLOCK / 64;
-constexpr int WK_STACK = 192;  // >= 7 pending siblings x 21 levels + 8
+// Batch passes keep the stack below WK_BATCH_LIMIT; single-node passes then
+// grow it by at most 7 per level of the remaining depth.
+constexpr int WK_STACK = 1024;
+constexpr int WK_ILP = 2;  // entries a lane works on at a time
+constexpr int WK_BATCH_LIMIT = WK_STACK - 8 * (MAXL + 2);
 
 struct WalkArgs {
     double theta2;
@@ -1066,174 +1068,264 @@ __device__ __forceinline__ void oct_term(const float *__restrict__ T, double R0,
     o2 = su * r2 + 7.5f * w2 * ir7 - 1.5f * t2 * ir5;
 }
 
+// One wavefront walks for T = 64 / G Morton-consecutive targets with one
+// stack of (node, target mask) entries.  A pass takes up to 64 entries off
+// the stack, one per lane: every lane loads its node's record (and moments),
+// so one memory latency covers them all, and leaves it in LDS; then lane
+// sub * T + t applies the opening test to target t and the entries
+// sub, sub + G, ...; the targets that open an entry form the mask of its
+// children.  The interaction set is exactly the per-particle walk's; only the
+// order of the FP64 sums differs.
+//
+// Bound by VALU issue (16 FP64 instructions of 4.75 cycles per G entries of
+// a pass) once the chip is full.  The walk it replaced visited one node at a
+// time through scalar loads, a latency of 600 to 800 cycles each; what each G
+// measured stands at the choice in tree_walk.
+//
 // QUAD: add the quadrupole term of accepted nodes.  FEAT: do not add it but
 // accumulate per-target features of the walk for the learned correction,
 // 16 FP32 per particle in original order, without the factor G:
 // (quadrupole sum x3, sum (M l^3 / d^6) R x3, sum M l^2 / d^4,
 // sum M l^3 / d^5, accepted nodes, particle interactions, octupole sum x3,
 // 0, 0, 0) with l the node's side, R = x_i - com and d = |R| (softened).
-template <bool QUAD, bool FEAT>
-__global__ __launch_bounds__(WK_BLOCK) void k_walk(const NodeRec *__restrict__ nodes,
-                                                   const double4 *__restrict__ P,
-                                                   const long long *__restrict__ skeys,
-                                                   const int *__restrict__ sidx, int n,
-                                                   WalkArgs args, double *__restrict__ a,
-                                                   unsigned long long *__restrict__ n_int,
-                                                   const float *__restrict__ quad,
-                                                   const float *__restrict__ oct,
-                                                   float *__restrict__ feat)
-{
-    __shared__ int stk_node[WK_WAVES][WK_STACK];
-    __shared__ unsigned long long stk_mask[WK_WAVES][WK_STACK];
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int s = (blockIdx.x * WK_WAVES + wave) * 64 + lane;
-    const bool valid = s < n;
-    const unsigned long long all = __ballot(valid);
-    if (all == 0) return;
+struct WalkEntry {
+    double cx, cy, cz;  // centre of mass; of a single-particle leaf its particle
+    double l2;          // (-1 there: below every theta^2 d^2)
+    float mass;
+    int first, count;
+    int single;
+};
+static_assert(sizeof(WalkEntry) == 48, "three 16-byte LDS reads");
 
-    double xi0 = 0.0, xi1 = 0.0, xi2 = 0.0;
-    long long key = 0;
-    if (valid) {
-        const double4 p = P[s];
-        xi0 = p.x;
-        xi1 = p.y;
-        xi2 = p.z;
-        key = skeys[s];
-    }
+template <int G, bool QUAD, bool FEAT>
+__global__ __launch_bounds__(64) void k_walk(const NodeRec *__restrict__ nodes,
+                                             const double4 *__restrict__ P,
+                                             const int *__restrict__ sidx, int n, WalkArgs args,
+                                             double *__restrict__ a,
+                                             unsigned long long *__restrict__ n_int,
+                                             const float *__restrict__ quad,
+                                             const float *__restrict__ oct,
+                                             float *__restrict__ feat)
+{
+    constexpr int T = 64 / G;
+    using Mask = unsigned;  // one bit per target
+    static_assert(G >= 2 && 64 % (WK_ILP * G) == 0, "targets fit a Mask; the slots of a pass divide evenly");
+    constexpr Mask TMASK = static_cast<Mask>(~0ull >> (64 - T));
+    __shared__ int stk_node[WK_STACK];
+    __shared__ Mask stk_mask[WK_STACK];
+    __shared__ __align__(16) WalkEntry ent[64];
+    __shared__ Mask emask[64];  // targets that visit the entry, then those that open it
+    __shared__ __align__(16) float4 eq[QUAD || FEAT ? 64 : 1][2];
+    __shared__ __align__(16) float4 eo[FEAT ? 64 : 1][3];
+    const int lane = threadIdx.x;
+    const int sub = lane / T, tl = lane % T;
+    const int s = blockIdx.x * T + tl;
+    const bool valid = s < n;
+    const double4 ps = P[valid ? s : n - 1];
     double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-    unsigned cnt = 0;             // per-lane interactions of the rare opened-leaf path
-    unsigned long long wcnt = 0;  // the wavefront's other interactions (uniform)
+    unsigned long long wcnt = 0;  // the wavefront's interactions (uniform)
+    bool overflow = false;
     float fq0 = 0.0f, fq1 = 0.0f, fq2 = 0.0f, fs2 = 0.0f, fs3 = 0.0f;
     float fv0 = 0.0f, fv1 = 0.0f, fv2 = 0.0f;
     float fo0 = 0.0f, fo1 = 0.0f, fo2 = 0.0f;
     unsigned nacc = 0, npp = 0;
-    int *snode = stk_node[wave];
-    unsigned long long *smask = stk_mask[wave];
 
-    int sp = 0;
-    {
-        const int c0 = nodes[0].child0, nc = nodes[0].nchild;
-        for (int c = nc - 1; c >= 0; c--) {
-            if (lane == 0) {
-                snode[sp] = c0 + c;
-                smask[sp] = all;
-            }
-            sp++;
-        }
-    }
-    __builtin_amdgcn_wave_barrier();
-    while (sp > 0) {
-        sp--;
-        const int node = __builtin_amdgcn_readfirstlane(snode[sp]);
-        const unsigned long long M =
-            (static_cast<unsigned long long>(__builtin_amdgcn_readfirstlane(
-                 static_cast<int>(smask[sp] >> 32)))
-             << 32) |
-            static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(smask[sp])));
-        __builtin_amdgcn_wave_barrier();
+    // the root holds every target: its children are the first pass (a root
+    // that is a leaf is opened like any other)
+    int top = 0;
+    int kn = 1;
+    int node = 0;
+    Mask mask = static_cast<Mask>(__ballot(valid)) & TMASK;
+    while (kn > 0) {
+        const bool have = lane < kn;
         const NodeRec nd = nodes[node];
-        // (M is uniform: the lane's bit as a per-lane predicate, no VALU work)
-        const bool act = __builtin_amdgcn_inverse_ballot_w64(M);
-        unsigned long long O = 0;  // lanes that open this node
+        const bool single = nd.nchild == 0 && nd.count == 1;
+        {
+            WalkEntry e;
+            e.cx = nd.cx, e.cy = nd.cy, e.cz = nd.cz;
+            e.l2 = nd.l2;
+            e.mass = nd.fmass;
+            e.first = nd.first;
+            e.count = nd.count;
+            e.single = single;
+            if (single) {
+                const double4 p = P[nd.first];
+                e.cx = p.x, e.cy = p.y, e.cz = p.z;
+                e.mass = static_cast<float>(p.w);
+                e.l2 = -1.0;  // accepted by every other target
+            }
+            ent[lane] = e;
+            emask[lane] = have ? mask : 0;
+            if (QUAD || FEAT) {
+                const float4 *q = reinterpret_cast<const float4 *>(quad + 8 * static_cast<size_t>(node));
+                eq[lane][0] = q[0];
+                eq[lane][1] = q[1];
+            }
+            if (FEAT) {
+                const float4 *q = reinterpret_cast<const float4 *>(oct + 12 * static_cast<size_t>(node));
+                eo[lane][0] = q[0];
+                eo[lane][1] = q[1];
+                eo[lane][2] = q[2];
+            }
+        }
+        __syncthreads();
         // The VALU executes an instruction for the whole wavefront whatever
         // its lane mask, so the terms are formed branch-free for every lane
         // and lanes that do not take them add an exact zero (the running sums
         // start at +0 and a sum of products that cancels is +0, never -0, so
         // adding fma(-0, R, a) = a leaves every bit unchanged).
-        if (nd.nchild == 0 && nd.count == 1) {
-            // single-particle leaf: its monopole is the particle itself
-            const bool use = act && nd.first != s;
-            wcnt += static_cast<unsigned>(__popcll(__ballot(use)));
-            {
-                const double4 p = P[nd.first];
-                const double R0 = xi0 - p.x, R1 = xi1 - p.y, R2 = xi2 - p.z;
-                const double r2 = R0 * R0 + R1 * R1 + R2 * R2 + args.eps2;
-                const float ri = __builtin_amdgcn_rsqf(static_cast<float>(r2));
-                const float mr3 = static_cast<float>(p.w) * (ri * ri * ri);
-                const double w = static_cast<double>(use ? mr3 : 0.0f);
-                a0 = __builtin_fma(-w, R0, a0);
-                a1 = __builtin_fma(-w, R1, a1);
-                a2 = __builtin_fma(-w, R2, a2);
-                if (FEAT) npp += use ? 1u : 0u;
+        // (two entries at a time, so that their chains overlap; the slots past
+        // kn hold the root and no targets)
+        for (int e0 = 0; e0 < kn; e0 += WK_ILP * G) {
+            WalkEntry e[WK_ILP];
+            Mask M[WK_ILP];
+            double R0[WK_ILP], R1[WK_ILP], R2[WK_ILP], d2[WK_ILP], w[WK_ILP];
+            float ri[WK_ILP], mr3[WK_ILP];
+            bool accept[WK_ILP];
+#pragma unroll
+            for (int u = 0; u < WK_ILP; u++) {
+                e[u] = ent[e0 + u * G + sub];
+                M[u] = emask[e0 + u * G + sub];
             }
-            continue;
-        }
-        const bool included = (key >> (3 * (MAXL - nd.depth))) == nd.prefix;
-        const double R0 = xi0 - nd.cx, R1 = xi1 - nd.cy, R2 = xi2 - nd.cz;
-        const double d2 = R0 * R0 + R1 * R1 + R2 * R2;
-        const double l2 = nd.l2;
-        const bool accept = act && !included && l2 < args.theta2 * d2;
-        const unsigned long long AM = __ballot(accept);
-        wcnt += static_cast<unsigned>(__popcll(AM));
-        O = M & ~AM;  // act && !accept
-        // (no branch around the terms: a visit where no lane accepts is rare
-        // enough that computing them anyway is cheaper than merging the sums)
-        {
-            const float ri = __builtin_amdgcn_rsqf(static_cast<float>(d2 + args.eps2));
-            const float mr3 = nd.fmass * (ri * ri * ri);
-            const double w = static_cast<double>(accept ? mr3 : 0.0f);
-            a0 = __builtin_fma(-w, R0, a0);
-            a1 = __builtin_fma(-w, R1, a1);
-            a2 = __builtin_fma(-w, R2, a2);
+#pragma unroll
+            for (int u = 0; u < WK_ILP; u++) {
+                R0[u] = ps.x - e[u].cx;
+                R1[u] = ps.y - e[u].cy;
+                R2[u] = ps.z - e[u].cz;
+            }
+#pragma unroll
+            for (int u = 0; u < WK_ILP; u++) d2[u] = R0[u] * R0[u] + R1[u] * R1[u] + R2[u] * R2[u];
+#pragma unroll
+            for (int u = 0; u < WK_ILP; u++) {
+                ri[u] = __builtin_amdgcn_rsqf(static_cast<float>(d2[u] + args.eps2));
+                const bool own = static_cast<unsigned>(s - e[u].first) < static_cast<unsigned>(e[u].count);
+                accept[u] = ((M[u] >> tl) & 1u) && !own && e[u].l2 < args.theta2 * d2[u];
+            }
+#pragma unroll
+            for (int u = 0; u < WK_ILP; u++) {
+                const unsigned long long A = __ballot(accept[u]);
+                wcnt += static_cast<unsigned>(__popcll(A));
+                if (tl == 0) emask[e0 + u * G + sub] = M[u] & ~(static_cast<Mask>(A >> (sub * T)) & TMASK);
+                mr3[u] = e[u].mass * (ri[u] * ri[u] * ri[u]);
+                w[u] = static_cast<double>(accept[u] ? mr3[u] : 0.0f);
+            }
+#pragma unroll
+            for (int u = 0; u < WK_ILP; u++) {
+                a0 = __builtin_fma(-w[u], R0[u], a0);
+                a1 = __builtin_fma(-w[u], R1[u], a1);
+                a2 = __builtin_fma(-w[u], R2[u], a2);
+            }
             if (QUAD || FEAT) {
-                float o0, o1, o2;
-                quad_term(quad + 8 * static_cast<size_t>(node), R0, R1, R2, ri, o0, o1, o2);
-                if (QUAD) {
-                    a0 += static_cast<double>(accept ? o0 : 0.0f);
-                    a1 += static_cast<double>(accept ? o1 : 0.0f);
-                    a2 += static_cast<double>(accept ? o2 : 0.0f);
-                } else {
-                    // M l^2 / d^4 and M l^3 / d^5 (l: cell side, d: distance to the COM)
-                    const float lr = static_cast<float>(__builtin_sqrt(l2)) * ri;
-                    const float mr2 = mr3 * static_cast<float>(__builtin_sqrt(d2 + args.eps2));
-                    const float lr3 = lr * lr * lr;
-                    const float k3 = mr3 * lr3;
-                    float t0, t1, t2;
-                    oct_term(oct + 12 * static_cast<size_t>(node), R0, R1, R2, ri, t0, t1, t2);
-                    if (accept) {
-                        fq0 += o0;
-                        fq1 += o1;
-                        fq2 += o2;
-                        fo0 += t0;
-                        fo1 += t1;
-                        fo2 += t2;
-                        fs2 = __builtin_fmaf(mr2, lr * lr, fs2);
-                        fs3 = __builtin_fmaf(mr2, lr3, fs3);
-                        fv0 = __builtin_fmaf(k3, static_cast<float>(R0), fv0);
-                        fv1 = __builtin_fmaf(k3, static_cast<float>(R1), fv1);
-                        fv2 = __builtin_fmaf(k3, static_cast<float>(R2), fv2);
-                        nacc++;
+#pragma unroll
+                for (int u = 0; u < WK_ILP; u++) {
+                    const int ei = e0 + u * G + sub;
+                    const bool acc_node = accept[u] && !e[u].single;
+                    float o0, o1, o2;
+                    const float4 qa = eq[ei][0], qb = eq[ei][1];
+                    const float q[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+                    quad_term(q, R0[u], R1[u], R2[u], ri[u], o0, o1, o2);
+                    if (QUAD) {
+                        a0 += static_cast<double>(acc_node ? o0 : 0.0f);
+                        a1 += static_cast<double>(acc_node ? o1 : 0.0f);
+                        a2 += static_cast<double>(acc_node ? o2 : 0.0f);
+                    } else {
+                        // M l^2 / d^4 and M l^3 / d^5 (l: cell side, d: distance to the COM)
+                        const float lr = static_cast<float>(__builtin_sqrt(e[u].l2)) * ri[u];
+                        const float mr2 = mr3[u] * static_cast<float>(__builtin_sqrt(d2[u] + args.eps2));
+                        const float lr3 = lr * lr * lr;
+                        const float k3 = mr3[u] * lr3;
+                        const float4 ta = eo[ei][0], tb = eo[ei][1], tc = eo[ei][2];
+                        const float tt[10] = {ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w, tc.x, tc.y};
+                        float t0, t1, t2;
+                        oct_term(tt, R0[u], R1[u], R2[u], ri[u], t0, t1, t2);
+                        if (acc_node) {
+                            fq0 += o0;
+                            fq1 += o1;
+                            fq2 += o2;
+                            fo0 += t0;
+                            fo1 += t1;
+                            fo2 += t2;
+                            fs2 = __builtin_fmaf(mr2, lr * lr, fs2);
+                            fs3 = __builtin_fmaf(mr2, lr3, fs3);
+                            fv0 = __builtin_fmaf(k3, static_cast<float>(R0[u]), fv0);
+                            fv1 = __builtin_fmaf(k3, static_cast<float>(R1[u]), fv1);
+                            fv2 = __builtin_fmaf(k3, static_cast<float>(R2[u]), fv2);
+                            nacc++;
+                        } else if (accept[u]) {
+                            npp++;
+                        }
                     }
                 }
             }
         }
-        if (O == 0) continue;
-        if (nd.nchild == 0) {
-            const bool mine = __builtin_amdgcn_inverse_ballot_w64(O);
-            for (int t = nd.first; t < nd.first + nd.count; t++) {
-                const double4 p = P[t];
-                if (mine && t != s) {
-                    pp_force(xi0, xi1, xi2, p.x, p.y, p.z, p.w, args.eps2, a0, a1, a2);
-                    cnt++;
-                    npp++;
+        __syncthreads();
+        const Mask O = have && !single ? emask[lane] : 0;
+        // opened leaves of several particles: their particles one by one
+        unsigned long long multi = __ballot(O != 0 && nd.nchild == 0);
+        while (multi) {
+            const int k = __ffsll(static_cast<long long>(multi)) - 1;
+            multi &= multi - 1;
+            const int first = __builtin_amdgcn_readlane(nd.first, k);
+            const int count = __builtin_amdgcn_readlane(nd.count, k);
+            const bool mine = (emask[k] >> tl) & 1u;
+            for (int t0 = first; t0 < first + count; t0 += G) {
+                const int t = t0 + sub;
+                const bool use = mine && t < first + count && t != s;
+                const double4 p = P[t < first + count ? t : first];
+                if (use) pp_force(ps.x, ps.y, ps.z, p.x, p.y, p.z, p.w, args.eps2, a0, a1, a2);
+                wcnt += static_cast<unsigned>(__popcll(__ballot(use)));
+                if (FEAT) npp += use ? 1u : 0u;
+            }
+        }
+        // opened internal nodes -> children on the stack, in lane order: the
+        // exclusive prefix of the child counts (0..8) from four bit-plane
+        // ballots
+        {
+            const int c = O != 0 ? nd.nchild : 0;
+            const unsigned long long below = (1ull << lane) - 1;
+            int before = 0, total = 0;
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const unsigned long long B = __ballot((c >> b) & 1);
+                before += __popcll(B & below) << b;
+                total += __popcll(B) << b;
+            }
+            if (top + total <= WK_STACK) {
+                for (int q = 0; q < c; q++) {
+                    stk_node[top + before + q] = nd.child0 + q;
+                    stk_mask[top + before + q] = O;
                 }
+                top += total;
+            } else {
+                overflow = true;
             }
-        } else if (sp + nd.nchild <= WK_STACK) {
-            // children pushed last-to-first (child0 on top), one lane each
-            if (lane < nd.nchild) {
-                snode[sp + lane] = nd.child0 + nd.nchild - 1 - lane;
-                smask[sp + lane] = O;
-            }
-            sp += nd.nchild;
-            __builtin_amdgcn_wave_barrier();
-        } else if (lane == 0 && n_int) {
-            // cannot happen for depth <= 21 (at most 7 pending siblings per
-            // level); flagged through the counter instead of overflowing
-            atomicAdd(n_int, 1ull << 62);
+        }
+        __syncthreads();
+        kn = min(top, 64);
+        if (top + 7 * kn > WK_BATCH_LIMIT) kn = max(1, (WK_BATCH_LIMIT - top) / 7);
+        kn = min(kn, top);
+        node = 0;
+        mask = 0;
+        if (lane < kn) {
+            node = stk_node[top - kn + lane];
+            mask = stk_mask[top - kn + lane];
+        }
+        top -= kn;
+    }
+#pragma unroll
+    for (int o = T; o < 64; o <<= 1) {
+        a0 += __shfl_xor(a0, o);
+        a1 += __shfl_xor(a1, o);
+        a2 += __shfl_xor(a2, o);
+        if (FEAT) {
+            fq0 += __shfl_xor(fq0, o), fq1 += __shfl_xor(fq1, o), fq2 += __shfl_xor(fq2, o);
+            fv0 += __shfl_xor(fv0, o), fv1 += __shfl_xor(fv1, o), fv2 += __shfl_xor(fv2, o);
+            fo0 += __shfl_xor(fo0, o), fo1 += __shfl_xor(fo1, o), fo2 += __shfl_xor(fo2, o);
+            fs2 += __shfl_xor(fs2, o), fs3 += __shfl_xor(fs3, o);
+            nacc += __shfl_xor(nacc, o), npp += __shfl_xor(npp, o);
         }
     }
-    if (valid) {
+    if (valid && sub == 0) {
         const int i = sidx[s];
         a[3 * i + 0] = args.G * a0;
         a[3 * i + 1] = args.G * a1;
@@ -1246,10 +1338,9 @@ __global__ __launch_bounds__(WK_BLOCK) void k_walk(const NodeRec *__restrict__ n
             f[3] = make_float4(fo2, 0.0f, 0.0f, 0.0f);
         }
     }
-    // interaction count: one atomic per wave
-    unsigned long long tot = cnt;
-    for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off);
-    if (lane == 0 && n_int) atomicAdd(n_int, tot + wcnt);
+    // interaction count: one atomic per wave (an overflow, which the batch
+    // limit excludes, is flagged through it)
+    if (lane == 0 && n_int) atomicAdd(n_int, wcnt + (overflow ? 1ull << 62 : 0ull));
 }
 
 // ------------------------------------------------------------------ group walk
@@ -2238,21 +2329,28 @@ ErrorStatus tree_walk(Context *c, DeviceTree *t, const double *x, double G, doub
     GS_TRY(slot(c, SLOT_MISC, 256, &p));
     unsigned long long *cnt = reinterpret_cast<unsigned long long *>(static_cast<char *>(p) + 64);
     GS_HIP(hipMemsetAsync(cnt, 0, sizeof(unsigned long long), c->stream));
-    const int waves = (t->n + 63) / 64;
-    const int grid = (waves + WK_WAVES - 1) / WK_WAVES;
     const int rec = timing_begin(c, "bh_walk");
-    if (feat)
-        hipLaunchKernelGGL((k_walk<false, true>), dim3(grid), dim3(WK_BLOCK), 0, c->stream,
-                           t->nodes, t->P, t->skeys, t->sidx, t->n, args, a, cnt, t->quadf, t->octf,
-                           feat);
-    else if (order >= 2)
-        hipLaunchKernelGGL((k_walk<true, false>), dim3(grid), dim3(WK_BLOCK), 0, c->stream,
-                           t->nodes, t->P, t->skeys, t->sidx, t->n, args, a, cnt, t->quadf, t->octf,
-                           feat);
-    else
-        hipLaunchKernelGGL((k_walk<false, false>), dim3(grid), dim3(WK_BLOCK), 0, c->stream,
-                           t->nodes, t->P, t->skeys, t->sidx, t->n, args, a, cnt, t->quadf, t->octf,
-                           feat);
+    auto walk = [&](auto kernel, int g) {
+        const int targets = 64 / g;
+        hipLaunchKernelGGL(kernel, dim3((t->n + targets - 1) / targets), dim3(64), 0, c->stream,
+                           t->nodes, t->P, t->sidx, t->n, args, a, cnt, t->quadf, t->octf, feat);
+    };
+    // Entries per pass step.  More entries, fewer targets per wavefront: more
+    // wavefronts and fewer nodes that only some of the targets visit, but
+    // more passes per target.  Monopole walk, theta 0.5, us for G = 1 / 2 / 4
+    // / 8 / 16 (and the walk by single nodes before): n = 10000: 475 / 239 /
+    // 141 / 94 / 76 (1022); 60000: 799 / 441 / 286 / 279 / 350 (1721); 262144:
+    // 1818 / 1161 / 1078 / 1191 / 1571 (2636); 2097152: 13014 / 8750 / 8848 /
+    // 10251 / 13868 (12623).  With quadrupoles at 2097152: 20.3 / 15.7 / 15.5
+    // / 16.8 / 21.0 ms (18.1).
+    auto pick = [&](auto k4, auto k8, auto k16) {
+        if (t->n <= 64 * c->cu_count) walk(k16, 16);
+        else if (t->n <= 512 * c->cu_count) walk(k8, 8);
+        else walk(k4, 4);
+    };
+    if (feat) pick(k_walk<4, false, true>, k_walk<8, false, true>, k_walk<16, false, true>);
+    else if (order >= 2) pick(k_walk<4, true, false>, k_walk<8, true, false>, k_walk<16, true, false>);
+    else pick(k_walk<4, false, false>, k_walk<8, false, false>, k_walk<16, false, false>);
     timing_end(c, rec);
     GS_HIP(hipGetLastError());
     if (interactions) {

@@ -428,3 +428,19 @@ def test_group_walk_beyond_one_scan_level():
     sim.close()
     print(f"group walk N=6e6 uniform: median {med:.2e} p99 {p99:.2e}")
     assert med < 1e-3 and p99 < 5e-3
+
+
+@pytest.mark.parametrize("n", [2, 62, 66, 16384, 16386, 131072, 131074])
+@pytest.mark.parametrize("leaf", [1, 8])
+def test_walk_forms_against_the_oracle(n, leaf):
+    """Around the sizes where the walk changes the number of targets per wavefront (16384 / 16386, 131072 / 131074 on
+    256 CUs) and at the smallest: equal interaction counts, forces to FP32 rounding; monopoles and quadrupoles."""
+    x, v, m = ic.two_spheres(n, 50 + n % 97)
+    t = O.build_tree(x, m, leaf)
+    q = O.octree_quad(x, m, t)
+    for method, quad in ((3, None), (19, q)):
+        a = L.acceleration(x, m, method, eps=1e-2, theta=0.7, leaf=leaf)
+        ao, cnt = O.bh_walk(x, m, t, 0.7, eps=1e-2, want_counts=True, quad=quad)
+        assert L.last_walk_interactions() == int(cnt.sum())
+        e = np.linalg.norm(a - ao, axis=1) / np.linalg.norm(ao, axis=1)
+        assert np.median(e) < 1e-6 and e.max() < 1e-4
