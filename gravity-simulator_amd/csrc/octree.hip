@@ -23,6 +23,7 @@
 //                  rsqrt.
 #include <cmath>
 #include <cstring>
+#include <utility>
 
 #include "gs_internal.h"
 #include "octree.h"
@@ -150,12 +151,12 @@ __global__ void k_morton(const double *__restrict__ x, int n, const double *__re
 // ------------------------------------------------------------------ radix sort
 constexpr int RS_BLOCK = 256;
 constexpr int RS_WAVES = RS_BLOCK / 64;
-constexpr int RS_ROUNDS = 8;                          // keys per lane
-constexpr int RS_TILE = RS_BLOCK * RS_ROUNDS;         // 2048 keys per tile
+constexpr int RS_MAX_ROUNDS = 8;                      // keys per lane: 2048 per tile
 constexpr int RS_BITS = 8;
 constexpr int RS_BINS = 1 << RS_BITS;
 constexpr int RS_PASSES = 8;                          // 64 bits (bit 63 is always 0)
 
+template <int ROUNDS>
 __global__ __launch_bounds__(RS_BLOCK) void k_rs_hist(const long long *__restrict__ keys, int n,
                                                       int shift, unsigned *__restrict__ hist,
                                                       int ntiles)
@@ -163,8 +164,9 @@ __global__ __launch_bounds__(RS_BLOCK) void k_rs_hist(const long long *__restric
     __shared__ unsigned h[RS_BINS];
     h[threadIdx.x] = 0;
     __syncthreads();
-    const int base = blockIdx.x * RS_TILE;
-    for (int k = 0; k < RS_ROUNDS; k++) {
+    const int base = blockIdx.x * (RS_BLOCK * ROUNDS);
+#pragma unroll
+    for (int k = 0; k < ROUNDS; k++) {
         const int q = base + k * RS_BLOCK + threadIdx.x;
         if (q < n) atomicAdd(&h[(keys[q] >> shift) & (RS_BINS - 1)], 1u);
     }
@@ -219,12 +221,13 @@ __global__ __launch_bounds__(RS_BLOCK) void k_rs_rowscan(unsigned *__restrict__ 
     if (threadIdx.x == 0) dtot[blockIdx.x] = carry;
 }
 
-// Stable scatter: wave w owns tile positions [w*512, (w+1)*512), visited in
-// 8 rounds of 64 consecutive keys; within a round, peers with equal digits
+// Stable scatter: wave w owns a quarter of the tile's positions, visited
+// in rounds of 64 consecutive keys; within a round, peers with equal digits
 // are found with 8 ballots and ranked by lane order.  The tile is then
 // reordered by digit in LDS, so that consecutive threads write consecutive
 // addresses of each digit's run instead of scattering single keys.
 static_assert(RS_BLOCK == RS_BINS, "one thread per digit for the tile offsets");
+template <int ROUNDS>
 __global__ __launch_bounds__(RS_BLOCK) void k_rs_scatter(const long long *__restrict__ kin,
                                                          const int *__restrict__ iin, int n,
                                                          int shift,
@@ -234,13 +237,14 @@ __global__ __launch_bounds__(RS_BLOCK) void k_rs_scatter(const long long *__rest
                                                          long long *__restrict__ kout,
                                                          int *__restrict__ iout)
 {
+    constexpr int TILE = RS_BLOCK * ROUNDS;
     __shared__ unsigned wcount[RS_WAVES][RS_BINS];
     __shared__ unsigned toff[RS_BINS];   // first tile position of each digit
     __shared__ unsigned goff[RS_BINS];   // first output position of each digit
     __shared__ unsigned wsum[RS_WAVES];
     __shared__ unsigned dsum[RS_WAVES];
-    __shared__ long long skey[RS_TILE];
-    __shared__ int sval[RS_TILE];
+    __shared__ long long skey[TILE];
+    __shared__ int sval[TILE];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     for (int b = threadIdx.x; b < RS_WAVES * RS_BINS; b += RS_BLOCK)
@@ -249,16 +253,21 @@ __global__ __launch_bounds__(RS_BLOCK) void k_rs_scatter(const long long *__rest
 
     volatile unsigned *cnt = wcount[wave];
     const unsigned long long lt_mask = (1ull << lane) - 1ull;
-    const int base = blockIdx.x * RS_TILE + wave * (RS_ROUNDS * 64);
-    long long key[RS_ROUNDS];
-    int val[RS_ROUNDS];
-    unsigned rank[RS_ROUNDS];
-    int dig[RS_ROUNDS];
-    for (int r = 0; r < RS_ROUNDS; r++) {
+    const int base = blockIdx.x * TILE + wave * (ROUNDS * 64);
+    long long key[ROUNDS];
+    int val[ROUNDS];
+    unsigned rank[ROUNDS];
+    int dig[ROUNDS];
+    // (every round's pairs requested before the first is ranked)
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
         const int q = base + r * 64 + lane;
-        const bool ok = q < n;
-        key[r] = ok ? kin[q] : 0;
-        val[r] = ok ? iin[q] : 0;
+        key[r] = kin[q < n ? q : n - 1];
+        val[r] = iin[q < n ? q : n - 1];
+    }
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        const bool ok = base + r * 64 + lane < n;
         const int d = ok ? static_cast<int>((key[r] >> shift) & (RS_BINS - 1)) : -1;
         dig[r] = d;
         unsigned long long peers = __ballot(ok);
@@ -308,7 +317,8 @@ __global__ __launch_bounds__(RS_BLOCK) void k_rs_scatter(const long long *__rest
         goff[d] = dadd + dincl - dt + row;
     }
     __syncthreads();
-    for (int r = 0; r < RS_ROUNDS; r++) {
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
         const int d = dig[r];
         if (d < 0) continue;
         unsigned lp = toff[d] + rank[r];
@@ -317,7 +327,7 @@ __global__ __launch_bounds__(RS_BLOCK) void k_rs_scatter(const long long *__rest
         sval[lp] = val[r];
     }
     __syncthreads();
-    const int tile_n = min(RS_TILE, n - blockIdx.x * RS_TILE);
+    const int tile_n = min(TILE, n - blockIdx.x * TILE);
     for (int p = threadIdx.x; p < tile_n; p += RS_BLOCK) {
         const long long k = skey[p];
         const int d = static_cast<int>((k >> shift) & (RS_BINS - 1));
@@ -1362,9 +1372,18 @@ __global__ __launch_bounds__(64) void k_walk(const NodeRec *__restrict__ nodes,
 // theta 0.5, the launch takes 5.2 ms against 6.0 ms with 2048 entries (fewer
 // resident wavefronts) and 5.8 / 12.2 ms with 768 / 512 (more single-node
 // passes once the frontier reaches the batch limit below).  One wavefront per
-// workgroup: 6.0 ms against 6.7 with two and 8.2 with four (2048 entries).
-constexpr int GW_WAVES = 1;
-constexpr int GW_BLOCK = 64 * GW_WAVES;
+// workgroup: 6.0 ms against 6.7 with two and 8.2 with four groups (2048
+// entries).
+// Few groups do not fill the chip and the one with the longest list sets the
+// time, so for n <= 512 particles per CU GW_SPLIT wavefronts share a group:
+// they take the first passes alike (wavefront 0 collecting the terms) until
+// the stack holds GW_SHARE entries per wavefront, then every GW_SPLIT-th
+// entry each, and their sums are added at the end.  Walk at theta 0.5, one /
+// four / eight / sixteen wavefronts: n = 10000: 363 / 280 / 239 / 382 us,
+// 60000: 2216 / 1335 / 832 / 981, 120000: 900 / - / 655 / 1886, 160000: 517 /
+// - / 856 / -, 262144: 991 / 988 / 1337 / 3636.
+constexpr int GW_SPLIT = 8;
+constexpr int GW_SHARE = 32;
 constexpr int GW_STACK = 1024;
 constexpr int GW_LIST = 128;
 // batch passes keep the stack below this; single-node passes then grow it by
@@ -1670,28 +1689,26 @@ __device__ __forceinline__ void far_eval(FarMoments F, float d0, float d1, float
     o2 = F.A2 + (P2 - F.Q * d2) + d2 * Sd + 0.5f * (F.S2 * dd - T2);
 }
 
-template <bool QUAD, bool LE>
-__global__ __launch_bounds__(GW_BLOCK) void k_walk_group(const NodeRec *__restrict__ nodes,
+template <bool QUAD, bool LE, int W>
+__global__ __launch_bounds__(64 * W) void k_walk_group(const NodeRec *__restrict__ nodes,
                                                          const double4 *__restrict__ P,
                                                          const int *__restrict__ sidx, int n,
                                                          const int2 *__restrict__ groups,
-                                                         int num_groups, WalkArgs args,
+                                                         WalkArgs args,
                                                          double *__restrict__ a,
                                                          unsigned long long *__restrict__ n_int,
                                                          const float *__restrict__ quad)
 {
-    __shared__ int stk_all[GW_WAVES][GW_STACK];
-    __shared__ float4 nl_all[GW_WAVES][GW_LIST];  // accepted nodes: com - centre, mass
-    __shared__ int ni_all[GW_WAVES][GW_LIST];     // their node indices
-    __shared__ float4 pl_all[GW_WAVES][GW_LIST];  // particles: x - centre, mass
-    __shared__ int pi_all[GW_WAVES][GW_LIST];     // their sorted positions
-    __shared__ int rinc_all[GW_WAVES][64];        // opened multi-particle leaves:
-    __shared__ int rbeg_all[GW_WAVES][64];        // inclusive count prefix, first - offset
+    __shared__ __align__(16) int stk_all[W][GW_STACK];
+    __shared__ float4 nl_all[W][GW_LIST];  // accepted nodes: com - centre, mass
+    __shared__ int ni_all[W][GW_LIST];     // their node indices
+    __shared__ float4 pl_all[W][GW_LIST];  // particles: x - centre, mass
+    __shared__ int pi_all[W][GW_LIST];     // their sorted positions
+    __shared__ int rinc_all[W][64];        // opened multi-particle leaves:
+    __shared__ int rbeg_all[W][64];        // inclusive count prefix, first - offset
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int gi = blockIdx.x * GW_WAVES + wave;
-    if (gi >= num_groups) return;
-    const int2 grp = groups[gi];  // (first sorted position, count <= 64)
+    const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int2 grp = groups[blockIdx.x];  // (first sorted position, count <= 64)
     const int g0 = grp.x;
     const int gend = g0 + grp.y;
     const int s = g0 + lane;
@@ -1767,10 +1784,13 @@ __global__ __launch_bounds__(GW_BLOCK) void k_walk_group(const NodeRec *__restri
             float r2 = __builtin_fmaf(dx, dx, eps2);
             r2 = __builtin_fmaf(dy, dy, r2);
             r2 = __builtin_fmaf(dz, dz, r2);
+            // the lane's own entry: an infinite distance, so a zero weight and no
+            // close pair (a select on the weight instead makes the compiler
+            // branch around each row's reciprocal root)
+            r2 = pi[e] == s ? __builtin_inff() : r2;
             const float ri = __builtin_amdgcn_rsqf(r2);
-            const bool me = pi[e] == s;
-            const float w = me ? 0.0f : (q.w * ri) * (ri * ri);
-            mn = fminf(mn, me ? __builtin_inff() : r2);
+            const float w = (q.w * ri) * (ri * ri);
+            mn = fminf(mn, r2);
             f0 = __builtin_fmaf(dx, w, f0);
             f1 = __builtin_fmaf(dy, w, f1);
             f2 = __builtin_fmaf(dz, w, f2);
@@ -1830,7 +1850,9 @@ __global__ __launch_bounds__(GW_BLOCK) void k_walk_group(const NodeRec *__restri
     int k = 1;
     int node = 0;
     NodeRec nd = nodes[0];
+    bool shared = W > 1;  // the wavefronts of the group still walk alike
     while (k > 0) {
+        const bool lead = !shared || wave == 0;
         const bool act = lane < k;
         const bool leaf = nd.nchild == 0;
         const bool single_leaf = act && leaf && nd.count == 1;
@@ -1849,17 +1871,17 @@ __global__ __launch_bounds__(GW_BLOCK) void k_walk_group(const NodeRec *__restri
             const bool farz = rg2 < args.phi2 * (y0 * y0 + y1 * y1 + y2 * y2);
             accept = accept || (!incl && farz && nd.l2 < args.thetaf2 * d2);
             far = act && accept && farz;
-            if (far)
+            if (far && lead)
                 far_add(F, static_cast<float>(y0), static_cast<float>(y1), static_cast<float>(y2),
                         nd.fmass, eps2, quad + 8 * static_cast<size_t>(node));
-            const unsigned nf = __popcll(__ballot(far));
+            const unsigned nf = __popcll(__ballot(far && lead));
             nfar += nf;
             cnt += nf;
         }
         // single-particle leaves not expanded: their particle into the particle list
-        const bool single = single_leaf && !far;
-        const bool take_node = act && !single_leaf && accept && !far;
-        const bool multi = act && leaf && !single_leaf && !accept;
+        const bool single = single_leaf && !far && lead;
+        const bool take_node = act && !single_leaf && accept && !far && lead;
+        const bool multi = act && leaf && !single_leaf && !accept && lead;
         const bool open = act && !leaf && !accept;
         // accepted nodes -> node list
         {
@@ -1905,6 +1927,20 @@ __global__ __launch_bounds__(GW_BLOCK) void k_walk_group(const NodeRec *__restri
             }
         }
         __builtin_amdgcn_wave_barrier();
+        if (W > 1 && shared && top >= GW_SHARE * W) {
+            // every W-th entry from here on (slot i reads slot i W + wave, never
+            // one that an earlier round of the loop wrote)
+            const int mine = (top - wave + W - 1) / W;
+            for (int i0 = 0; i0 < mine; i0 += 64) {
+                const int i = i0 + lane;
+                const int v = i < mine ? stk[i * W + wave] : 0;
+                __builtin_amdgcn_wave_barrier();
+                if (i < mine) stk[i] = v;
+                __builtin_amdgcn_wave_barrier();
+            }
+            top = mine;
+            shared = false;
+        }
         // the next pass: at most 64 entries, fewer when its children could
         // bring the stack past the batch limit
         int kn = min(top, 64);
@@ -1974,7 +2010,26 @@ __global__ __launch_bounds__(GW_BLOCK) void k_walk_group(const NodeRec *__restri
         A1 += static_cast<double>(o1);
         A2 += static_cast<double>(o2);
     }
-    if (valid) {
+    // the wavefronts' sums in wavefront order (their stacks are free now)
+    unsigned long long tot = cnt;
+    if (W > 1) {
+        double(*sum)[64] = reinterpret_cast<double(*)[64]>(stk);
+        static_assert(sizeof(int) * GW_STACK >= 3 * 64 * sizeof(double), "the sums fit the stack");
+        sum[0][lane] = A0;
+        sum[1][lane] = A1;
+        sum[2][lane] = A2;
+        rinc[lane] = static_cast<int>(cnt);
+        __syncthreads();
+        if (wave == 0)
+            for (int w = 1; w < W; w++) {
+                const double(*other)[64] = reinterpret_cast<const double(*)[64]>(stk_all[w]);
+                A0 += other[0][lane];
+                A1 += other[1][lane];
+                A2 += other[2][lane];
+                tot += static_cast<unsigned>(rinc_all[w][lane]);
+            }
+    }
+    if (valid && wave == 0) {
         const int i = sidx[s];
         a[3 * i + 0] = args.G * A0;
         a[3 * i + 1] = args.G * A1;
@@ -1982,10 +2037,10 @@ __global__ __launch_bounds__(GW_BLOCK) void k_walk_group(const NodeRec *__restri
     }
     // (a particle's own entry is in its group's particle list exactly once:
     // every node holding it is opened, down to its leaf)
-    unsigned long long tot = valid ? cnt - 1u : 0u;
+    tot = valid && wave == 0 ? tot - 1u : 0u;
     for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off);
     if (lane == 0 && n_int) {
-        atomicAdd(n_int, tot + (overflow ? (1ull << 62) : 0ull));
+        if (wave == 0 || overflow) atomicAdd(n_int, tot + (overflow ? (1ull << 62) : 0ull));
         if (LE) atomicAdd(n_int + 1, static_cast<unsigned long long>(nfar));
     }
 }
@@ -2030,32 +2085,44 @@ static ErrorStatus ensure_nodes(Context *c, DeviceTree *t, int need)
     return make_success_error_status();
 }
 
+// Keys per lane of a tile: few for few particles, since a tile's rounds are
+// ranked one after the other and the CUs have room for more tiles.  Sort of
+// n = 60000 with 2 / 4 / 8 keys: 95 / 106 / 138 us; 262144: 124 / 124 / 150;
+// 524288: 170 / 151 / 164; 1048576: 269 / 214 / 201.
+static int rs_rounds(int n) { return n <= 262144 ? 2 : n <= 786432 ? 4 : RS_MAX_ROUNDS; }
+
 size_t radix_hist_elements(int n)
 {
     // the tile counts, then the digit totals
-    return static_cast<size_t>((n + RS_TILE - 1) / RS_TILE) * RS_BINS + RS_BINS;
+    const int tile = RS_BLOCK * rs_rounds(n);
+    return static_cast<size_t>((n + tile - 1) / tile) * RS_BINS + RS_BINS;
+}
+
+template <int ROUNDS>
+static void radix_pass(Context *c, const long long *k0, const int *i0, long long *k1, int *i1, int n,
+                       int shift, unsigned *hist)
+{
+    const int ntiles = (n + RS_BLOCK * ROUNDS - 1) / (RS_BLOCK * ROUNDS);
+    unsigned *dtot = hist + static_cast<size_t>(ntiles) * RS_BINS;
+    hipLaunchKernelGGL(k_rs_hist<ROUNDS>, dim3(ntiles), dim3(RS_BLOCK), 0, c->stream, k0, n, shift,
+                       hist, ntiles);
+    hipLaunchKernelGGL(k_rs_rowscan, dim3(RS_BINS), dim3(RS_BLOCK), 0, c->stream, hist, ntiles, dtot);
+    hipLaunchKernelGGL(k_rs_scatter<ROUNDS>, dim3(ntiles), dim3(RS_BLOCK), 0, c->stream, k0, i0, n,
+                       shift, hist, dtot, ntiles, k1, i1);
 }
 
 ErrorStatus radix_sort_pairs(Context *c, long long *k0, int *i0, long long *k1, int *i1, int n,
                              int passes, unsigned *hist, long long **ko, int **io)
 {
-    const int ntiles = (n + RS_TILE - 1) / RS_TILE;
-    unsigned *dtot = hist + static_cast<size_t>(ntiles) * RS_BINS;
+    const int rounds = rs_rounds(n);
     for (int pass = 0; pass < passes; pass++) {
         const int shift = pass * RS_BITS;
-        hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(RS_BLOCK), 0, c->stream, k0, n, shift,
-                           hist, ntiles);
-        hipLaunchKernelGGL(k_rs_rowscan, dim3(RS_BINS), dim3(RS_BLOCK), 0, c->stream, hist, ntiles,
-                           dtot);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(RS_BLOCK), 0, c->stream, k0, i0, n,
-                           shift, hist, dtot, ntiles, k1, i1);
+        if (rounds == 2) radix_pass<2>(c, k0, i0, k1, i1, n, shift, hist);
+        else if (rounds == 4) radix_pass<4>(c, k0, i0, k1, i1, n, shift, hist);
+        else radix_pass<RS_MAX_ROUNDS>(c, k0, i0, k1, i1, n, shift, hist);
         GS_HIP(hipGetLastError());
-        long long *tk = k0;
-        k0 = k1;
-        k1 = tk;
-        int *ti = i0;
-        i0 = i1;
-        i1 = ti;
+        std::swap(k0, k1);
+        std::swap(i0, i1);
     }
     *ko = k0;
     *io = i0;
@@ -2434,19 +2501,17 @@ ErrorStatus tree_walk_group(Context *c, DeviceTree *t, double G, double eps, dou
     hipLaunchKernelGGL(k_group_runs<true>, pgrid, dim3(256), 0, c->stream, t->nodes, parents,
                        static_cast<int>(num_parents), t->n, t->P, cap, offs, wide, groups);
     GS_HIP(hipGetLastError());
-    const int grid = (static_cast<int>(num_groups) + GW_WAVES - 1) / GW_WAVES;
-    if (order >= 2)
-        hipLaunchKernelGGL((k_walk_group<true, false>), dim3(grid), dim3(GW_BLOCK), 0, c->stream,
-                           t->nodes, t->P, t->sidx, t->n, groups, static_cast<int>(num_groups), args,
-                           a, cnt, t->quadf);
-    else if (args.phi2 > 0.0)
-        hipLaunchKernelGGL((k_walk_group<false, true>), dim3(grid), dim3(GW_BLOCK), 0, c->stream,
-                           t->nodes, t->P, t->sidx, t->n, groups, static_cast<int>(num_groups), args,
-                           a, cnt, t->quadf);
-    else
-        hipLaunchKernelGGL((k_walk_group<false, false>), dim3(grid), dim3(GW_BLOCK), 0, c->stream,
-                           t->nodes, t->P, t->sidx, t->n, groups, static_cast<int>(num_groups), args,
-                           a, cnt, t->quadf);
+    auto walk = [&](auto kernel, int waves) {
+        hipLaunchKernelGGL(kernel, dim3(num_groups), dim3(64 * waves), 0, c->stream, t->nodes, t->P,
+                           t->sidx, t->n, groups, args, a, cnt, t->quadf);
+    };
+    auto pick = [&](auto k1, auto kw) {
+        if (t->n <= 512 * c->cu_count) walk(kw, GW_SPLIT);
+        else walk(k1, 1);
+    };
+    if (order >= 2) pick(k_walk_group<true, false, 1>, k_walk_group<true, false, GW_SPLIT>);
+    else if (args.phi2 > 0.0) pick(k_walk_group<false, true, 1>, k_walk_group<false, true, GW_SPLIT>);
+    else pick(k_walk_group<false, false, 1>, k_walk_group<false, false, GW_SPLIT>);
     timing_end(c, rec);
     GS_HIP(hipGetLastError());
     unsigned long long h[2] = {0, 0};
