@@ -129,34 +129,9 @@ struct GsSim {
     // the other half of the ping-pong of the fused FP64 Leapfrog step; x, xe
     // and v hold the state whenever no step call is running
     double *x2 = nullptr, *xe2 = nullptr, *v2 = nullptr;
-    // captured Leapfrog step (drift, forces, kick) and what it was captured for
-    hipGraphExec_t lf_exec = nullptr;
-    struct Key {
-        int method = -1;
-        double eps = 0.0, dt = 0.0;
-        Fp32Config cfg;
-        void *partial = nullptr;
-        double *x = nullptr;  // the state buffers current when captured
-        bool operator==(const Key &o) const
-        {
-            return method == o.method && eps == o.eps && dt == o.dt && cfg.kind == o.cfg.kind &&
-                   cfg.block == o.cfg.block && cfg.ipt == o.cfg.ipt && cfg.jsplit == o.cfg.jsplit &&
-                   partial == o.partial && x == o.x;
-        }
-    } lf_key;
 };
 
 namespace gs {
-
-// Methods whose force evaluation is a fixed sequence of kernel launches on
-// the stream (no host synchronisation, allocation or memset), so a Leapfrog
-// step can be captured into a HIP graph and replayed.
-static bool graph_method(int method)
-{
-    return method == ACCELERATION_METHOD_PAIRWISE || method == ACCELERATION_METHOD_MASSLESS ||
-           method == ACCELERATION_METHOD_PAIRWISE_FP32 ||
-           method == ACCELERATION_METHOD_MASSLESS_FP32;
-}
 
 // The FP64 direct sums run the whole step as one kernel (drift, forces and
 // kick fused, into the other half of the ping-pong); the other methods as
@@ -183,53 +158,6 @@ static ErrorStatus lf_step(Context *c, GsSim *s, const AccelerationParam *p, dou
     GS_HIP(launch_lf_drift(c, s->x, s->xe, s->v, s->n, dt));
     GS_TRY(device_acceleration(c, s->x, s->m, s->n, s->G, p, s->a));
     GS_HIP(launch_lf_kick(c, s->v, s->ve, s->a, s->n, dt));
-    return make_success_error_status();
-}
-
-// Steps one graph replay performs: two for the fused step (there and back
-// through the ping-pong, starting from and ending at parity 1), one
-// otherwise.
-static int lf_graph_steps(const AccelerationParam *p) { return fused_step_method(p->method) ? 2 : 1; }
-
-// Capture one step into s->lf_exec unless the cached graph was captured for
-// the same parameters and buffers.  Called after an eager step, so every
-// buffer the step needs already exists and nothing allocates while capturing.
-static ErrorStatus lf_graph(Context *c, GsSim *s, const AccelerationParam *p, double dt)
-{
-    GsSim::Key key;
-    key.method = p->method;
-    key.eps = p->softening_length;
-    key.dt = dt;
-    key.cfg = fp32_config();
-    key.partial = c->slots[SLOT_PARTIAL].ptr;
-    key.x = s->x;
-    if (s->lf_exec && key == s->lf_key) return make_success_error_status();
-    int parity = 1;  // a captured fused pair starts after one eager step
-    if (s->lf_exec) {
-        GS_HIP(hipGraphExecDestroy(s->lf_exec));
-        s->lf_exec = nullptr;
-    }
-    GS_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    ErrorStatus st = make_success_error_status();
-    for (int r = 0; r < lf_graph_steps(p) && st.return_code == GRAV_SUCCESS; r++)
-        st = lf_step(c, s, p, dt, parity);
-    hipGraph_t graph = nullptr;
-    const hipError_t e = hipStreamEndCapture(c->stream, &graph);
-    if (st.return_code != GRAV_SUCCESS) {
-        if (graph) (void)hipGraphDestroy(graph);
-        return st;
-    }
-    GS_HIP(e);
-    const hipError_t ei = hipGraphInstantiate(&s->lf_exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    GS_HIP(ei);
-    if (key.partial != c->slots[SLOT_PARTIAL].ptr) {
-        // a buffer moved while capturing: the graph would point at freed memory
-        (void)hipGraphExecDestroy(s->lf_exec);
-        s->lf_exec = nullptr;
-        return WRAP_RAISE_ERROR(GRAV_FAILURE, "Leapfrog graph capture saw a buffer reallocation");
-    }
-    s->lf_key = key;
     return make_success_error_status();
 }
 
@@ -490,7 +418,6 @@ ErrorStatus gs_sim_destroy(GsSim *s)
         std::lock_guard<std::recursive_mutex> lk(c->mu);
         (void)hipStreamSynchronize(c->stream);
     }
-    if (s->lf_exec) (void)hipGraphExecDestroy(s->lf_exec);
     (void)hipFree(s->x);
     (void)hipFree(s->v);
     (void)hipFree(s->m);
@@ -590,19 +517,20 @@ ErrorStatus gs_sim_leapfrog_steps(GsSim *s, const AccelerationParam *p, double d
     Context *c;
     GS_TRY(context(&c));
     std::lock_guard<std::recursive_mutex> lk(c->mu);
-    // with per-kernel timing on, every step runs eagerly so that its kernels
-    // carry their own events
-    const int per = lf_graph_steps(p);
-    const bool graph = k >= 1 + 2 * per && graph_method(p->method) && !c->timing;
-    int64 i = 0;
-    int parity = 0;
-    if (graph) {
-        GS_TRY(lf_step(c, s, p, dt, parity));  // allocates what the step needs
-        i = 1;
-        GS_TRY(lf_graph(c, s, p, dt));
-        for (; i + per <= k; i += per) GS_HIP(hipGraphLaunch(s->lf_exec, c->stream));
+    // A few particles run all the steps in one workgroup (with per-kernel
+    // timing on, the steps' kernels carry their own events instead).  Otherwise
+    // the steps' kernels are launched one by one, at about 4.5 us each, which
+    // is what a step costs up to 128 particles; above, the device is the
+    // slower side.  (A HIP graph of two steps took 18 us to launch: 256 steps
+    // of n = 128 in 2309 us against 1371, of n = 1024 in 3203 against 2576.)
+    if (k > 0 && fused_step_method(p->method) && s->n <= lf_small_max() && !c->timing) {
+        GS_HIP(launch_lf_steps_small(c, s->x, s->xe, s->v, s->ve, s->m, s->n, s->G,
+                                     p->softening_length, p->method == ACCELERATION_METHOD_MASSLESS,
+                                     dt, k, s->a));
+        return make_success_error_status();
     }
-    for (; i < k; i++) GS_TRY(lf_step(c, s, p, dt, parity));
+    int parity = 0;
+    for (int64 i = 0; i < k; i++) GS_TRY(lf_step(c, s, p, dt, parity));
     if (parity) {
         // an odd number of fused steps: the state is in the second half
         const size_t b3 = sizeof(double) * 3 * s->n;

@@ -156,6 +156,13 @@ hipError_t launch_lf_step_f64(Context *c, const double *x, const double *xe, con
                               const double *m, int n, double G, double eps, bool skip_massless,
                               double dt, double *a, double *xo, double *xeo, double *vo, double *ve);
 
+// `steps` such steps of at most lf_small_max() particles in place, in one
+// workgroup.
+int lf_small_max();
+hipError_t launch_lf_steps_small(Context *c, double *x, double *xe, double *v, double *ve,
+                                 const double *m, int n, double G, double eps, bool skip_massless,
+                                 double dt, int64 steps, double *a);
+
 // Leapfrog updates (src/integrator.c:973-1094 op order).
 hipError_t launch_lf_half_kick(Context *c, double *v, double *ve, const double *a, int n,
                                double dt);

@@ -50,8 +50,7 @@ static ErrorStatus leapfrog_gpu(System *system, IntegratorParam *ip, Acceleratio
     status->num_steps = 0;
     // steps 0 .. total-2 end at (i+1) dt <= (total-1) dt < tf, so only the last
     // one can be clamped (src/integrator.c:1001-1006): the others run in
-    // chunks (a replayed HIP graph for the direct-sum methods), checking the
-    // exit flag between chunks.  A chunk ends early at a step that is due for
+    // chunks, checking the exit flag between chunks.  A chunk ends early at a step that is due for
     // a snapshot (t = steps dt >= next output time, src/integrator.c:1045).
     const int64 chunk = 1024;
     while (st.return_code == GRAV_SUCCESS && status->num_steps < total - 1) {

@@ -95,3 +95,18 @@ def test_graph_replayed_steps_equal_eager_steps(method):
         sg.acceleration(p, copy=False)  # eager work on the stream between replays
     sg.close()
     se.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 48, 49, 63, 64, 65])
+@pytest.mark.parametrize("method", [1, 2])
+def test_small_runs_in_one_workgroup_bitwise(n, method):
+    """Runs around the sizes where the one-workgroup steps change, over a chunk boundary (1024 steps), with a clamped
+    last step."""
+    x, v, m = ic.plummer(n, 80 + n) if n > 1 else (np.zeros((1, 3)), np.ones((1, 3)), np.ones(1))
+    if method == 2:
+        m[(n + 1) // 2:] = 0.0
+    dt, tf = 1e-3, 1.0805
+    ids, xg, vg, mg, steps = L.launch_simulation(x, v, m, 1.0, _abi.INTEGRATOR_LEAPFROG, dt, tf, method=method, eps=0.05)
+    xo, vo, so = O.leapfrog(x, v, m, 1.0, dt, tf, eps=0.05, method=method)
+    assert steps == so
+    assert np.array_equal(xg, xo) and np.array_equal(vg, vo)
