@@ -900,8 +900,8 @@ struct F32pPlan {
 // 2^14 workgroups), then 2 and 1 while the chip gets fewer rounds of
 // wavefronts (8 per SIMD) than the tail of the last one can hide in, then
 // parts of a tile down to 16 sources until there are two rounds: a wavefront
-// waits for its scalar loads about 6 times as long as it computes on them, so
-// every SIMD needs its 8, and the sums' folds cost little next to that.
+// alone mostly waits for its scalar loads, so every SIMD needs its 8, and the
+// sums' folds cost little next to that.
 // Evaluations at n = 6007: 49 us with whole tiles in one chunk, 23 here (16
 // and 128 sources a unit: 24 and 27); 12000: 73, 54 (64 and 256: 52 and 61);
 // 24000: 197, 175 (2 tiles: 193); 131072: 4.4 ms either way.
@@ -1208,7 +1208,8 @@ hipError_t launch_copy(Context *c, const void *src, void *dst, size_t bytes)
 // from v_rsq_f64 and two Newton steps (within an ulp; the compiler's sqrt and
 // division where r^2 is out of range, coincident particles among them).
 // Bound by FP64 issue.  One MI355X, before (one thread per particle over all
-// later ones) and now: 1024 particles 0.19 ms -> 0.02, 20000 3.2 -> 0.2 ms.
+// later ones) and now: the whole call for 1024 particles 215 -> 39 us, 20000
+// 3.2 -> 0.35 ms.
 constexpr int EN_K = 4;
 
 __global__ __launch_bounds__(64) void k_energy(const double *__restrict__ x,
@@ -1272,11 +1273,13 @@ __global__ __launch_bounds__(64) void k_energy(const double *__restrict__ x,
     if (lane == 0) partials[blockIdx.y * nb + bi] = e;
 }
 
-// Wavefronts: enough chunks of offsets for 8 per CU where there are that many offsets.
+// Wavefronts: chunks of offsets up to 8 per CU where there are that many
+// offsets, so that the partial sums stay within 16 KiB up to 131072 particles:
+// a process's first larger copy to the host takes the runtime about 6 ms.
 static dim3 energy_grid(int n, int cu_count, int *offsets)
 {
     const int nb = (n + 63) / 64, all = nb / 2 + 1;
-    int chunks = (8 * cu_count + nb - 1) / nb;
+    int chunks = std::max(1, 8 * cu_count / nb);
     if (chunks > all) chunks = all;
     *offsets = (all + chunks - 1) / chunks;
     return dim3(nb, (all + *offsets - 1) / *offsets);
