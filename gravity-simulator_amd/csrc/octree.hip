@@ -15,7 +15,7 @@
 //                  search on the sorted keys, counted, scanned, emitted)
 //   multipoles     bottom-up per level; leaves sum their particles in sorted
 //                  order, internal nodes sum their children (FP64)
-//   k_walk         one wavefront walks for 4 to 16 Morton-consecutive targets
+//   k_walk         one wavefront walks for 4 to 32 Morton-consecutive targets
 //                  with a shared explicit stack of (node, target mask), up to
 //                  64 entries a pass: each target applies the reference
 //                  opening test itself; those that accept a node add its
@@ -1088,9 +1088,9 @@ __device__ __forceinline__ void oct_term(const float *__restrict__ T, double R0,
 // order of the FP64 sums differs.
 //
 // Bound by VALU issue (16 FP64 instructions of 4.75 cycles per G entries of
-// a pass) once the chip is full.  The walk it replaced visited one node at a
-// time through scalar loads, a latency of 600 to 800 cycles each; what each G
-// measured stands at the choice in tree_walk.
+// a pass) once the chip is full.  k_walk_single visits one node at a time
+// through scalar loads, each waiting for the last one's; what they measured
+// stands at the choice in tree_walk.
 //
 // QUAD: add the quadrupole term of accepted nodes.  FEAT: do not add it but
 // accumulate per-target features of the walk for the learned correction,
@@ -1351,6 +1351,193 @@ __global__ __launch_bounds__(64) void k_walk(const NodeRec *__restrict__ nodes,
     // interaction count: one atomic per wave (an overflow, which the batch
     // limit excludes, is flagged through it)
     if (lane == 0 && n_int) atomicAdd(n_int, wcnt + (overflow ? 1ull << 62 : 0ull));
+}
+
+// The same walk by single nodes: 64 targets, one per lane, a node at a time,
+// its record through scalar loads.  Every visit waits for its record, but
+// serves 64 targets; what each measured stands at the choice in tree_walk.
+constexpr int WS_BLOCK = 256;
+constexpr int WS_WAVES = WS_BLOCK / 64;
+constexpr int WS_STACK = 192;  // >= 7 pending siblings x 21 levels + 8
+
+template <bool QUAD, bool FEAT>
+__global__ __launch_bounds__(WS_BLOCK) void k_walk_single(const NodeRec *__restrict__ nodes,
+                                                          const double4 *__restrict__ P,
+                                                          const long long *__restrict__ skeys,
+                                                          const int *__restrict__ sidx, int n,
+                                                          WalkArgs args, double *__restrict__ a,
+                                                          unsigned long long *__restrict__ n_int,
+                                                          const float *__restrict__ quad,
+                                                          const float *__restrict__ oct,
+                                                          float *__restrict__ feat)
+{
+    __shared__ int stk_node[WS_WAVES][WS_STACK];
+    __shared__ unsigned long long stk_mask[WS_WAVES][WS_STACK];
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int s = (blockIdx.x * WS_WAVES + wave) * 64 + lane;
+    const bool valid = s < n;
+    const unsigned long long all = __ballot(valid);
+    if (all == 0) return;
+
+    double xi0 = 0.0, xi1 = 0.0, xi2 = 0.0;
+    long long key = 0;
+    if (valid) {
+        const double4 p = P[s];
+        xi0 = p.x;
+        xi1 = p.y;
+        xi2 = p.z;
+        key = skeys[s];
+    }
+    double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+    unsigned cnt = 0;             // per-lane interactions of the rare opened-leaf path
+    unsigned long long wcnt = 0;  // the wavefront's other interactions (uniform)
+    float fq0 = 0.0f, fq1 = 0.0f, fq2 = 0.0f, fs2 = 0.0f, fs3 = 0.0f;
+    float fv0 = 0.0f, fv1 = 0.0f, fv2 = 0.0f;
+    float fo0 = 0.0f, fo1 = 0.0f, fo2 = 0.0f;
+    unsigned nacc = 0, npp = 0;
+    int *snode = stk_node[wave];
+    unsigned long long *smask = stk_mask[wave];
+
+    int sp = 0;
+    {
+        const int c0 = nodes[0].child0, nc = nodes[0].nchild;
+        for (int c = nc - 1; c >= 0; c--) {
+            if (lane == 0) {
+                snode[sp] = c0 + c;
+                smask[sp] = all;
+            }
+            sp++;
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    while (sp > 0) {
+        sp--;
+        const int node = __builtin_amdgcn_readfirstlane(snode[sp]);
+        const unsigned long long M =
+            (static_cast<unsigned long long>(__builtin_amdgcn_readfirstlane(
+                 static_cast<int>(smask[sp] >> 32)))
+             << 32) |
+            static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(smask[sp])));
+        __builtin_amdgcn_wave_barrier();
+        const NodeRec nd = nodes[node];
+        // (M is uniform: the lane's bit as a per-lane predicate, no VALU work)
+        const bool act = __builtin_amdgcn_inverse_ballot_w64(M);
+        unsigned long long O = 0;  // lanes that open this node
+        // The VALU executes an instruction for the whole wavefront whatever
+        // its lane mask, so the terms are formed branch-free for every lane
+        // and lanes that do not take them add an exact zero (the running sums
+        // start at +0 and a sum of products that cancels is +0, never -0, so
+        // adding fma(-0, R, a) = a leaves every bit unchanged).
+        if (nd.nchild == 0 && nd.count == 1) {
+            // single-particle leaf: its monopole is the particle itself
+            const bool use = act && nd.first != s;
+            wcnt += static_cast<unsigned>(__popcll(__ballot(use)));
+            {
+                const double4 p = P[nd.first];
+                const double R0 = xi0 - p.x, R1 = xi1 - p.y, R2 = xi2 - p.z;
+                const double r2 = R0 * R0 + R1 * R1 + R2 * R2 + args.eps2;
+                const float ri = __builtin_amdgcn_rsqf(static_cast<float>(r2));
+                const float mr3 = static_cast<float>(p.w) * (ri * ri * ri);
+                const double w = static_cast<double>(use ? mr3 : 0.0f);
+                a0 = __builtin_fma(-w, R0, a0);
+                a1 = __builtin_fma(-w, R1, a1);
+                a2 = __builtin_fma(-w, R2, a2);
+                if (FEAT) npp += use ? 1u : 0u;
+            }
+            continue;
+        }
+        const bool included = (key >> (3 * (MAXL - nd.depth))) == nd.prefix;
+        const double R0 = xi0 - nd.cx, R1 = xi1 - nd.cy, R2 = xi2 - nd.cz;
+        const double d2 = R0 * R0 + R1 * R1 + R2 * R2;
+        const double l2 = nd.l2;
+        const bool accept = act && !included && l2 < args.theta2 * d2;
+        const unsigned long long AM = __ballot(accept);
+        wcnt += static_cast<unsigned>(__popcll(AM));
+        O = M & ~AM;  // act && !accept
+        // (no branch around the terms: a visit where no lane accepts is rare
+        // enough that computing them anyway is cheaper than merging the sums)
+        {
+            const float ri = __builtin_amdgcn_rsqf(static_cast<float>(d2 + args.eps2));
+            const float mr3 = nd.fmass * (ri * ri * ri);
+            const double w = static_cast<double>(accept ? mr3 : 0.0f);
+            a0 = __builtin_fma(-w, R0, a0);
+            a1 = __builtin_fma(-w, R1, a1);
+            a2 = __builtin_fma(-w, R2, a2);
+            if (QUAD || FEAT) {
+                float o0, o1, o2;
+                quad_term(quad + 8 * static_cast<size_t>(node), R0, R1, R2, ri, o0, o1, o2);
+                if (QUAD) {
+                    a0 += static_cast<double>(accept ? o0 : 0.0f);
+                    a1 += static_cast<double>(accept ? o1 : 0.0f);
+                    a2 += static_cast<double>(accept ? o2 : 0.0f);
+                } else {
+                    // M l^2 / d^4 and M l^3 / d^5 (l: cell side, d: distance to the COM)
+                    const float lr = static_cast<float>(__builtin_sqrt(l2)) * ri;
+                    const float mr2 = mr3 * static_cast<float>(__builtin_sqrt(d2 + args.eps2));
+                    const float lr3 = lr * lr * lr;
+                    const float k3 = mr3 * lr3;
+                    float t0, t1, t2;
+                    oct_term(oct + 12 * static_cast<size_t>(node), R0, R1, R2, ri, t0, t1, t2);
+                    if (accept) {
+                        fq0 += o0;
+                        fq1 += o1;
+                        fq2 += o2;
+                        fo0 += t0;
+                        fo1 += t1;
+                        fo2 += t2;
+                        fs2 = __builtin_fmaf(mr2, lr * lr, fs2);
+                        fs3 = __builtin_fmaf(mr2, lr3, fs3);
+                        fv0 = __builtin_fmaf(k3, static_cast<float>(R0), fv0);
+                        fv1 = __builtin_fmaf(k3, static_cast<float>(R1), fv1);
+                        fv2 = __builtin_fmaf(k3, static_cast<float>(R2), fv2);
+                        nacc++;
+                    }
+                }
+            }
+        }
+        if (O == 0) continue;
+        if (nd.nchild == 0) {
+            const bool mine = __builtin_amdgcn_inverse_ballot_w64(O);
+            for (int t = nd.first; t < nd.first + nd.count; t++) {
+                const double4 p = P[t];
+                if (mine && t != s) {
+                    pp_force(xi0, xi1, xi2, p.x, p.y, p.z, p.w, args.eps2, a0, a1, a2);
+                    cnt++;
+                    npp++;
+                }
+            }
+        } else if (sp + nd.nchild <= WS_STACK) {
+            // children pushed last-to-first (child0 on top), one lane each
+            if (lane < nd.nchild) {
+                snode[sp + lane] = nd.child0 + nd.nchild - 1 - lane;
+                smask[sp + lane] = O;
+            }
+            sp += nd.nchild;
+            __builtin_amdgcn_wave_barrier();
+        } else if (lane == 0 && n_int) {
+            // cannot happen for depth <= 21 (at most 7 pending siblings per
+            // level); flagged through the counter instead of overflowing
+            atomicAdd(n_int, 1ull << 62);
+        }
+    }
+    if (valid) {
+        const int i = sidx[s];
+        a[3 * i + 0] = args.G * a0;
+        a[3 * i + 1] = args.G * a1;
+        a[3 * i + 2] = args.G * a2;
+        if (FEAT) {
+            float4 *f = reinterpret_cast<float4 *>(feat + 16 * static_cast<size_t>(i));
+            f[0] = make_float4(fq0, fq1, fq2, fv0);
+            f[1] = make_float4(fv1, fv2, fs2, fs3);
+            f[2] = make_float4(static_cast<float>(nacc), static_cast<float>(npp), fo0, fo1);
+            f[3] = make_float4(fo2, 0.0f, 0.0f, 0.0f);
+        }
+    }
+    // interaction count: one atomic per wave
+    unsigned long long tot = cnt;
+    for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off);
+    if (lane == 0 && n_int) atomicAdd(n_int, tot + wcnt);
 }
 
 // ------------------------------------------------------------------ group walk
@@ -2402,22 +2589,50 @@ ErrorStatus tree_walk(Context *c, DeviceTree *t, const double *x, double G, doub
         hipLaunchKernelGGL(kernel, dim3((t->n + targets - 1) / targets), dim3(64), 0, c->stream,
                            t->nodes, t->P, t->sidx, t->n, args, a, cnt, t->quadf, t->octf, feat);
     };
+    auto single = [&](auto kernel) {
+        const int waves = (t->n + 63) / 64;
+        hipLaunchKernelGGL(kernel, dim3((waves + WS_WAVES - 1) / WS_WAVES), dim3(WS_BLOCK), 0,
+                           c->stream, t->nodes, t->P, t->skeys, t->sidx, t->n, args, a, cnt, t->quadf,
+                           t->octf, feat);
+    };
     // Entries per pass step.  More entries, fewer targets per wavefront: more
     // wavefronts and fewer nodes that only some of the targets visit, but
-    // more passes per target.  Monopole walk, theta 0.5, us for G = 1 / 2 / 4
-    // / 8 / 16 (and the walk by single nodes before): n = 10000: 475 / 239 /
-    // 141 / 94 / 76 (1022); 60000: 799 / 441 / 286 / 279 / 350 (1721); 262144:
-    // 1818 / 1161 / 1078 / 1191 / 1571 (2636); 2097152: 13014 / 8750 / 8848 /
-    // 10251 / 13868 (12623).  With quadrupoles at 2097152: 20.3 / 15.7 / 15.5
-    // / 16.8 / 21.0 ms (18.1).
-    auto pick = [&](auto k4, auto k8, auto k16) {
+    // more passes per target.  Monopole walk, theta 0.5, us for G = 2 / 4 / 8
+    // / 16 (and by single nodes): n = 10000: 239 / 141 / 94 / 76 (1022);
+    // 60000: 441 / 286 / 279 / 350 (1721); 262144: 1161 / 1078 / 1191 / 1571
+    // (2636); 2097152: 8750 / 8848 / 10251 / 13868 (12623).
+    //
+    // The smaller the angle, the more of the visits neighbours share: past
+    // 1024 particles per CU two entries are the better choice below theta 0.5
+    // (2^21, G = 2 / 4, ms: theta 0.4 14.4 / 15.3, 0.3 38.3 / 47.2), and below
+    // an angle that grows with n and with the work of an accepted node the
+    // walk by single nodes.  Single / G = 2, ms, monopoles: 2^19, theta 0.15:
+    // 48.7 / 45.3; 2^20, 0.2: 54.7 / 57.8, 0.25: 33.0 / 30.5; 2^21, 0.25: 61.9
+    // / 73.5, 0.3: 39.4 / 38.3; 2^22, 0.3: 78.3 / 84.9, 0.35: 54.4 / 47.4.
+    // Quadrupoles: 2^19, 0.2: 38.6 / 39.3; 2^20, 0.25: 47.1 / 51.6, 0.3: 30.4
+    // / 28.8; 2^21, 0.3: 57.0 / 66.2, 0.35: 39.8 / 39.7; 2^22, 0.35: 78.8 /
+    // 83.5, 0.4: 55.3 / 53.9.  Features: 2^20, 0.3: 60.5 / 61.4, 0.35: 43.0 /
+    // 41.0; 2^21, 0.35: 81.1 / 87.5, 0.4: 57.0 / 59.4, 0.55: 29.9 / 29.5.  At
+    // 2^18 and theta 0.1, 58.9 / 32.6 and with quadrupoles 72.6 / 51.3.
+    const bool many = t->n > 1024 * c->cu_count;
+    const double theta_single =
+        0.40 - 175.0 / std::sqrt(static_cast<double>(t->n)) + (feat ? 0.12 : order >= 2 ? 0.06 : 0.0);
+    auto pick = [&](auto k1, auto k2, auto k4, auto k8, auto k16) {
         if (t->n <= 64 * c->cu_count) walk(k16, 16);
         else if (t->n <= 512 * c->cu_count) walk(k8, 8);
+        else if (many && theta < theta_single) single(k1);
+        else if (many && theta < 0.5) walk(k2, 2);
         else walk(k4, 4);
     };
-    if (feat) pick(k_walk<4, false, true>, k_walk<8, false, true>, k_walk<16, false, true>);
-    else if (order >= 2) pick(k_walk<4, true, false>, k_walk<8, true, false>, k_walk<16, true, false>);
-    else pick(k_walk<4, false, false>, k_walk<8, false, false>, k_walk<16, false, false>);
+    if (feat)
+        pick(k_walk_single<false, true>, k_walk<2, false, true>, k_walk<4, false, true>,
+             k_walk<8, false, true>, k_walk<16, false, true>);
+    else if (order >= 2)
+        pick(k_walk_single<true, false>, k_walk<2, true, false>, k_walk<4, true, false>,
+             k_walk<8, true, false>, k_walk<16, true, false>);
+    else
+        pick(k_walk_single<false, false>, k_walk<2, false, false>, k_walk<4, false, false>,
+             k_walk<8, false, false>, k_walk<16, false, false>);
     timing_end(c, rec);
     GS_HIP(hipGetLastError());
     if (interactions) {

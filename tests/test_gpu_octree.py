@@ -446,6 +446,35 @@ def test_walk_forms_against_the_oracle(n, leaf):
         assert np.median(e) < 1e-6 and e.max() < 1e-4
 
 
+@pytest.mark.parametrize("theta", [0.49, 0.5])
+def test_walk_of_many_particles_against_the_oracle(theta):
+    """Past 262144 particles on 256 CUs, either side of theta 0.5 (32 and 16 targets per wavefront)."""
+    n = 262146
+    x, v, m = ic.two_spheres(n, 31)
+    t = O.build_tree(x, m, 1)
+    a = L.acceleration(x, m, 3, eps=1e-2, theta=theta, leaf=1)
+    ao, cnt = O.bh_walk(x, m, t, theta, eps=1e-2, want_counts=True)
+    assert L.last_walk_interactions() == int(cnt.sum())
+    e = np.linalg.norm(a - ao, axis=1) / np.linalg.norm(ao, axis=1)
+    assert np.median(e) < 1e-6 and e.max() < 1e-4
+
+
+@pytest.mark.parametrize("method,shift", [(3, 0.0), (19, 0.06)])
+@pytest.mark.parametrize("n,leaf", [(400002, 1), (262146, 8)])
+def test_walk_by_single_nodes_equals_the_walk_by_passes(method, shift, n, leaf):
+    """The angle at which the walk changes form, less and plus 1e-12 of it: the same interactions (no l^2 / d^2 lies
+    that close to theta^2), forces equal to FP32 rounding of the terms, as against the oracle above."""
+    x, v, m = ic.two_spheres(n, 33)
+    th = 0.40 - 175.0 / np.sqrt(n) + shift
+    out = []
+    for s in (-1e-12, 1e-12):
+        a = L.acceleration(x, m, method, eps=1e-2, theta=th * (1 + s), leaf=leaf)
+        out.append((a, L.last_walk_interactions()))
+    assert out[0][1] == out[1][1]
+    e = np.linalg.norm(out[0][0] - out[1][0], axis=1) / np.linalg.norm(out[1][0], axis=1)
+    assert np.median(e) < 1e-6 and e.max() < 1e-4
+
+
 @pytest.mark.parametrize("n", [2, 66, 700, 131072, 131074])
 def test_group_walk_forms_against_the_oracle(n):
     """Several wavefronts per group (up to 131072 particles on 256 CUs) and one: equal interaction counts and forces to
