@@ -5,8 +5,9 @@
 // ends of the range (scale, class and fix-up instructions; the division's go
 // through the one VCC register, which keeps independent divisions of a lane
 // from overlapping).  Inside the range the remaining steps give the same
-// correctly rounded results on their own.  Measured issue cost per wave64 on
-// MI355X: sqrt 86 cycles and division 61, against 59 and 38 here.
+// correctly rounded results on their own.  Issue cost per wave64 on MI355X:
+// the compiler's sqrt 86 cycles and division 61 (measured), these about 59
+// and 38 by their instructions at the measured rates.
 #pragma once
 
 #include <hip/hip_runtime.h>
