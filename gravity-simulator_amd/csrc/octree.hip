@@ -1562,13 +1562,16 @@ __global__ __launch_bounds__(WS_BLOCK) void k_walk_single(const NodeRec *__restr
 // workgroup: 6.0 ms against 6.7 with two and 8.2 with four groups (2048
 // entries).
 // Few groups do not fill the chip and the one with the longest list sets the
-// time, so for n <= 512 particles per CU GW_SPLIT wavefronts share a group:
+// time, so for n <= 256 particles per CU GW_SPLIT wavefronts share a group:
 // they take the first passes alike (wavefront 0 collecting the terms) until
 // the stack holds GW_SHARE entries per wavefront, then every GW_SPLIT-th
 // entry each, and their sums are added at the end.  Walk at theta 0.5, one /
 // four / eight / sixteen wavefronts: n = 10000: 363 / 280 / 239 / 382 us,
 // 60000: 2216 / 1335 / 832 / 981, 120000: 900 / - / 655 / 1886, 160000: 517 /
-// - / 856 / -, 262144: 991 / 988 / 1337 / 3636.
+// - / 856 / -, 262144: 991 / 988 / 1337 / 3636.  At 120000 the sharing loses
+// for smaller angles and quadrupoles (before it / with eight: theta 0.2 3373 /
+// 3922 us, quadrupoles at 0.35 2431 / 2989, at 0.2 5092 / 7472); at 60000 it
+// gains for all (quadrupoles at 0.35 4539 / 1075, at 0.2 5744 / 2871).
 constexpr int GW_SPLIT = 8;
 constexpr int GW_SHARE = 32;
 constexpr int GW_STACK = 1024;
@@ -2721,7 +2724,7 @@ ErrorStatus tree_walk_group(Context *c, DeviceTree *t, double G, double eps, dou
                            t->sidx, t->n, groups, args, a, cnt, t->quadf);
     };
     auto pick = [&](auto k1, auto kw) {
-        if (t->n <= 512 * c->cu_count) walk(kw, GW_SPLIT);
+        if (t->n <= 256 * c->cu_count) walk(kw, GW_SPLIT);
         else walk(k1, 1);
     };
     if (order >= 2) pick(k_walk_group<true, false, 1>, k_walk_group<true, false, GW_SPLIT>);
