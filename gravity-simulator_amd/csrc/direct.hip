@@ -1071,8 +1071,9 @@ hipError_t launch_direct_f32(Context *c, const double *x, const double *m, int n
 // FP32 direct sum for a list of targets against all n sources (the learned
 // correction's labels and spot check).  The shared-target kernel of
 // launch_direct_f32 (kind 2, 16 wavefronts per 64 targets): the targets'
-// positions are gathered into a compact array and the sources divided by the
-// same rule, so that even a few hundred targets fill the chip.
+// positions are gathered into a compact array and the sources divided into
+// `split` chunks of whole tiles or, for split = 0, by f32p_plan's rule, so
+// that even a few hundred targets fill the chip.
 __global__ void k_gather_targets(const double *__restrict__ x, const int *__restrict__ idx,
                                  int nt, double *__restrict__ xt)
 {
@@ -1091,24 +1092,36 @@ hipError_t launch_gather_rows3(Context *c, const double *src, const int *idx, in
 
 constexpr int TARGET_WAVES = 16;  // wavefronts per 64 targets in launch_direct_f32_targets
 
-size_t direct_f32_targets_bytes(Context *c, int n, int nt)
+// Training turns the last bits of its labels into 1e-4 of the weights (bf16
+// products, tens of dependent optimiser steps), so the labels' sums keep this
+// one division, whatever f32p_plan finds faster: a sample trains the same
+// weights on any card.  Chunks of at least one tile per wavefront, about 1024
+// workgroups in all (131072 labels: 5.3 ms, by f32p_plan's rule 5.2).
+int direct_f32_label_split(int n, int nt)
+{
+    const int wgs = (nt + 63) / 64;
+    const int split = std::min((1024 + wgs - 1) / wgs, f32s_tiles(n) / TARGET_WAVES);
+    return std::max(split, 1);
+}
+
+size_t direct_f32_targets_bytes(Context *c, int n, int nt, int split)
 {
     const size_t nt3 = 3 * static_cast<size_t>(nt);
     const size_t nt_tiles = f32s_tiles(n);
-    const F32pPlan p = f32p_plan(n, nt, TARGET_WAVES, 0, c->cu_count);
+    const F32pPlan p = f32p_plan(n, nt, TARGET_WAVES, split, c->cu_count);
     return 512 + nt3 * sizeof(double) * (1 + p.chunks) + nt_tiles * ST_TILE * sizeof(float4) +
            nt_tiles * sizeof(double4);
 }
 
 hipError_t launch_direct_f32_targets(Context *c, const double *x, const double *m, int n, double G,
-                                     double eps, const int *targets, int nt, double *out,
+                                     double eps, const int *targets, int nt, int split, double *out,
                                      void *buf, size_t bytes)
 {
     if (nt <= 0) return hipSuccess;
-    if (bytes < direct_f32_targets_bytes(c, n, nt)) return hipErrorInvalidValue;
+    if (bytes < direct_f32_targets_bytes(c, n, nt, split)) return hipErrorInvalidValue;
     const int ntiles = f32s_tiles(n);
     const int n_pad = ntiles * ST_TILE;
-    const F32pPlan plan = f32p_plan(n, nt, TARGET_WAVES, 0, c->cu_count);
+    const F32pPlan plan = f32p_plan(n, nt, TARGET_WAVES, split, c->cu_count);
     const int nsplit = plan.chunks;
     const size_t nt3 = 3 * static_cast<size_t>(nt);
     auto align = [](char *p) {

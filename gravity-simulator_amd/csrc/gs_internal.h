@@ -120,11 +120,14 @@ hipError_t launch_direct_f32(Context *c, const double *x, const double *m, int n
                              double eps, double *a, void *partial_buf, size_t partial_bytes,
                              const Fp32Config &cfg);
 size_t direct_f32_partial_bytes(int n, const Fp32Config &cfg, int cu_count);
-// Same arithmetic for the listed targets only: out[t] = a(targets[t]).
+// Same arithmetic for the listed targets only: out[t] = a(targets[t]).  split:
+// source chunks (0: chosen for speed; direct_f32_label_split: the training
+// labels', which no choice made for speed changes).
 hipError_t launch_direct_f32_targets(Context *c, const double *x, const double *m, int n, double G,
-                                     double eps, const int *targets, int nt, double *out,
+                                     double eps, const int *targets, int nt, int split, double *out,
                                      void *buf, size_t bytes);
-size_t direct_f32_targets_bytes(Context *c, int n, int nt);
+size_t direct_f32_targets_bytes(Context *c, int n, int nt, int split);
+int direct_f32_label_split(int n, int nt);
 // out[t] = src[idx[t]] for rows of 3 doubles.
 hipError_t launch_gather_rows3(Context *c, const double *src, const int *idx, int nt, double *out);
 // FP32 issue-rate probe: kind 0 v_fmac_f32, 1 v_mul_f32, 2 v_rsq_f32 chains,
@@ -182,10 +185,11 @@ ErrorStatus tree_build(Context *c, const double *x, const double *m, int n, int 
 // Walk; writes a (device, AoS, original order).  order 1: monopoles (the
 // reference's), 2: with quadrupole terms.  feat != NULL: monopole walk that
 // also writes 16 FP32 features per particle for the learned correction (the
-// tree built with second and third moments).
+// tree built with second and third moments).  by_nodes: the walk by single
+// nodes whatever the size, so that a particle's sums keep one order.
 ErrorStatus tree_walk(Context *c, DeviceTree *t, const double *x, double G, double eps,
                       double theta, double *a, long long *interactions, int order = 1,
-                      float *feat = nullptr);
+                      float *feat = nullptr, bool by_nodes = false);
 // Group walk (one wavefront per 64 sorted particles, group opening test);
 // order 1: monopoles, 2: with quadrupole terms (tree built with_quad).
 // phi > 0 (monopole walk only): nodes with rg < phi |com - c| (rg the

@@ -38,7 +38,7 @@ static ErrorStatus spot_check(Context *c, const double *x, const double *m, int 
                               double eps, const double *a, int ns, double *p99)
 {
     const std::vector<int> tg = strided_targets(n, ns);
-    const size_t need_bytes = direct_f32_targets_bytes(c, n, ns);
+    const size_t need_bytes = direct_f32_targets_bytes(c, n, ns, 0);
     void *buf, *sp;
     GS_TRY(slot(c, SLOT_PARTIAL, need_bytes, &buf));
     const size_t off = ((sizeof(int) * ns + 255) / 256) * 256;
@@ -48,7 +48,7 @@ static ErrorStatus spot_check(Context *c, const double *x, const double *m, int 
     double *dg = dr + 3 * static_cast<size_t>(ns);
     GS_HIP(hipMemcpyAsync(dt, tg.data(), sizeof(int) * ns, hipMemcpyHostToDevice, c->stream));
     const int rec = timing_begin(c, "spot_check");
-    GS_HIP(launch_direct_f32_targets(c, x, m, n, G, eps, dt, ns, dr, buf, need_bytes));
+    GS_HIP(launch_direct_f32_targets(c, x, m, n, G, eps, dt, ns, 0, dr, buf, need_bytes));
     timing_end(c, rec);
     GS_HIP(launch_gather_rows3(c, a, dt, ns, dg));
     // reference and gathered result: one copy
@@ -73,9 +73,11 @@ static ErrorStatus spot_check(Context *c, const double *x, const double *m, int 
 }
 
 // Coarse walk with features: a (device), raw or normalised features into F.
+// by_nodes: see tree_walk.
 static ErrorStatus coarse_walk(Context *c, const double *x, const double *m, int n, double G,
                                double eps, double theta, int leaf, double *a, bool normalise,
-                               float **F_out, DeviceTree **t_out, float **wf_out = nullptr)
+                               float **F_out, DeviceTree **t_out, float **wf_out = nullptr,
+                               bool by_nodes = false)
 {
     DeviceTree *t;
     GS_TRY(tree_build(c, x, m, n, leaf, nullptr, -1.0, true, &t, true));
@@ -83,7 +85,7 @@ static ErrorStatus coarse_walk(Context *c, const double *x, const double *m, int
     GS_TRY(slot(c, SLOT_FEAT, sizeof(float) * MLP_WALK_FEAT * static_cast<size_t>(n), &wf));
     GS_TRY(slot(c, SLOT_MLP_X, sizeof(float) * MLP_F * static_cast<size_t>(n), &F));
     GS_TRY(tree_walk(c, t, x, G, eps, theta, a, &g_learned_interactions, 1,
-                     static_cast<float *>(wf)));
+                     static_cast<float *>(wf), by_nodes));
     const int rec = timing_begin(c, "learned_features");
     GS_TRY(mlp_features(c, a, static_cast<float *>(wf), n, G, normalise, static_cast<float *>(F)));
     timing_end(c, rec);
@@ -258,7 +260,10 @@ static ErrorStatus build_samples(Context *c, const System *system, double eps, d
     double *x, *m, *a;
     GS_TRY(upload_xm(c, system, &x, &m, &a));
     float *F, *wf;
-    GS_TRY(coarse_walk(c, x, m, n, G, eps, theta, leaf_or_default(leaf), a, false, &F, nullptr, &wf));
+    // (the walk's sums in the one order of the walk by single nodes: like the
+    // labels', their last bits show in the weights)
+    GS_TRY(coarse_walk(c, x, m, n, G, eps, theta, leaf_or_default(leaf), a, false, &F, nullptr, &wf,
+                       true));
     std::vector<int> perm(n);
     for (int i = 0; i < n; i++) perm[i] = i;
     unsigned long long st = 0x853C49E6748FEA9Bull ^ (static_cast<unsigned long long>(seed) << 1);
@@ -270,7 +275,8 @@ static ErrorStatus build_samples(Context *c, const System *system, double eps, d
     S.idx.assign(perm.begin(), perm.begin() + ns);
     // labels from the FP32 split-precision direct sum
     void *sp, *buf;
-    const size_t lb = direct_f32_targets_bytes(c, n, ns);
+    const int split = direct_f32_label_split(n, ns);
+    const size_t lb = direct_f32_targets_bytes(c, n, ns, split);
     GS_TRY(slot(c, SLOT_PARTIAL, lb, &buf));
     auto up = [](size_t b) { return ((b + 255) / 256) * 256; };
     const size_t off_ref = up(sizeof(int) * ns);
@@ -284,7 +290,7 @@ static ErrorStatus build_samples(Context *c, const System *system, double eps, d
     float *dwf = reinterpret_cast<float *>(static_cast<char *>(sp) + off_wf);
     double *dac = reinterpret_cast<double *>(static_cast<char *>(sp) + off_ac);
     GS_HIP(hipMemcpyAsync(didx, S.idx.data(), sizeof(int) * ns, hipMemcpyHostToDevice, c->stream));
-    GS_HIP(launch_direct_f32_targets(c, x, m, n, G, eps, didx, ns, dref, buf, lb));
+    GS_HIP(launch_direct_f32_targets(c, x, m, n, G, eps, didx, ns, split, dref, buf, lb));
     GS_HIP(mlp_gather_rows(c, F, didx, ns, MLP_F, dfs));
     GS_HIP(mlp_gather_rows(c, wf, didx, ns, MLP_WALK_FEAT, dwf));
     GS_HIP(launch_gather_rows3(c, a, didx, ns, dac));

@@ -2568,7 +2568,8 @@ ErrorStatus tree_build(Context *c, const double *x, const double *m, int n, int 
 }
 
 ErrorStatus tree_walk(Context *c, DeviceTree *t, const double *x, double G, double eps,
-                      double theta, double *a, long long *interactions, int order, float *feat)
+                      double theta, double *a, long long *interactions, int order, float *feat,
+                      bool by_nodes)
 {
     (void)x;
     if ((order == 2 || feat) && !t->has_quad)
@@ -2621,7 +2622,8 @@ ErrorStatus tree_walk(Context *c, DeviceTree *t, const double *x, double G, doub
     const double theta_single =
         0.40 - 175.0 / std::sqrt(static_cast<double>(t->n)) + (feat ? 0.12 : order >= 2 ? 0.06 : 0.0);
     auto pick = [&](auto k1, auto k2, auto k4, auto k8, auto k16) {
-        if (t->n <= 64 * c->cu_count) walk(k16, 16);
+        if (by_nodes) single(k1);
+        else if (t->n <= 64 * c->cu_count) walk(k16, 16);
         else if (t->n <= 512 * c->cu_count) walk(k8, 8);
         else if (many && theta < theta_single) single(k1);
         else if (many && theta < 0.5) walk(k2, 2);
