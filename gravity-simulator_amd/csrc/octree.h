@@ -54,7 +54,8 @@ struct DeviceTree {
 
 // Stable LSD radix sort of n (key, index) pairs on the low 8 * passes bits of
 // the (non-negative) keys, alternating between (k0, i0) and (k1, i1); the
-// sorted pairs end in (*ko, *io).  hist holds radix_hist_elements(n) counters.
+// sorted pairs end in (*ko, *io).  hist holds radix_hist_elements(n) counters,
+// which serve any smaller n as well (never fewer for more keys).
 size_t radix_hist_elements(int n);
 ErrorStatus radix_sort_pairs(Context *c, long long *k0, int *i0, long long *k1, int *i1, int n,
                              int passes, unsigned *hist, long long **ko, int **io);

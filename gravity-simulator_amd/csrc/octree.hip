@@ -21,6 +21,7 @@
 //                  opening test itself; those that accept a node add its
 //                  monopole, the others descend.  Geometry and sums in FP64, 1/r^3 through FP32
 //                  rsqrt.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <utility>
@@ -2279,13 +2280,21 @@ static ErrorStatus ensure_nodes(Context *c, DeviceTree *t, int need)
 // ranked one after the other and the CUs have room for more tiles.  Sort of
 // n = 60000 with 2 / 4 / 8 keys: 95 / 106 / 138 us; 262144: 124 / 124 / 150;
 // 524288: 170 / 151 / 164; 1048576: 269 / 214 / 201.
-static int rs_rounds(int n) { return n <= 262144 ? 2 : n <= 786432 ? 4 : RS_MAX_ROUNDS; }
+constexpr int RS_FEW = 262144, RS_MIDDLE = 786432;
+static int rs_rounds(int n) { return n <= RS_FEW ? 2 : n <= RS_MIDDLE ? 4 : RS_MAX_ROUNDS; }
 
+// The tile counts and digit totals of a sort of n keys or fewer: where the
+// tiles grow, a sort of just fewer keys needs more counts than one of n.
 size_t radix_hist_elements(int n)
 {
-    // the tile counts, then the digit totals
-    const int tile = RS_BLOCK * rs_rounds(n);
-    return static_cast<size_t>((n + tile - 1) / tile) * RS_BINS + RS_BINS;
+    auto need = [](int k) {
+        const int tile = RS_BLOCK * rs_rounds(k);
+        return static_cast<size_t>((k + tile - 1) / tile) * RS_BINS + RS_BINS;
+    };
+    size_t most = need(n);
+    for (int edge : {RS_FEW, RS_MIDDLE})
+        if (n > edge) most = std::max(most, need(edge));
+    return most;
 }
 
 template <int ROUNDS>

@@ -180,3 +180,17 @@ def test_cell_starts_and_face_stencils(grid, n):
     ref = P.acceleration_pm(x, m, c, bw, 70.0, 0.3, rho, grid, 0.5)
     # (2^3 nodes: every difference cancels, both sides hold rounding noise of about 1e-13)
     assert np.abs(a - ref).max() <= 1e-10 * max(np.abs(ref).max(), 1.0)
+
+
+@pytest.mark.parametrize("sizes", [(300000, 262144), (800000, 786432, 262144)])
+def test_fewer_particles_on_the_same_grid(sizes):
+    """The grid's sort buffers are kept between calls and sized by the most particles so far; a smaller set may sort in
+    smaller tiles, which need more counters."""
+    grid, c, bw = 64, np.zeros(3), 1.0
+    for n in sizes:
+        x, m = _clustered(n, n)
+        rho = m.sum() / 8.0
+        print("pm", n, flush=True)
+        a = L.acceleration_pm(x, m, c, bw, 0.7, 0.3, rho, grid, 0.5)
+        ref = P.acceleration_pm(x, m, c, bw, 0.7, 0.3, rho, grid, 0.5)
+        assert np.abs(a - ref).max() < 1e-10 * np.abs(ref).max(), n
