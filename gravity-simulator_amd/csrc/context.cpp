@@ -81,19 +81,10 @@ ErrorStatus slot(Context *c, Slot s, size_t bytes, void **out)
     return make_success_error_status();
 }
 
-ErrorStatus pinned(Context *c, size_t bytes, void **out)
+ErrorStatus pinned(Context *c, PinnedUse use, void **out)
 {
-    if (c->pinned_bytes < bytes) {
-        if (c->pinned) {
-            GS_HIP(hipStreamSynchronize(c->stream));
-            GS_HIP(hipHostFree(c->pinned));
-            c->pinned = nullptr;
-            c->pinned_bytes = 0;
-        }
-        GS_HIP(hipHostMalloc(&c->pinned, bytes, hipHostMallocDefault));
-        c->pinned_bytes = bytes;
-    }
-    *out = c->pinned;
+    if (!c->pinned) GS_HIP(hipHostMalloc(&c->pinned, PIN_COUNT * PIN_BYTES, hipHostMallocDefault));
+    *out = static_cast<char *>(c->pinned) + use * PIN_BYTES;
     return make_success_error_status();
 }
 

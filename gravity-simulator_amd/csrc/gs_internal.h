@@ -67,9 +67,7 @@ struct Context {
     char name[256] = {0};
     std::recursive_mutex mu;
     Buffer slots[SLOT_COUNT];
-    // pinned host staging for small readbacks
-    void *pinned = nullptr;
-    size_t pinned_bytes = 0;
+    void *pinned = nullptr;  // PIN_COUNT regions, allocated by the first pinned()
 
     // timing
     bool timing = false;
@@ -92,7 +90,17 @@ hipError_t noalloc_scratch_init(int device);
 
 // Grow-only device buffer for a slot.
 ErrorStatus slot(Context *c, Slot s, size_t bytes, void **out);
-ErrorStatus pinned(Context *c, size_t bytes, void **out);
+
+// Pinned host memory for small readbacks: PIN_BYTES per use, never moved or
+// freed, so that a run may hold its region across force evaluations, which
+// use the tree's.  A region belongs to whoever holds the context's mutex.
+enum PinnedUse {
+    PIN_TREE,  // sizes read back by the tree build
+    PIN_RUN,   // error sums and maxima of the adaptive integrators
+    PIN_COUNT
+};
+constexpr size_t PIN_BYTES = 1024;
+ErrorStatus pinned(Context *c, PinnedUse use, void **out);
 
 // Kernel timing: wrap a launch as
 //   int t = timing_begin(c, "name");  launch...;  timing_end(c, t);

@@ -488,7 +488,7 @@ ErrorStatus ias15_gpu(System *system, IntegratorParam *ip, AccelerationParam *ap
     const double *hmax = nullptr;
     if (small) {
         void *hp;
-        GS_TRY(pinned(c, 64, &hp));
+        GS_TRY(pinned(c, PIN_RUN, &hp));
         hmax = static_cast<const double *>(hp);
         sn = SmallN::plan(n);
         A.m = S.m, A.g = S.g, A.b = S.b, A.b06 = S.b0 + 6 * n3, A.e = S.e;

@@ -2440,8 +2440,9 @@ static ErrorStatus tree_build_flat(Context *c, DeviceTree *t, int n, int leaf_ca
     GS_TRY(slot(c, SLOT_MISC, 256, &p));
     unsigned *total_dev = static_cast<unsigned *>(p);
     void *hp;
-    GS_TRY(pinned(c, 256, &hp));
+    GS_TRY(pinned(c, PIN_TREE, &hp));
     unsigned *lev_host = static_cast<unsigned *>(hp);
+    static_assert(sizeof(unsigned) * (FB_DEPTHS + 1) <= PIN_BYTES, "the level bounds fit the region");
 
     hipLaunchKernelGGL(k_fb_digits, dim3((n + 1 + FB_PAD + 255) / 256), dim3(256), 0, c->stream,
                        t->skeys, n, Ld);
@@ -2526,7 +2527,7 @@ ErrorStatus tree_build(Context *c, const double *x, const double *m, int n, int 
     GS_TRY(slot(c, SLOT_MISC, 256, &p));
     total_dev = static_cast<unsigned *>(p);
     void *hp;
-    GS_TRY(pinned(c, 256, &hp));
+    GS_TRY(pinned(c, PIN_TREE, &hp));
     unsigned *total_host = static_cast<unsigned *>(hp);
     for (int d = 1; d <= MAXL; d++) {
         const int lb = t->level_begin[d - 1], le = t->level_end[d - 1];

@@ -528,7 +528,7 @@ ErrorStatus rk_embedded_gpu(System *system, IntegratorParam *ip, AccelerationPar
            *tve = txe + n3, *tx = tve + n3, *xk = tx + n3, *vk = xk + St * n3,
            *terms = vk + St * n3;
     void *hp;
-    GS_TRY(pinned(c, 64, &hp));
+    GS_TRY(pinned(c, PIN_RUN, &hp));
     double *hsum = static_cast<double *>(hp);
     GS_TRY(S.upload(system));
     SnapshotWriter snaps;

@@ -5,6 +5,10 @@ With the bitwise FP64 force methods every update keeps the reference's
 operation order and the embedded error norm is summed in index order, so
 final states and step counts are bitwise equal to the reference's golden
 runs (f9) and to the oracle."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -103,3 +107,32 @@ def test_embedded_one_workgroup_sizes_and_sequential_sum_bitwise(integ, n):
         xo, vo, so = O.rk_embedded(x, v, m, 1.0, integ, 1e-9, tf, eps=1e-2, method=method)
         assert r[4] == so
         assert np.array_equal(r[1], xo) and np.array_equal(r[2], vo)
+
+
+_TREE_RUN = """
+import sys
+import numpy as np
+from grav_sim_amd import ic
+from grav_sim_amd import lib as L
+x, v, m = ic.plummer(300, 23)
+r = L.launch_simulation(x, v, m, 1.0, 6, -1.0, 0.05, method=3, eps=0.05, theta=0.05, leaf=1, tolerance=1e-6)
+np.savez(sys.argv[1], x=r[1], v=r[2], steps=r[4])
+"""
+
+
+def test_embedded_with_tree_forces_as_the_first_run_of_a_process(tmp_path):
+    """The run's error sum lies in pinned host memory that it holds across the tree builds of its force evaluations.  A
+    new process, in which nothing has been pinned before the run, must give what this one gives, and both the run with
+    the direct sum up to the walk's FP32 reciprocal roots (at this angle hardly a node is accepted)."""
+    out = tmp_path / "run.npz"
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join(sys.path))
+    print("new process: DOPRI, Barnes-Hut, n = 300", flush=True)
+    subprocess.run([sys.executable, "-c", _TREE_RUN, str(out)], env=env, check=True, timeout=100)
+    f = np.load(out)
+    x, v, m = ic.plummer(300, 23)
+    r = L.launch_simulation(x, v, m, 1.0, 6, -1.0, 0.05, method=3, eps=0.05, theta=0.05, leaf=1, tolerance=1e-6)
+    assert r[4] == f["steps"] and np.array_equal(r[1], f["x"]) and np.array_equal(r[2], f["v"])
+    xo, vo, so = O.rk_embedded(x, v, m, 1.0, 6, 1e-6, 0.05, eps=0.05, method=1)
+    print(f"steps {r[4]} (direct sum {so}), max |dx| {np.abs(r[1] - xo).max():.1e}")
+    assert abs(int(r[4]) - so) <= 1
+    assert np.abs(r[1] - xo).max() < 1e-6 and np.abs(r[2] - vo).max() < 1e-5
