@@ -1007,6 +1007,12 @@ constexpr int WK_STACK = 1024;
 constexpr int WK_ILP = 2;  // entries a lane works on at a time
 constexpr int WK_BATCH_LIMIT = WK_STACK - 8 * (MAXL + 2);
 
+// The mark of a stack that would have overflowed, in a walk's interaction
+// counter: set by an OR, since several wavefronts may set it (four additions
+// of 2^62 would cancel, and the eight wavefronts of a shared group that walk
+// alike would all add theirs).
+constexpr unsigned long long WALK_OVERFLOW = 1ull << 63;
+
 struct WalkArgs {
     double theta2;
     double eps2;
@@ -1351,7 +1357,10 @@ __global__ __launch_bounds__(64) void k_walk(const NodeRec *__restrict__ nodes,
     }
     // interaction count: one atomic per wave (an overflow, which the batch
     // limit excludes, is flagged through it)
-    if (lane == 0 && n_int) atomicAdd(n_int, wcnt + (overflow ? 1ull << 62 : 0ull));
+    if (lane == 0 && n_int) {
+        atomicAdd(n_int, wcnt);
+        if (overflow) atomicOr(n_int, WALK_OVERFLOW);
+    }
 }
 
 // The same walk by single nodes: 64 targets, one per lane, a node at a time,
@@ -1519,7 +1528,7 @@ __global__ __launch_bounds__(WS_BLOCK) void k_walk_single(const NodeRec *__restr
         } else if (lane == 0 && n_int) {
             // cannot happen for depth <= 21 (at most 7 pending siblings per
             // level); flagged through the counter instead of overflowing
-            atomicAdd(n_int, 1ull << 62);
+            atomicOr(n_int, WALK_OVERFLOW);
         }
     }
     if (valid) {
@@ -2231,7 +2240,8 @@ __global__ __launch_bounds__(64 * W) void k_walk_group(const NodeRec *__restrict
     tot = valid && wave == 0 ? tot - 1u : 0u;
     for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off);
     if (lane == 0 && n_int) {
-        if (wave == 0 || overflow) atomicAdd(n_int, tot + (overflow ? (1ull << 62) : 0ull));
+        if (wave == 0) atomicAdd(n_int, tot);
+        if (overflow) atomicOr(n_int, WALK_OVERFLOW);
         if (LE) atomicAdd(n_int + 1, static_cast<unsigned long long>(nfar));
     }
 }
@@ -2654,7 +2664,7 @@ ErrorStatus tree_walk(Context *c, DeviceTree *t, const double *x, double G, doub
         unsigned long long h = 0;
         GS_HIP(hipMemcpyAsync(&h, cnt, sizeof(h), hipMemcpyDeviceToHost, c->stream));
         GS_HIP(hipStreamSynchronize(c->stream));
-        if (h >> 62)
+        if (h & WALK_OVERFLOW)
             return WRAP_RAISE_ERROR(GRAV_FAILURE, "Barnes-Hut walk stack overflow");
         *interactions = static_cast<long long>(h);
     }
@@ -2747,7 +2757,7 @@ ErrorStatus tree_walk_group(Context *c, DeviceTree *t, double G, double eps, dou
     unsigned long long h[2] = {0, 0};
     GS_HIP(hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, c->stream));
     GS_HIP(hipStreamSynchronize(c->stream));
-    if (h[0] >> 62) return WRAP_RAISE_ERROR(GRAV_FAILURE, "Barnes-Hut group walk stack overflow");
+    if (h[0] & WALK_OVERFLOW) return WRAP_RAISE_ERROR(GRAV_FAILURE, "Barnes-Hut group walk stack overflow");
     if (interactions) *interactions = static_cast<long long>(h[0]);
     if (far_pairs) *far_pairs = static_cast<long long>(h[1]);
     return make_success_error_status();
