@@ -137,12 +137,16 @@ __global__ void k_pm_cell_keys(const double *__restrict__ x, int n, int N, doubl
 // PM_SPAN, the lanes write them side by side, each finding its cell's
 // particle among the 64 keys; otherwise every lane writes the cells up to its
 // particle's, and runs of more than PM_GAP empty cells are left to the next
-// kernel, one wavefront per run, so that a clustered distribution's empty
-// space is not one thread's loop.  (2^21 particles on 256^3 cells: 24 us with
-// the next kernel, 63 with the second form alone, 49 for clearing and filling
-// pairs of positions.)
+// kernel in pieces of PM_PIECE cells, one wavefront per piece, so that a
+// clustered distribution's empty space is neither one thread's loop nor one
+// wavefront's.  (2^21 particles on 256^3 cells, spread evenly: 24 us with the
+// next kernel, 63 with the second form alone, 49 for clearing and filling
+// pairs of positions.  All in one clump, sigma 3 % of the box: 42 us for both
+// kernels, 1268 with one wavefront per run.)
 constexpr int PM_GAP = 64;
 constexpr int PM_SPAN = 4096;
+constexpr int PM_PIECE = 8192;
+static_assert(PM_PIECE > PM_GAP + 1, "a run of L cells has at most L / (PM_GAP + 1) pieces");
 
 __global__ __launch_bounds__(PM_BLOCK) void k_pm_cell_starts(const long long *__restrict__ key, int n,
                                                              int cells, int *__restrict__ start,
@@ -173,14 +177,16 @@ __global__ __launch_bounds__(PM_BLOCK) void k_pm_cell_starts(const long long *__
     if (p > n) return;
     const int lo = (lane == 0 ? before : keys[wave][lane - 1]) + 1;
     if (mine - lo >= PM_GAP) {
-        gaps[atomicAdd(num_gaps, 1u)] = make_int2(lo, p);
+        const int pieces = (mine - lo) / PM_PIECE + 1;
+        int2 *g = gaps + atomicAdd(num_gaps, static_cast<unsigned>(pieces));
+        for (int k = 0; k < pieces; k++) g[k] = make_int2(lo + k * PM_PIECE, p);
         return;
     }
     for (int c = lo; c <= mine; c++) start[c] = p;
 }
 
-// (every gap but the one of the last particle ends at the cell of particle
-// gap.y; their number is at most cells / PM_GAP + 1)
+// Pieces of runs of empty cells: from cell gap.x, PM_PIECE cells or up to the
+// cell of particle gap.y (of gap.y = n: the end).
 __global__ void k_pm_fill_gaps(const long long *__restrict__ key, int n, int cells,
                                const int2 *__restrict__ gaps, const unsigned *__restrict__ num_gaps,
                                int *__restrict__ start)
@@ -189,7 +195,8 @@ __global__ void k_pm_fill_gaps(const long long *__restrict__ key, int n, int cel
     const int lane = threadIdx.x & 63;
     for (unsigned g = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); g < *num_gaps; g += waves) {
         const int2 gap = gaps[g];
-        const int hi = gap.y == n ? cells : static_cast<int>(key[gap.y]);
+        const int end = gap.y == n ? cells : static_cast<int>(key[gap.y]);
+        const int hi = min(end, gap.x + PM_PIECE - 1);
         for (int c = gap.x + lane; c <= hi; c += 64) start[c] = gap.y;
     }
 }
@@ -448,7 +455,7 @@ struct PmWork {
     double *grid = nullptr;   // deposited density, then the potential (N^3)
     double2 *spec = nullptr;  // half spectrum N x N x (N/2 + 1)
     int *start = nullptr;     // first sorted position of each cell's particles (N^3 + 1)
-    int2 *gaps = nullptr;     // long runs of empty cells (first cell, particle after them)
+    int2 *gaps = nullptr;     // pieces of long runs of empty cells (first cell, particle after them)
     int passes = 0;           // radix passes for keys below N^3
     // (cell, particle) sort buffers for up to `cap` particles
     int cap = 0;
@@ -511,7 +518,7 @@ struct PmWork {
         GS_HIP(hipMalloc(reinterpret_cast<void **>(&grid), sizeof(double) * n3));
         GS_HIP(hipMalloc(reinterpret_cast<void **>(&spec), sizeof(double2) * nh));
         GS_HIP(hipMalloc(reinterpret_cast<void **>(&start), sizeof(int) * (n3 + 1)));
-        // (disjoint gaps of more than PM_GAP cells, after their counter)
+        // (at most one piece per PM_GAP + 1 of the cells, after their counter)
         GS_HIP(hipMalloc(reinterpret_cast<void **>(&gaps), sizeof(int2) * (n3 / PM_GAP + 3)));
         int bits = 0;
         while ((1ull << bits) < n3) bits++;
