@@ -81,7 +81,7 @@ __device__ __forceinline__ void stumpff_series(double z, Div div, double &t2, do
     t2 = t2 / 2.0;
 }
 
-__device__ void stumpff(double z, double &c0, double &c1, double &c2, double &c3)
+__device__ __forceinline__ void stumpff(double z, double &c0, double &c1, double &c2, double &c3)
 {
     int k = 0;
     while (fabs(z) > 0.1) {
@@ -114,7 +114,7 @@ __device__ void stumpff(double z, double &c0, double &c1, double &c2, double &c3
 // Returns 1 when the particle is to be removed (non-converged with error
 // above 1e-5 or a non-finite Stumpff argument), 2 when the Stumpff argument
 // was not finite (reported when removal is off).
-__device__ int kepler_drift(double *jx, double *jv, double gm, double dt)
+__device__ __forceinline__ int kepler_drift(double *jx, double *jv, double gm, double dt)
 {
     const double x0 = jx[0], x1 = jx[1], x2 = jx[2];
     const double v0 = jv[0], v1 = jv[1], v2 = jv[2];
@@ -168,7 +168,7 @@ __device__ __forceinline__ double cube_plus(double a, double b, double c, double
 }
 
 // Block-wide exclusive scan of small integers (WF_BLOCK threads).
-__device__ int block_scan_excl(int v, int *total, int *buf)
+__device__ __forceinline__ int block_scan_excl(int v, int *total, int *buf)
 {
     const int t = threadIdx.x;
     buf[t] = v;
@@ -225,7 +225,7 @@ union WfScratch {
 static_assert(sizeof(WfScratch) == sizeof(int) * WF_MAX_N, "the quotients fit in the flags");
 
 // Sort (distance, index) ascending, lexicographically, for n <= WF_MAX_N.
-__device__ void bitonic_sort(WfShared &S, int n)
+__device__ __forceinline__ void bitonic_sort(WfShared &S, int n)
 {
     int P = 1;
     while (P < n) P <<= 1;
@@ -265,7 +265,7 @@ constexpr int WF_OET_PASSES = 24;
 // finish in a few passes; if they do not within WF_OET_PASSES, the bitonic
 // sort takes the partly sorted pairs.  The pairs are distinct, so both give
 // the same order.  NaN distances go straight to the bitonic sort.
-__device__ void sort_pairs(WfShared &S, int n)
+__device__ __forceinline__ void sort_pairs(WfShared &S, int n)
 {
     int unsorted = 0, nan = 0;
     for (int i = threadIdx.x; i < n; i += WF_BLOCK) {
@@ -302,7 +302,7 @@ __device__ void sort_pairs(WfShared &S, int n)
 // Distances from the particle whose id is 0 (src/system.c:1232-1277) and
 // their sort: S.idx[i] = the current place of the particle that goes to
 // sorted place i (the identity when there is no particle with id 0).
-__device__ void sort_keys(WfShared &S, int n, const double *pos, const int *ids)
+__device__ __forceinline__ void sort_keys(WfShared &S, int n, const double *pos, const int *ids)
 {
     if (threadIdx.x == 0) {
         int pr = -1;
@@ -334,7 +334,7 @@ __device__ void sort_keys(WfShared &S, int n, const double *pos, const int *ids)
 
 // sort_keys, then permute (pos, vel, m, ids) through the alternate buffers;
 // only the particles that changed place move.
-__device__ void sort_by_distance(WfShared &S, int n, double *pos, double *vel, double *m,
+__device__ __forceinline__ void sort_by_distance(WfShared &S, int n, double *pos, double *vel, double *m,
                                  int *ids, double *pos2, double *vel2, double *m2, int *ids2)
 {
     sort_keys(S, n, pos, ids);
@@ -368,7 +368,7 @@ __device__ void sort_by_distance(WfShared &S, int n, double *pos, double *vel, d
 // Massive list (m != 0, or every particle for the pairwise form) and the
 // cumulative masses eta at each massive particle, summed in index order
 // (src/integrator_whfast.c:1266-1279; massless particles add exactly 0).
-__device__ void massive_list(WfShared &S, int n, const double *m, int method,
+__device__ __forceinline__ void massive_list(WfShared &S, int n, const double *m, int method,
                              const short *perm = nullptr)
 {
     // the mass at sorted place i: m[i], or m[perm[i]] before the arrays are permuted
@@ -434,7 +434,7 @@ struct MassiveCursor {
 };
 
 // eta[i] for every particle, into S.key (free between the sorts).
-__device__ void fill_eta(WfShared &S, int n)
+__device__ __forceinline__ void fill_eta(WfShared &S, int n)
 {
     const int nm = S.nm < WF_MAX_MASSIVE ? S.nm : WF_MAX_MASSIVE;
     MassiveCursor mc;
@@ -449,7 +449,7 @@ __device__ void fill_eta(WfShared &S, int n)
 // with an unchanged eta, so once c maps onto itself it stays there for the
 // rest of the run of massless particles: the loop then only forms q from the
 // cached quotient, which is bitwise what the full recurrence produces.
-__device__ void j2c_component(int n, int d, const double *jq, double *q, const double *m,
+__device__ __forceinline__ void j2c_component(int n, int d, const double *jq, double *q, const double *m,
                               const WfShared &S)
 {
     const double *eta = S.key;
@@ -496,7 +496,7 @@ __device__ __forceinline__ double run_quotient(const WfShared &S, const WfScratc
 // non-finite jq), or whose walk meets c == -0 or no fixed point within J2C_K,
 // are marked in X.j.fallback for the serial recurrence; both give the same
 // bits.  Called by all threads.
-__device__ void j2c_quotients(int n, const double *jq, const WfShared &S, WfScratch &X, int bad)
+__device__ __forceinline__ void j2c_quotients(int n, const double *jq, const WfShared &S, WfScratch &X, int bad)
 {
     const int tid = threadIdx.x;
     const int nm = S.nm < WF_MAX_MASSIVE ? S.nm : WF_MAX_MASSIVE;
@@ -547,7 +547,7 @@ __device__ void j2c_quotients(int n, const double *jq, const WfShared &S, WfScra
 
 // Second half: q for every particle into global memory; the serial
 // recurrence for the components marked in X.j.fallback.
-__device__ void j2c_fill(int n, const double *jq, double *q, const double *m, const WfShared &S,
+__device__ __forceinline__ void j2c_fill(int n, const double *jq, double *q, const double *m, const WfShared &S,
                          const WfScratch &X)
 {
     const int tid = threadIdx.x;
@@ -574,7 +574,7 @@ __device__ void j2c_fill(int n, const double *jq, double *q, const double *m, co
 }
 
 // Both halves, with the non-finite check over the massless particles.
-__device__ void j2c_block(int n, const double *jq, double *q, const double *m, WfShared &S,
+__device__ __forceinline__ void j2c_block(int n, const double *jq, double *q, const double *m, WfShared &S,
                           WfScratch &X)
 {
     if (threadIdx.x == 0) S.bad = 0;
@@ -593,7 +593,7 @@ __device__ void j2c_block(int n, const double *jq, double *q, const double *m, W
 
 // Cartesian -> Jacobi (src/integrator_whfast.c:682-724), one lane per
 // component; particle 0 gets the centre of mass.
-__device__ void c2j_component(int n, int d, const double *q, double *jq, const double *m,
+__device__ __forceinline__ void c2j_component(int n, int d, const double *q, double *jq, const double *m,
                               const WfShared &S)
 {
     const double *eta = S.key;
@@ -612,7 +612,8 @@ __device__ void c2j_component(int n, int d, const double *q, double *jq, const d
 // xi, x0: Cartesian positions of particle i and of particle 0; jxi: its
 // Jacobi position; ginside: for a massless particle, the number of massive
 // particles inside it; fast: the massive particles' positions and G m lie in
-// the range pull3 takes.
+// the range pull3 takes.  PULLS massive particles' pulls are formed at a time.
+template <int PULLS>
 __device__ __forceinline__ void accel_kick_v(const WfShared &S, int i, bool massive, int p,
                                              const double *xi, const double *x0,
                                              const double *jxi, int ginside, double m0, double G,
@@ -640,7 +641,7 @@ __device__ __forceinline__ void accel_kick_v(const WfShared &S, int i, bool mass
     // each sum in ordinal order; the pulls of the inner ones are the outer
     // form's with every sign changed, which is exact
     double in[3] = {0.0, 0.0, 0.0}, out[3] = {0.0, 0.0, 0.0};
-    constexpr int K = 2;
+    constexpr int K = PULLS;
     for (int q0 = 1; q0 < nm; q0 += K) {
         double t[K][3], gm[K], f[K][3];
 #pragma unroll
@@ -697,17 +698,18 @@ __device__ __forceinline__ void accel_kick_v(const WfShared &S, int i, bool mass
 }
 
 // The same with the positions read from global memory.
-__device__ void accel_kick(const WfShared &S, int i, bool massive, int p, const double *x,
+template <int PULLS>
+__device__ __forceinline__ void accel_kick(const WfShared &S, int i, bool massive, int p, const double *x,
                            const double *jx, const double *m, double G, double eps3,
                            double *jv, double dt, double *jv_sync)
 {
     int g = 0;  // massive particles inside i
     if (!massive)
         while (g < S.nm && S.mlist[g] < i) g++;
-    accel_kick_v(S, i, massive, p, &x[3 * i], x, &jx[3 * i], g, m[0], G, eps3, jv, dt, false, jv_sync);
+    accel_kick_v<PULLS>(S, i, massive, p, &x[3 * i], x, &jx[3 * i], g, m[0], G, eps3, jv, dt, false, jv_sync);
 }
 
-__device__ void load_massive_positions(WfShared &S, const double *x)
+__device__ __forceinline__ void load_massive_positions(WfShared &S, const double *x)
 {
     for (int q = threadIdx.x; q < S.nm; q += WF_BLOCK) {
         const int j = S.mlist[q];
@@ -722,7 +724,7 @@ __device__ void load_massive_positions(WfShared &S, const double *x)
 // exterior ordinal ascending): for a massless particle with g massive
 // particles inside it, pairs (q < g <= r); for massive particle p, pairs
 // (q < p < r) (src/integrator_whfast.c:930-949, 1099-1119, 1222-1250).
-__device__ void straddle_sums(WfShared &S, double G, double eps3)
+__device__ __forceinline__ void straddle_sums(WfShared &S, double G, double eps3)
 {
     const int nm = S.nm;
     if (nm <= WF_PAIR_NM) {
@@ -788,7 +790,8 @@ __device__ void straddle_sums(WfShared &S, double G, double eps3)
 }
 
 // jv_sync != NULL: also the half-step-back velocities of a snapshot.
-__device__ void accel_kick_all(WfShared &S, int n, const double *x, const double *jx,
+template <int PULLS>
+__device__ __forceinline__ void accel_kick_all(WfShared &S, int n, const double *x, const double *jx,
                                const double *m, double G, double eps3, double *jv, double dt,
                                int method, double *jv_sync = nullptr)
 {
@@ -796,10 +799,10 @@ __device__ void accel_kick_all(WfShared &S, int n, const double *x, const double
     straddle_sums(S, G, eps3);
     // massive particles (ordinal >= 1), one per thread
     for (int p = 1 + static_cast<int>(threadIdx.x); p < S.nm; p += WF_BLOCK)
-        accel_kick(S, S.mlist[p], true, p, x, jx, m, G, eps3, jv, dt, jv_sync);
+        accel_kick<PULLS>(S, S.mlist[p], true, p, x, jx, m, G, eps3, jv, dt, jv_sync);
     if (method == 2) {
         for (int i = 1 + threadIdx.x; i < n; i += WF_BLOCK)
-            if (m[i] == 0.0) accel_kick(S, i, false, -1, x, jx, m, G, eps3, jv, dt, jv_sync);
+            if (m[i] == 0.0) accel_kick<PULLS>(S, i, false, -1, x, jx, m, G, eps3, jv, dt, jv_sync);
     }
     __syncthreads();
 }
@@ -809,7 +812,8 @@ __device__ void accel_kick_all(WfShared &S, int n, const double *x, const double
 // registers; global positions are written only when `write_x` (they are
 // an output, not an input, of the next step).  Requires no component marked
 // for the serial recurrence.
-__device__ void kick_from_quotients(WfShared &S, const WfScratch &X, int n, double *x,
+template <int PULLS>
+__device__ __forceinline__ void kick_from_quotients(WfShared &S, const WfScratch &X, int n, double *x,
                                     const double *jx, double G, double eps3, double *jv, double dt,
                                     int method, bool write_x, double *jv_sync)
 {
@@ -831,7 +835,7 @@ __device__ void kick_from_quotients(WfShared &S, const WfScratch &X, int n, doub
     const double m0 = S.mm[0];
     for (int p = 1 + static_cast<int>(threadIdx.x); p < nm; p += WF_BLOCK) {
         const int i = S.mlist[p];
-        accel_kick_v(S, i, true, p, S.mx[p], S.mx[0], &jx[3 * i], 0, m0, G, eps3, jv, dt,
+        accel_kick_v<PULLS>(S, i, true, p, S.mx[p], S.mx[0], &jx[3 * i], 0, m0, G, eps3, jv, dt,
                      fast, jv_sync);
     }
     if (method == 2) {
@@ -848,7 +852,7 @@ __device__ void kick_from_quotients(WfShared &S, const WfScratch &X, int n, doub
                 x[3 * i + 1] = xi[1];
                 x[3 * i + 2] = xi[2];
             }
-            accel_kick_v(S, i, false, -1, xi, S.mx[0], jxi, g + 1, m0, G, eps3, jv, dt,
+            accel_kick_v<PULLS>(S, i, false, -1, xi, S.mx[0], jxi, g + 1, m0, G, eps3, jv, dt,
                          fast, jv_sync);
         }
     }
@@ -857,7 +861,7 @@ __device__ void kick_from_quotients(WfShared &S, const WfScratch &X, int n, doub
 
 // Remove flagged particles preserving order (src/system.c:444-528 and the
 // Jacobi / eta arrays in src/integrator_whfast.c:624-670).
-__device__ int compact(WfShared &S, int n, const int *flag, double *jx, double *jv, double *m,
+__device__ __forceinline__ int compact(WfShared &S, int n, const int *flag, double *jx, double *jv, double *m,
                        int *ids, double *jx2, double *jv2, double *m2, int *ids2)
 {
     int o = 0;
@@ -912,16 +916,18 @@ __global__ __launch_bounds__(WF_BLOCK) void k_whfast_init(WfArgs A)
     else if (threadIdx.x >= 64 && threadIdx.x < 67) c2j_component(n, threadIdx.x - 64, v, jv, m, S);
     __syncthreads();
     const double eps3 = A.eps * A.eps * A.eps;
-    accel_kick_all(S, n, x, jx, m, A.G, eps3, jv, 0.5 * A.dt, A.method);
+    accel_kick_all<2>(S, n, x, jx, m, A.G, eps3, jv, 0.5 * A.dt, A.method);
 }
 
 // `nsteps` steps of the main loop (src/integrator_whfast.c:290-378).
-// Bound by the latency of each particle's FP64 chains.  210 VGPRs, two
-// wavefronts per SIMD, and two pulls at a time in the kick: held to 128
-// registers for four wavefronts, with one pull at a time through the
-// compiler's square root and divisions, 4096 systems took 125 ms per 200
-// steps and 512 systems 16.7; now 76 and 13.5 (one pull at a time: 77, 14.1).
-__global__ __launch_bounds__(WF_BLOCK) void k_whfast_steps(WfArgs A)
+// Bound by the latency of each particle's FP64 chains while all systems are
+// resident, then by the number that are.  PULLS = 2: 155 VGPRs, three
+// wavefronts per SIMD and so three systems per CU.  PULLS = 1, held to 128:
+// four.  (All device functions above are inlined: as calls they take the
+// registers of the largest, 210, whatever the kernel is held to.)
+template <int PULLS>
+__global__ __launch_bounds__(WF_BLOCK) __attribute__((amdgpu_waves_per_eu(PULLS == 1 ? 4 : 2))) void
+k_whfast_steps(WfArgs A)
 {
     __shared__ WfShared S;
     __shared__ WfScratch X;
@@ -1021,9 +1027,9 @@ __global__ __launch_bounds__(WF_BLOCK) void k_whfast_steps(WfArgs A)
         j2c_quotients(n, jx, S, X, pos_bad);
         if (X.j.fallback[0] | X.j.fallback[1] | X.j.fallback[2]) {
             j2c_fill(n, jx, x, m, S, X);
-            accel_kick_all(S, n, x, jx, m, A.G, eps3, jv, dt, A.method, jv_sync);
+            accel_kick_all<PULLS>(S, n, x, jx, m, A.G, eps3, jv, dt, A.method, jv_sync);
         } else {
-            kick_from_quotients(S, X, n, x, jx, A.G, eps3, jv, dt, A.method, last, jv_sync);
+            kick_from_quotients<PULLS>(S, X, n, x, jx, A.G, eps3, jv, dt, A.method, last, jv_sync);
         }
         if (snap) {
             // particle 0 gets no acceleration: jv + 0 * (-dt / 2) == jv
@@ -1190,7 +1196,16 @@ ErrorStatus whfast_ensemble(int num_systems, const int64 *offsets, int32 *ids, d
                 }
             }
         const int rec = timing_begin(c, "whfast_steps");
-        hipLaunchKernelGGL(k_whfast_steps, dim3(num_systems), dim3(WF_BLOCK), 0, c->stream, A);
+        // all resident at three per CU: two pulls at a time.  100 steps, ms, two
+        // / one at a time (and one through the compiler's square root and
+        // divisions, the form before): 512 systems of 9 particles 1.61 / 1.72
+        // (1.90), with up to 2000 test particles 8.0 / 8.4 (9.7); 768 with up to
+        // 100: 2.20 / 2.36 (2.69); 1024 of 9: 3.2 / 1.81 (1.95), up to 2000: 10.0
+        // / 8.4 (9.6); 4096 of 9: 9.5 / 7.6 (8.3), up to 2000: 30 / 28 (36).
+        if (num_systems <= 3 * c->cu_count)
+            hipLaunchKernelGGL(k_whfast_steps<2>, dim3(num_systems), dim3(WF_BLOCK), 0, c->stream, A);
+        else
+            hipLaunchKernelGGL(k_whfast_steps<1>, dim3(num_systems), dim3(WF_BLOCK), 0, c->stream, A);
         timing_end(c, rec);
         e = hipGetLastError();
         done += A.nsteps;

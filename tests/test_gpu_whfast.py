@@ -61,8 +61,8 @@ def test_whfast_odd_step_counts_match_oracle_bitwise(tf):
 
 def test_whfast_planar_systems_match_oracle_bitwise():
     """Planar systems: every z is 0, so the z component of the Jacobi ->
-    Cartesian recurrence carries c == 0 and takes the serial path, while x and
-    y take the run-quotient path; both must give the oracle's bits.  Planets
+    Cartesian recurrence carries an exact zero through every quotient, while x
+    and y carry ordinary values; all must give the oracle's bits.  Planets
     at a ~ logU[0.4, 30] land between the test particles (a in [2, 3.5]) after
     the distance sort, so the massless runs have many lengths."""
     off, X, V, M = ic.ensemble(6, 31, max_test=400)
@@ -128,3 +128,22 @@ def test_centre_of_mass_coordinate_exactly_zero(flip):
         io, xo, vo, mo = O.whfast(x[:k], v[:k], m[:k], 1.0, 0.01, 0.4, method=method)
         assert np.array_equal(ids, io) and np.array_equal(mg, mo)
         assert np.array_equal(xg, xo) and np.array_equal(vg, vo)
+
+
+@pytest.mark.parametrize("few,many", [((4, 700), (0, 0)), ((3, 1900), (765, 0)), ((3, 1900), (766, 0)), ((900, 60), (0, 0))])
+def test_forms_chosen_by_the_number_of_systems(few, many):
+    """Ensembles around the number of systems (768 on 256 CUs) from which the kick forms one pull at a time (systems and
+    most test particles each), with a particle that is removed in the first step."""
+    parts = [ic.ensemble(n, 71 + n, max_test=t) for n, t in (few, many) if n]
+    off = np.concatenate([[0], np.cumsum(np.concatenate([np.diff(p[0]) for p in parts]))]).astype(np.int64)
+    X, V, M = (np.concatenate([p[k] for p in parts]) for k in (1, 2, 3))
+    big = int(np.argmax(np.diff(off)))
+    gone = int(off[big + 1]) - 1
+    V[gone] = [1e200, 0.0, 0.0]
+    res = L.whfast_ensemble(off, X, V, M, 1.0, 0.01, 0.12, method=2)
+    for s in range(len(off) - 1):
+        sl = slice(off[s], off[s + 1])
+        io, xo, vo, mo = O.whfast(X[sl], V[sl], M[sl], 1.0, 0.01, 0.12, method=2)
+        ids, x, v, m = res[s]
+        assert np.array_equal(ids, io) and np.array_equal(x, xo) and np.array_equal(v, vo) and np.array_equal(m, mo), s
+    assert len(res[big][0]) == off[big + 1] - off[big] - 1
