@@ -1001,8 +1001,9 @@ __global__ void k_fb_fix(NodeRec *__restrict__ nodes, int nn, const long long *_
 }
 
 // ------------------------------------------------------------------ walk
-// Batch passes keep the stack below WK_BATCH_LIMIT; single-node passes then
-// grow it by at most 7 per level of the remaining depth.
+// Passes keep the stack below WK_BATCH_LIMIT whatever their entries open: they
+// take at most one entry per 7 free places (WalkArgs::take); single-node
+// passes then grow it by at most 7 per level of the remaining depth.
 constexpr int WK_STACK = 1024;
 constexpr int WK_ILP = 2;  // entries a lane works on at a time
 constexpr int WK_BATCH_LIMIT = WK_STACK - 8 * (MAXL + 2);
@@ -1019,6 +1020,7 @@ struct WalkArgs {
     double G;
     double phi2;     // group walk: squared expansion ratio (0: no local expansions)
     double thetaf2;  // squared opening angle for far nodes (expanded ones)
+    int take;        // per-particle walk: 65536 entries taken per free place of the stack, rounded up
 };
 
 __device__ __forceinline__ void pp_force(double xi0, double xi1, double xi2, double px, double py,
@@ -1319,7 +1321,7 @@ __global__ __launch_bounds__(64) void k_walk(const NodeRec *__restrict__ nodes,
         }
         __syncthreads();
         kn = min(top, 64);
-        if (top + 7 * kn > WK_BATCH_LIMIT) kn = max(1, (WK_BATCH_LIMIT - top) / 7);
+        kn = min(kn, max(1, ((WK_BATCH_LIMIT - top) * args.take) >> 16));
         kn = min(kn, top);
         node = 0;
         mask = 0;
@@ -2603,6 +2605,15 @@ ErrorStatus tree_walk(Context *c, DeviceTree *t, const double *x, double G, doub
     args.G = G;
     args.phi2 = 0.0;
     args.thetaf2 = args.theta2;
+    // At small angles most entries of a pass are opened, so passes of one
+    // entry per 7 free places fill the stack within two levels, and the rest
+    // of the subtree goes entry by entry; one per 11 leaves room on every level
+    // (G = 2, us, 7 / 11 places: Plummer sphere of 140000, theta 0.2: 16300 /
+    // 6980, 524288: 46900 / 24900; two spheres of 2^21, 0.3: 38400 / 34800).  At
+    // larger angles few entries are opened and larger passes are the better
+    // choice (2^21, 0.5: 8760 / 9290).
+    const int places = theta < 0.35 ? 11 : 7;
+    args.take = (65536 + places - 1) / places;
     void *p;
     GS_TRY(slot(c, SLOT_MISC, 256, &p));
     unsigned long long *cnt = reinterpret_cast<unsigned long long *>(static_cast<char *>(p) + 64);
@@ -2628,19 +2639,23 @@ ErrorStatus tree_walk(Context *c, DeviceTree *t, const double *x, double G, doub
     //
     // The smaller the angle, the more of the visits neighbours share: past
     // 1024 particles per CU two entries are the better choice below theta 0.5
-    // (2^21, G = 2 / 4, ms: theta 0.4 14.4 / 15.3, 0.3 38.3 / 47.2), and below
-    // an angle that grows with n and with the work of an accepted node the
-    // walk by single nodes.  Single / G = 2, ms, monopoles: 2^19, theta 0.15:
-    // 48.7 / 45.3; 2^20, 0.2: 54.7 / 57.8, 0.25: 33.0 / 30.5; 2^21, 0.25: 61.9
-    // / 73.5, 0.3: 39.4 / 38.3; 2^22, 0.3: 78.3 / 84.9, 0.35: 54.4 / 47.4.
-    // Quadrupoles: 2^19, 0.2: 38.6 / 39.3; 2^20, 0.25: 47.1 / 51.6, 0.3: 30.4
-    // / 28.8; 2^21, 0.3: 57.0 / 66.2, 0.35: 39.8 / 39.7; 2^22, 0.35: 78.8 /
-    // 83.5, 0.4: 55.3 / 53.9.  Features: 2^20, 0.3: 60.5 / 61.4, 0.35: 43.0 /
-    // 41.0; 2^21, 0.35: 81.1 / 87.5, 0.4: 57.0 / 59.4, 0.55: 29.9 / 29.5.  At
-    // 2^18 and theta 0.1, 58.9 / 32.6 and with quadrupoles 72.6 / 51.3.
+    // (2^21, G = 2 / 4, ms: theta 0.4 14.4 / 15.3, 0.3 34.8 / 40.1), and past
+    // 1536 per CU, below an angle that grows with n and with the work of an
+    // accepted node, the walk by single nodes.  The lines are where that one
+    // overtakes on the first of three distributions.  Single / G = 2, ms, for
+    // a Plummer sphere (two spheres and a uniform box favour G = 2 down to
+    // smaller angles): monopoles, 800000, theta 0.2: 45.6 / 47.9; 2^20, 0.2:
+    // 55.4 / 53.5; 2^21, 0.25: 64.8 / 64.0, 0.3: 40.6 / 35.8.  Quadrupoles,
+    // 270000, 0.2: 26.2 / 22.7; 2^19, 0.25: 22.6 / 24.6, 0.3: 14.9 / 14.7;
+    // 2^20, 0.3: 29.8 / 30.7, 0.34: 22.5 / 21.6; 2^21, 0.34: 43.2 / 44.5,
+    // 0.36: 37.8 / 37.6.  Features: 2^19, 0.25: 47.4 / 47.9, 0.3: 31.5 / 30.5;
+    // 2^20, 0.34: 45.6 / 47.1, 0.42: 27.1 / 26.3; 2^21, 0.42: 50.8 / 54.0.
     const bool many = t->n > 1024 * c->cu_count;
-    const double theta_single =
-        0.40 - 175.0 / std::sqrt(static_cast<double>(t->n)) + (feat ? 0.12 : order >= 2 ? 0.06 : 0.0);
+    const double root = std::sqrt(static_cast<double>(t->n));
+    const double theta_single = t->n <= 1536 * c->cu_count ? 0.0
+                                : feat       ? 0.57 - 200.0 / root
+                                : order >= 2 ? 0.42 - 90.0 / root
+                                             : 0.34 - 175.0 / root;
     auto pick = [&](auto k1, auto k2, auto k4, auto k8, auto k16) {
         if (by_nodes) single(k1);
         else if (t->n <= 64 * c->cu_count) walk(k16, 16);

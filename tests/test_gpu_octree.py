@@ -459,19 +459,36 @@ def test_walk_of_many_particles_against_the_oracle(theta):
     assert np.median(e) < 1e-6 and e.max() < 1e-4
 
 
-@pytest.mark.parametrize("method,shift", [(3, 0.0), (19, 0.06)])
-@pytest.mark.parametrize("n,leaf", [(400002, 1), (262146, 8)])
-def test_walk_by_single_nodes_equals_the_walk_by_passes(method, shift, n, leaf):
-    """The angle at which the walk changes form, less and plus 1e-12 of it: the same interactions (no l^2 / d^2 lies
-    that close to theta^2), forces equal to FP32 rounding of the terms, as against the oracle above."""
-    x, v, m = ic.two_spheres(n, 33)
-    th = 0.40 - 175.0 / np.sqrt(n) + shift
+@pytest.mark.parametrize("method,line", [(3, lambda n: 0.34 - 175.0 / np.sqrt(n)), (19, lambda n: 0.42 - 90.0 / np.sqrt(n)),
+                                         (3, lambda n: 0.35), (19, lambda n: 0.35)],
+                         ids=["monopoles", "quadrupoles", "monopoles, passes", "quadrupoles, passes"])
+@pytest.mark.parametrize("dist,leaf", [("two_spheres", 1), ("plummer", 8)])
+def test_walk_forms_either_side_of_an_angle_agree(method, line, dist, leaf):
+    """The angle at which the walk goes over to single nodes, and the one below which its passes take fewer entries,
+    less and plus 1e-12 of it: the same interactions (no l^2 / d^2 lies that close to theta^2), forces equal to FP32
+    rounding of the terms, as against the oracle above."""
+    n = 400002
+    x, v, m = getattr(ic, dist)(n, 33)
+    th = line(n)
     out = []
     for s in (-1e-12, 1e-12):
         a = L.acceleration(x, m, method, eps=1e-2, theta=th * (1 + s), leaf=leaf)
         out.append((a, L.last_walk_interactions()))
     assert out[0][1] == out[1][1]
     e = np.linalg.norm(out[0][0] - out[1][0], axis=1) / np.linalg.norm(out[1][0], axis=1)
+    assert np.median(e) < 1e-6 and e.max() < 1e-4
+
+
+@pytest.mark.parametrize("theta", [0.1, 0.3])
+def test_walk_at_small_angles_against_the_oracle(theta):
+    """Most entries opened, a deep tree: passes limited by the room of the stack on every level."""
+    n = 20000
+    x, v, m = ic.plummer(n, 4)
+    t = O.build_tree(x, m, 1)
+    a = L.acceleration(x, m, 3, eps=1e-2, theta=theta, leaf=1)
+    ao, cnt = O.bh_walk(x, m, t, theta, eps=1e-2, want_counts=True)
+    assert L.last_walk_interactions() == int(cnt.sum())
+    e = np.linalg.norm(a - ao, axis=1) / np.linalg.norm(ao, axis=1)
     assert np.median(e) < 1e-6 and e.max() < 1e-4
 
 
