@@ -1574,16 +1574,17 @@ __global__ __launch_bounds__(WS_BLOCK) void k_walk_single(const NodeRec *__restr
 // workgroup: 6.0 ms against 6.7 with two and 8.2 with four groups (2048
 // entries).
 // Few groups do not fill the chip and the one with the longest list sets the
-// time, so for n <= 256 particles per CU GW_SPLIT wavefronts share a group:
-// they take the first passes alike (wavefront 0 collecting the terms) until
-// the stack holds GW_SHARE entries per wavefront, then every GW_SPLIT-th
-// entry each, and their sums are added at the end.  Walk at theta 0.5, one /
-// four / eight / sixteen wavefronts: n = 10000: 363 / 280 / 239 / 382 us,
-// 60000: 2216 / 1335 / 832 / 981, 120000: 900 / - / 655 / 1886, 160000: 517 /
-// - / 856 / -, 262144: 991 / 988 / 1337 / 3636.  At 120000 the sharing loses
-// for smaller angles and quadrupoles (before it / with eight: theta 0.2 3373 /
-// 3922 us, quadrupoles at 0.35 2431 / 2989, at 0.2 5092 / 7472); at 60000 it
-// gains for all (quadrupoles at 0.35 4539 / 1075, at 0.2 5744 / 2871).
+// time, so for few particles GW_SPLIT wavefronts share a group: they take the
+// first passes alike (wavefront 0 collecting the terms) until the stack holds
+// GW_SHARE entries per wavefront, then every GW_SPLIT-th entry each, and their
+// sums are added at the end.  Two such groups are resident per CU against
+// seventeen of one wavefront, so with many groups or short lists the sharing
+// loses: it is used up to 80 particles per CU, and at theta up to 0.5 up to
+// 160.  Walk, one / eight wavefronts, us: two spheres of 10000, theta 0.5: 348
+// / 221, 20000: 913 / 475; uniform box, theta 0.2, 20000: 577 / 204, 40000: 819
+// / 329; the same at 0.8, 20000: 160 / 166, 26000: 141 / 162, 40000: 150 / 197.
+// From 50000 the outcome turns with the particle number (two spheres at 0.35,
+// 60000: 2269 / 912, 65536 with quadrupoles: 1209 / 1911).
 constexpr int GW_SPLIT = 8;
 constexpr int GW_SHARE = 32;
 constexpr int GW_STACK = 1024;
@@ -2761,7 +2762,7 @@ ErrorStatus tree_walk_group(Context *c, DeviceTree *t, double G, double eps, dou
                            t->sidx, t->n, groups, args, a, cnt, t->quadf);
     };
     auto pick = [&](auto k1, auto kw) {
-        if (t->n <= 256 * c->cu_count) walk(kw, GW_SPLIT);
+        if (t->n <= (theta <= 0.5 ? 160 : 80) * c->cu_count) walk(kw, GW_SPLIT);
         else walk(k1, 1);
     };
     if (order >= 2) pick(k_walk_group<true, false, 1>, k_walk_group<true, false, GW_SPLIT>);

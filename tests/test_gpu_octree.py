@@ -492,14 +492,15 @@ def test_walk_at_small_angles_against_the_oracle(theta):
     assert np.median(e) < 1e-6 and e.max() < 1e-4
 
 
-@pytest.mark.parametrize("n", [2, 66, 700, 65536, 65538, 131074])
-def test_group_walk_forms_against_the_oracle(n):
-    """Several wavefronts per group (up to 65536 particles on 256 CUs) and one: equal interaction counts and forces to
-    FP32 rounding, without and with quadrupoles and with local expansions; trees too small to be shared out."""
+@pytest.mark.parametrize("n,th", [(2, 0.6), (66, 0.6), (700, 0.6), (20480, 0.6), (20482, 0.6), (40960, 0.5), (40962, 0.5),
+                                  (65538, 0.6), (131074, 0.6)])
+def test_group_walk_forms_against_the_oracle(n, th):
+    """Several wavefronts per group (up to 20480 particles on 256 CUs, at theta up to 0.5 up to 40960) and one: equal
+    interaction counts and forces to FP32 rounding, without and with quadrupoles and with local expansions; trees too
+    small to be shared out."""
     x, v, m = ic.two_spheres(n, 70 + n % 89)
     t = O.build_tree(x, m, 1)
     q = O.octree_quad(x, m, t)
-    th = 0.6
     for method, kw in ((20, {}), (21, dict(quad=q)), (22, dict(phi=0.1, theta_far=1.25 * th, quad_far=q))):
         a = L.acceleration(x, m, method, eps=1e-2, theta=th, leaf=1)
         ao, cnt = O.bh_walk_group(x, m, t, th, 64, eps=1e-2, **kw)[:2]
