@@ -69,32 +69,36 @@ def test_fp32_leapfrog_energy_tracks_fp64():
     assert abs(drifts[16] - drifts[1]) < 1e-8
 
 
-@pytest.mark.parametrize("method", [1, 16])
-def test_graph_replayed_steps_equal_eager_steps(method):
-    """Leapfrog steps replayed from a captured HIP graph (timing off) against
-    the same steps launched eagerly (timing on): bitwise equal after every
-    chunk, with eager work (energy, accelerations) between the replays."""
-    x, v, m = ic.plummer(4096, 31)
-    p = L.param(method, eps=1e-3)
+@pytest.mark.parametrize("n,method", [(2, 1), (2, 2), (48, 1), (48, 2), (64, 1), (64, 2), (65, 1), (65, 2), (4096, 1), (4096, 16)])
+def test_steps_with_and_without_kernel_timing_agree(n, method):
+    """With per-kernel timing on, every step's kernels are launched one by one; with it off, the FP64 direct sums of up
+    to 64 particles run a chunk's steps in one workgroup.  Bitwise equal states and energies after every chunk, with
+    other work (energy, accelerations) between the chunks, also where one run takes the forms in turn."""
+    x, v, m = ic.plummer(n, 31)
+    if method == 2:
+        m[(n + 1) // 2:] = 0.0
+    p = L.param(method, eps=1e-3 if n > 100 else 0.05)
     dt = 1e-3
-    sg, se = L.Sim(x, v, m, 1.0), L.Sim(x, v, m, 1.0)
-    sg.leapfrog_begin(p, dt)
-    se.leapfrog_begin(p, dt)
-    for chunk in (5, 17, 3, 40):
+    off, on, mixed = (L.Sim(x, v, m, 1.0) for _ in range(3))
+    for s in (off, on, mixed):
+        s.leapfrog_begin(p, dt)
+    for k, chunk in enumerate((5, 17, 3, 40)):
         L.timing_enable(False)
-        sg.leapfrog_steps(p, dt, chunk)
-        eg = sg.energy()
+        off.leapfrog_steps(p, dt, chunk)
         L.timing_enable(True)
-        se.leapfrog_steps(p, dt, chunk)
-        ee = se.energy()
+        on.leapfrog_steps(p, dt, chunk)
+        L.timing_enable(k % 2 == 1)
+        mixed.leapfrog_steps(p, dt, chunk)
         L.timing_enable(False)
-        xg, vg = sg.download()
-        xe, ve = se.download()
-        assert np.array_equal(xg, xe) and np.array_equal(vg, ve), chunk
-        assert eg == ee
-        sg.acceleration(p, copy=False)  # eager work on the stream between replays
-    sg.close()
-    se.close()
+        xo, vo = off.download()
+        e = off.energy()
+        for s in (on, mixed):
+            xs, vs = s.download()
+            assert np.array_equal(xs, xo) and np.array_equal(vs, vo), chunk
+            assert s.energy() == e
+        off.acceleration(p, copy=False)
+    for s in (off, on, mixed):
+        s.close()
 
 
 @pytest.mark.parametrize("n", [1, 2, 48, 49, 63, 64, 65])
