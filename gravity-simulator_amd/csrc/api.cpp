@@ -522,7 +522,10 @@ ErrorStatus gs_sim_leapfrog_steps(GsSim *s, const AccelerationParam *p, double d
     // the steps' kernels are launched one by one, at about 4.5 us each, which
     // is what a step costs up to 128 particles; above, the device is the
     // slower side.  (A HIP graph of two steps took 18 us to launch: 256 steps
-    // of n = 128 in 2309 us against 1371, of n = 1024 in 3203 against 2576.)
+    // of n = 128 in 2309 us against 1371, of n = 1024 in 3203 against 2576.
+    // An FP32 step is four or five launches; a graph of one took 24 to 40 us:
+    // 256 steps of n = 9 in 6210 us against 2640 to 3640, of 1024 in 9970
+    // against 3300 to 4800, of 4096 in 10170 against 4800.)
     if (k > 0 && fused_step_method(p->method) && s->n <= lf_small_max() && !c->timing) {
         GS_HIP(launch_lf_steps_small(c, s->x, s->xe, s->v, s->ve, s->m, s->n, s->G,
                                      p->softening_length, p->method == ACCELERATION_METHOD_MASSLESS,

@@ -50,8 +50,10 @@ constexpr int F64_BLOCK = 256;
 //                      workgroups are no more than the CUs; then FP64 issue.
 //   k_direct_f64_wide  64 targets per workgroup, one per lane; sources come
 //                      through scalar loads, the adding wavefront runs three
-//                      chains per lane.  Bound by FP64 issue: 34 instructions
-//                      of 4.75 cycles and v_rsq_f64 (16) per 64 terms.
+//                      chains per lane.  34 FP64 instructions of 4.75 cycles
+//                      and v_rsq_f64 (16) per 64 terms: their issue is about
+//                      three quarters of the time at 100000, the rest waits
+//                      for scalar loads and barriers.
 // One MI355X, kernel alone, before (one wavefront of 12 to 24 lanes adding
 // after every tile, its rows 2048 bytes apart, so every read a bank conflict)
 // and now: n = 1024 13.0 -> 8.2 us, 4096 91 -> 44, 16384 1150 -> 461,
@@ -1096,7 +1098,7 @@ constexpr int TARGET_WAVES = 16;  // wavefronts per 64 targets in launch_direct_
 // products, tens of dependent optimiser steps), so the labels' sums keep this
 // one division, whatever f32p_plan finds faster: a sample trains the same
 // weights on any card.  Chunks of at least one tile per wavefront, about 1024
-// workgroups in all (131072 labels: 5.3 ms, by f32p_plan's rule 5.2).
+// workgroups in all (131072 labels: 5.22 ms, by f32p_plan's rule 5.16).
 int direct_f32_label_split(int n, int nt)
 {
     const int wgs = (nt + 63) / 64;
@@ -1220,9 +1222,10 @@ hipError_t launch_copy(Context *c, const void *src, void *dst, size_t bytes)
 // The other block's particles come through scalar loads, K at a time.  1 / r
 // from v_rsq_f64 and two Newton steps (within an ulp; the compiler's sqrt and
 // division where r^2 is out of range, coincident particles among them).
-// Bound by FP64 issue.  One MI355X, before (one thread per particle over all
-// later ones) and now: the whole call for 1024 particles 215 -> 39 us, 20000
-// 3.2 -> 0.35 ms.
+// Short of wavefronts: 20000 particles give 1878, 1.8 per SIMD, and FP64 issue
+// takes 0.44 of the SIMDs' cycles (their number is held down by energy_grid).
+// One MI355X, before (one thread per particle over all later ones) and now:
+// the whole call for 1024 particles 215 -> 39 us, 20000 3.2 -> 0.35 ms.
 constexpr int EN_K = 4;
 
 __global__ __launch_bounds__(64) void k_energy(const double *__restrict__ x,

@@ -14,7 +14,7 @@
 
 namespace gs {
 
-// r2 in [2^-400, 2^400): the operands inverse_cube_ready accepts.
+// r2 in [2^-400, 2^400): the operands r2_in_range accepts.
 constexpr unsigned R2_HI_MIN = (1023u - 400u) << 20;
 constexpr unsigned R2_HI_SPAN = 800u << 20;
 
@@ -106,10 +106,11 @@ __device__ __forceinline__ bool coordinate_in_range(double a)
 }
 
 // q[u][d] = fl(fl(gm[u] t[u][d]) / fl(fl(fl(r r) r) + eps3)), r = fl(sqrt(
-// t[u].t[u])) summed left to right: one square root and three divisions by
-// the same value, whose reciprocal is formed once (v_rcp_f64 and two Newton
-// steps) and corrected per quotient by its exact remainder; K of them step by
-// step, so that their chains overlap.  `fast` promises t[u][d] zero or in
+// t[u].t[u])) summed left to right: one square root (Goldschmidt's iteration
+// with residual corrections, as in over_r3) and three divisions by the same
+// value, whose reciprocal is formed once (v_rcp_f64 and two Newton steps);
+// each quotient is corrected by its exact remainder (Markstein's theorem).  K
+// of them step by step, so that their chains overlap.  `fast` promises t[u][d] zero or in
 // [2^-453, 2^301), gm[u] in [2^-300, 2^300) and 0 <= eps3 < 2^300; |t|^2 is
 // checked here.  Zero numerators keep their sign (the corrections would turn
 // -0 into +0).

@@ -17,10 +17,11 @@
 //                  order, internal nodes sum their children (FP64)
 //   k_walk         one wavefront walks for 4 to 32 Morton-consecutive targets
 //                  with a shared explicit stack of (node, target mask), up to
-//                  64 entries a pass: each target applies the reference
-//                  opening test itself; those that accept a node add its
-//                  monopole, the others descend.  Geometry and sums in FP64, 1/r^3 through FP32
-//                  rsqrt.
+//                  64 entries a pass (k_walk_single: for 64 targets, a node at
+//                  a time): each target applies the reference opening test
+//                  itself; those that accept a node add its monopole, the
+//                  others descend.  Geometry and sums in FP64, 1/r^3 through
+//                  FP32 rsqrt.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -1096,8 +1097,9 @@ __device__ __forceinline__ void oct_term(const float *__restrict__ T, double R0,
 // children.  The interaction set is exactly the per-particle walk's; only the
 // order of the FP64 sums differs.
 //
-// Bound by VALU issue (16 FP64 instructions of 4.75 cycles per G entries of
-// a pass) once the chip is full.  k_walk_single visits one node at a time
+// Bound by VALU issue once the chip is full: at 2^21 particles 71 to 75 % of
+// the SIMDs' cycles at 4 per instruction, at 60000, with its last wavefronts,
+// 53 %.  k_walk_single visits one node at a time
 // through scalar loads, each waiting for the last one's; what they measured
 // stands at the choice in tree_walk.
 //
