@@ -1011,7 +1011,7 @@ constexpr int WK_BATCH_LIMIT = WK_STACK - 8 * (MAXL + 2);
 
 // The mark of a stack that would have overflowed, in a walk's interaction
 // counter: set by an OR, since several wavefronts may set it (four additions
-// of 2^62 would cancel, and the eight wavefronts of a shared group that walk
+// of 2^62 would cancel, and the wavefronts of a shared group that walk
 // alike would all add theirs).
 constexpr unsigned long long WALK_OVERFLOW = 1ull << 63;
 
@@ -1579,15 +1579,18 @@ __global__ __launch_bounds__(WS_BLOCK) void k_walk_single(const NodeRec *__restr
 // time, so for few particles GW_SPLIT wavefronts share a group: they take the
 // first passes alike (wavefront 0 collecting the terms) until the stack holds
 // GW_SHARE entries per wavefront, then every GW_SPLIT-th entry each, and their
-// sums are added at the end.  Two such groups are resident per CU against
-// seventeen of one wavefront, so with many groups or short lists the sharing
-// loses: it is used up to 80 particles per CU, and at theta up to 0.5 up to
-// 160.  Walk, one / eight wavefronts, us: two spheres of 10000, theta 0.5: 348
-// / 221, 20000: 913 / 475; uniform box, theta 0.2, 20000: 577 / 204, 40000: 819
-// / 329; the same at 0.8, 20000: 160 / 166, 26000: 141 / 162, 40000: 150 / 197.
-// From 50000 the outcome turns with the particle number (two spheres at 0.35,
-// 60000: 2269 / 912, 65536 with quadrupoles: 1209 / 1911).
-constexpr int GW_SPLIT = 8;
+// sums are added at the end.  Four such groups are resident per CU (two of
+// eight wavefronts) against seventeen of one, so with many groups or short
+// lists the sharing loses: it is used up to 320 particles per CU, at theta
+// above 0.65 up to 128.  Walk, one / four / eight wavefronts, us: two spheres,
+// theta 0.5, 20000: 932 / 497 / 481, 60000: 2216 / 1317 / 844; uniform box,
+// theta 0.2, 40000: 811 / 338 / 326, theta 0.8, 20000: 169 / 133 / 168; with
+// local expansions at 0.8, 60000: 168 / 196 / 280; two spheres of 131072 with
+// quadrupoles, theta 0.5: 893 / 1186 / 1587.  Against the walks of one wavefront
+// before their rows were free of branches, at 21 sizes from 1000 to 81920, five
+// angles and three distributions none is slower; with eight wavefronts uniform
+// boxes from 26000 and two spheres of 65536 were.
+constexpr int GW_SPLIT = 4;
 constexpr int GW_SHARE = 32;
 constexpr int GW_STACK = 1024;
 constexpr int GW_LIST = 128;
@@ -2764,7 +2767,7 @@ ErrorStatus tree_walk_group(Context *c, DeviceTree *t, double G, double eps, dou
                            t->sidx, t->n, groups, args, a, cnt, t->quadf);
     };
     auto pick = [&](auto k1, auto kw) {
-        if (t->n <= (theta <= 0.5 ? 160 : 80) * c->cu_count) walk(kw, GW_SPLIT);
+        if (t->n <= (theta <= 0.65 ? 320 : 128) * c->cu_count) walk(kw, GW_SPLIT);
         else walk(k1, 1);
     };
     if (order >= 2) pick(k_walk_group<true, false, 1>, k_walk_group<true, false, GW_SPLIT>);

@@ -492,10 +492,10 @@ def test_walk_at_small_angles_against_the_oracle(theta):
     assert np.median(e) < 1e-6 and e.max() < 1e-4
 
 
-@pytest.mark.parametrize("n,th", [(2, 0.6), (66, 0.6), (700, 0.6), (20480, 0.6), (20482, 0.6), (40960, 0.5), (40962, 0.5),
-                                  (65538, 0.6), (131074, 0.6)])
+@pytest.mark.parametrize("n,th", [(2, 0.6), (66, 0.6), (700, 0.6), (32768, 0.7), (32770, 0.7), (65538, 0.6), (81920, 0.65),
+                                  (81922, 0.65), (131074, 0.6)])
 def test_group_walk_forms_against_the_oracle(n, th):
-    """Several wavefronts per group (up to 20480 particles on 256 CUs, at theta up to 0.5 up to 40960) and one: equal
+    """Several wavefronts per group (up to 32768 particles on 256 CUs, at theta up to 0.65 up to 81920) and one: equal
     interaction counts and forces to FP32 rounding, without and with quadrupoles and with local expansions; trees too
     small to be shared out."""
     x, v, m = ic.two_spheres(n, 70 + n % 89)
